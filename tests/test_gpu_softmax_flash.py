@@ -99,6 +99,46 @@ def test_row_softmax_rows_against_oracle(gpu, oracle, rows, cols, masked):
         assert rc == 0, (r, rc, bad)
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("cols", [1, 3, 4, 5, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 513,
+                                  767, 769, 1023, 1025, 1281, 1537, 1793, 2047, 2049, 2304, 2305,
+                                  3585, 3841, 4095, 4097, 4609, 7681, 8191, 8193])
+def test_row_softmax_any_width(gpu, oracle, cols, masked):
+    """Every form of the register kernel at its first and last widths, rows
+    that start at any 4-byte (mask: 1-byte) address, a row count that leaves
+    waves and workgroups partly empty, one row rejected for a NaN in its last
+    column: element by element under the OCML policy against float64."""
+    from fe2o3_amd.runtime import Fe2o3Error
+    rows, bad_row = 19, 7
+    rng = np.random.default_rng(cols * 2 + masked)
+    x = (rng.standard_normal(rows * cols + 1) * 4.0).astype(np.float32)
+    x[1 + bad_row * cols + cols - 1] = np.nan
+    mask = (rng.random(rows * cols + 1) < 0.7).astype(np.uint8)
+    mask[1:1 + cols] = 0  # the first row fully masked
+    gi, gm = Guarded(gpu, x), Guarded(gpu, mask)
+    go = Guarded(gpu, np.full(rows * cols + 1, 7.0, np.float32))
+    n = rows * cols
+    prep = _k().row_softmax_gpu.Kernel.load(gpu).prepare(
+        gi.body.view(1, n), go.body.view(1, n), gm.body.view(1, n) if masked else None, rows, cols)
+    with pytest.raises(Fe2o3Error):
+        prep.launch()
+    out = go.download()
+    assert go.guards_intact() and gi.unchanged() and gm.unchanged() and out[0] == 7.0
+    got, xs = out[1:].reshape(rows, cols), x[1:].reshape(rows, cols)
+    for r in range(rows):
+        act = mask[1:].reshape(rows, cols)[r].astype(bool) if masked else np.ones(cols, bool)
+        if r == bad_row:
+            assert got[r].view(np.uint32).tolist() == [0x7FC00000] * cols
+        elif not act.any():
+            assert got[r].view(np.uint32).tolist() == [0] * cols
+        else:
+            w = np.where(act, np.exp(xs[r].astype(np.float64) - xs[r][act].max()), 0.0)
+            ref = (w / w.sum()).astype(np.float32)
+            m = act.astype(np.uint8) if masked else None
+            rc, bad = oracle.compare_row_softmax_v1(ref, got[r], m, **oracle.GFX_SOFTMAX_POLICY)
+            assert rc == 0, (r, rc, bad)
+
+
 def test_row_softmax_config3c_every_row(gpu, oracle):
     """BASELINE config 3c at full size: 1,048,576 rows x 4096 fp32 (the
     bench's N(0,1) input, seed 3).  Every row, element by element, against
