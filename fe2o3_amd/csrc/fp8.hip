@@ -11,13 +11,12 @@
 // The GEMM reuses the 256x256 tile machinery of the bf16 GEMM: one LDS stage
 // is 128 bytes of k per row, i.e. 128 fp8 values, each taken by one
 // v_mfma_f32_16x16x128_f8f6f4 (5.0 PFLOP/s dense peak).  Any M
-// and N run on it (edge tiles store only their valid rows and columns);
-// K not a multiple of 128, or unaligned operands, take a bounds-checked
-// 64x64-tile kernel that widens E4M3 to bf16 exactly while staging and
-// multiplies on bf16 MFMAs (the products are exact either way); K = 0
-// writes +0.
+// and N run on it (edge tiles store only their valid rows and columns).
+// Outputs of few tiles, at any alignment and K (K = 0 writes +0), take the
+// direct kernel (gemm_direct.hpp).
 #include "common.hpp"
 #include "gemm_core.hpp"
+#include "gemm_direct.hpp"
 #include "gemm_pipe.hpp"
 #include "internal.hpp"
 
@@ -117,7 +116,7 @@ constexpr int kFp8Smem = kFp8Stages * 2 * gemm_pipe::Geo<kFp8RowBytes>::kTileByt
 // the last valid row, and each tile stores only its valid rows and columns.
 // KT: K is a multiple of 16 but not of 128; the last stage is partial and
 // its chunks past K load zeros (gemm_pipe::Rows MASK), whose products are
-// zero (the generic kernel's zero padding of its last k step).
+// zero.
 template <bool STAGED, bool EDGE, bool KT = false>
 __global__ void __launch_bounds__(256, 1) gemm_fp8_kernel(const uint8_t* __restrict__ a,
                                                           const uint8_t* __restrict__ b,
@@ -245,68 +244,33 @@ int32_t repack_bytes(const uint8_t* src, uint32_t rows, uint32_t cols, uint8_t* 
 
 constexpr uint32_t kRepackMin = 128;  // outputs at least this in M and N repack
 
-// ---- any shape ---------------------------------------------------------------------------
-// 64x64 output tiles, 32 k per step; each operand element is widened to bf16
-// (exact) on its way to LDS, zero outside m x k / n x k, and four waves (2x2,
-// 32x32 each) multiply with v_mfma_f32_16x16x32_bf16.  The scale product is
-// applied to the fp32 sums, as on the fast path.
-constexpr int G8_BM = 64, G8_BN = 64, G8_BK = 32, G8_LDK = G8_BK + 8;
-
-__global__ void __launch_bounds__(256) gemm_fp8_generic_kernel(
-    const uint8_t* __restrict__ a, const uint8_t* __restrict__ b, const float* __restrict__ scale_a,
-    const float* __restrict__ scale_b, uint16_t* __restrict__ c, uint32_t m, uint32_t n,
-    uint32_t k) {
-  __shared__ __attribute__((aligned(16))) uint16_t a_lds[G8_BM * G8_LDK];
-  __shared__ __attribute__((aligned(16))) uint16_t b_lds[G8_BN * G8_LDK];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const uint64_t row0 = (uint64_t)blockIdx.y * G8_BM, col0 = (uint64_t)blockIdx.x * G8_BN;
-  f32x4_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (uint64_t k0 = 0; k0 < k; k0 += G8_BK) {
-    const int r = t >> 2, d0 = (t & 3) * 8;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint64_t gd = k0 + d0 + e;
-      const uint64_t ga = row0 + r, gb = col0 + r;
-      a_lds[r * G8_LDK + d0 + e] = (ga < m && gd < k) ? bf16_bits_from_e4m3(a[ga * k + gd]) : 0;
-      b_lds[r * G8_LDK + d0 + e] = (gb < n && gd < k) ? bf16_bits_from_e4m3(b[gb * k + gd]) : 0;
-    }
-    __syncthreads();
-    const int rc = lane & 15, chunk = lane >> 4;
-    bf16x8_t af[2], bf[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      af[i] = *reinterpret_cast<const bf16x8_t*>(a_lds + (wm * 32 + i * 16 + rc) * G8_LDK + chunk * 8);
-      bf[i] = *reinterpret_cast<const bf16x8_t*>(b_lds + (wn * 32 + i * 16 + rc) * G8_LDK + chunk * 8);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
-  }
-  const float sab = scale_a[0] * scale_b[0];
-  const int col_in = lane & 15, row_in = (lane >> 4) * 4;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint64_t gr = row0 + wm * 32 + i * 16 + row_in + e;
-        const uint64_t gc = col0 + wn * 32 + j * 16 + col_in;
-        if (gr < m && gc < n) c[gr * n + gc] = bf16_bits_from_f32(acc[i][j][e] * sab);
-      }
+// ---- few output tiles, any alignment, any K ----------------------------------------------
+template <bool WIDE>
+__global__ void __launch_bounds__(gemm_direct::kThreads, WIDE ? 2 : 4) gemm_fp8_direct_kernel(
+    int form, const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
+    const float* __restrict__ scale_a, const float* __restrict__ scale_b,
+    uint16_t* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t xcds) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  gemm_direct::run_form<gemm_direct::Fp8, WIDE>(form, a, b, c, m, n, k, scale_a[0] * scale_b[0],
+                                                xcds, smem);
 }
 
-__global__ void __launch_bounds__(256) zero_fill_bf16_kernel(uint16_t* __restrict__ c, uint64_t n) {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) c[i] = 0;
+int32_t launch_direct(const uint8_t* a, const uint8_t* b, const float* sa, const float* sb,
+                      uint16_t* c, uint32_t m, uint32_t n, uint32_t k,
+                      const tile_plan::Topology& topo, hipStream_t s) {
+  static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
+      {(const void*)gemm_fp8_direct_kernel<true>,
+       (const void*)gemm_fp8_direct_kernel<false>}, gemm_direct::kWideSmem);
+  if (lds_rc != FE2O3_OK) return lds_rc;
+  const gemm_direct::Launch l = gemm_direct::plan(m, n, k, 1u, topo.cus);
+  if (l.grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
+  if (l.wide)
+    gemm_fp8_direct_kernel<true><<<(unsigned)l.grid, gemm_direct::kThreads, l.smem, s>>>(
+        l.form, a, b, sa, sb, c, m, n, k, topo.xcds);
+  else
+    gemm_fp8_direct_kernel<false><<<(unsigned)l.grid, gemm_direct::kThreads, l.smem, s>>>(
+        l.form, a, b, sa, sb, c, m, n, k, topo.xcds);
+  return fe2o3_host::after_launch();
 }
 
 // one workgroup per 4096-element step, at most 8192 striding over the rest
@@ -343,9 +307,9 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_128_kernel<3, edge, k tail>", (const void*)gemm_fp8_128_kernel<3, false, false, true>, 256, kFp8SmallSmem<3>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_128_kernel<2, edge, tail, k tail>", (const void*)gemm_fp8_128_kernel<2, false, true, true>, 256, kFp8SmallSmem<2>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_128_kernel<3, edge, tail, k tail>", (const void*)gemm_fp8_128_kernel<3, false, true, true>, 256, kFp8SmallSmem<3>}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_generic_kernel", (const void*)gemm_fp8_generic_kernel, 256, 0}),
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel", (const void*)gemm_fp8_direct_kernel<false>, gemm_direct::kThreads, gemm_direct::kLightSmem}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "repack_bytes_kernel", (const void*)repack_bytes_kernel, 256, 0}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "zero_fill_bf16_kernel", (const void*)zero_fill_bf16_kernel, 256, 0})};
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel<wide>", (const void*)gemm_fp8_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem})};
 
 }  // namespace
 
@@ -470,11 +434,13 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   if (c_len == 0) return FE2O3_OK;
   if ((a_len && !a) || (b_len && !b) || !c || !scale_a || !scale_b) return FE2O3_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
-  if (k == 0) {  // the empty sum: +0 (a fill kernel, so the launch can be captured)
-    const uint64_t blocks = (c_len + 255) / 256;
-    zero_fill_bf16_kernel<<<(unsigned)(blocks < 4096u ? blocks : 4096u), 256, 0, s>>>(c, c_len);
-    return fe2o3_host::after_launch();
-  }
+  tile_plan::Topology topo;
+  const int32_t topo_rc = fe2o3_host::device_topology(&topo);
+  if (topo_rc != FE2O3_OK) return topo_rc;
+  // Few output tiles, and K = 0 (the empty sum, +0): the direct kernel,
+  // whatever the operands' alignment.
+  if (k == 0 || (gemm_direct::k_fits(k, 1u) && gemm_direct::prefer(m, n, k, 1u, topo.cus)))
+    return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
   // fast path: 16-byte operand rows (K a multiple of 16) and a 256-row fp8
   // panel (256 * k bytes) within its buffer resource's 32-bit range; K not a
   // multiple of 128 takes the edge tiles with a partial last stage
@@ -486,7 +452,7 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   // then runs on kp, whose zeros fall where its partial last stage puts
   // zeros anyway, so an operand that is only misaligned gives the bits of
   // the aligned one.  Outputs below 128 x 128, and devices without
-  // stream-ordered scratch, take the generic kernel.
+  // stream-ordered scratch, take the direct kernel.
   const uint32_t kp = (k + 15u) & ~15u;
   const bool repack = !fast && m >= kRepackMin && n >= kRepackMin && 256ull * kp < (1ull << 31);
   void* scratch = nullptr;
@@ -494,21 +460,15 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
     const bool ra = k % 16 != 0 || !aligned_a, rb = k % 16 != 0 || !aligned_b;
     const uint64_t a_bytes = ra ? (uint64_t)m * kp : 0, b_bytes = rb ? (uint64_t)n * kp : 0;
     if (fe2o3_host::scratch_alloc(&scratch, a_bytes + b_bytes, s) != FE2O3_OK) {
-      (void)hipGetLastError();  // no stream-ordered scratch: the generic kernel
+      (void)hipGetLastError();  // no stream-ordered scratch: the direct kernel
       scratch = nullptr;
     }
   }
-  if (!fast && scratch == nullptr) {
-    const dim3 grid((n + G8_BN - 1) / G8_BN, (m + G8_BM - 1) / G8_BM);
-    if (grid.y > 65535u) return FE2O3_ERR_SHAPE;
-    gemm_fp8_generic_kernel<<<grid, 256, 0, s>>>(a, b, scale_a, scale_b, c, m, n, k);
-    return fe2o3_host::after_launch();
-  }
+  if (!fast && scratch == nullptr)
+    return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
   // every kernel's LDS limit is raised before anything is launched, so a
   // failure leaves C untouched
   int32_t rc = set_fp8_lds();
-  tile_plan::Topology topo;
-  if (rc == FE2O3_OK) rc = fe2o3_host::device_topology(&topo);
   const tile_plan::Plan plan = rc == FE2O3_OK ? tile_plan::plan(m, n, topo) : tile_plan::Plan{};
   if (rc == FE2O3_OK && (plan.grid > 0x7fffffffu || plan.tail_grid > 0x7fffffffu))
     rc = FE2O3_ERR_SHAPE;

@@ -6,11 +6,11 @@
 // 256x256 pipelined MFMA tile of gemm_pipe.hpp with 64 k per LDS stage and
 // two stages, workgroups ordered XCD-aware (gemm_core.hpp); m or n not a
 // multiple of 256 (or an unaligned C) runs its edge form, and k not a
-// multiple of 64 either form with a partial last stage.  Any other shape
-// (k not a multiple of 8, misaligned A or B) uses a bounds-checked
-// 64x64-tile MFMA kernel.
+// multiple of 64 either form with a partial last stage.  Outputs of few
+// tiles, at any alignment and K, take the direct kernel (gemm_direct.hpp).
 #include "common.hpp"
 #include "gemm_core.hpp"
+#include "gemm_direct.hpp"
 #include "gemm_pipe.hpp"
 #include "internal.hpp"
 
@@ -20,57 +20,15 @@ namespace {
 
 using namespace fe2o3;
 
-// ---- generic path -------------------------------------------------------------------
-constexpr int N_BM = 64, N_BN = 64, N_BK = 32, N_LDK = N_BK + 8;
-
-__global__ void __launch_bounds__(256) gemm_bf16_nt_generic_kernel(
-    const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
-    uint32_t m, uint32_t n, uint32_t k) {
-  __shared__ __attribute__((aligned(16))) uint16_t a_lds[N_BM * N_LDK];
-  __shared__ __attribute__((aligned(16))) uint16_t b_lds[N_BN * N_LDK];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const uint64_t row0 = (uint64_t)blockIdx.y * N_BM, col0 = (uint64_t)blockIdx.x * N_BN;
-  f32x4_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  for (uint64_t k0 = 0; k0 < k; k0 += N_BK) {
-    const int r = t >> 2, d0 = (t & 3) * 8;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const uint64_t gd = k0 + d0 + e;
-      const uint64_t ga = row0 + r, gb = col0 + r;
-      a_lds[r * N_LDK + d0 + e] = (ga < m && gd < k) ? a[ga * k + gd] : (uint16_t)0;
-      b_lds[r * N_LDK + d0 + e] = (gb < n && gd < k) ? b[gb * k + gd] : (uint16_t)0;
-    }
-    __syncthreads();
-    const int rc = lane & 15, chunk = lane >> 4;
-    bf16x8_t af[2], bf[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      af[i] = *reinterpret_cast<const bf16x8_t*>(a_lds + (wm * 32 + i * 16 + rc) * N_LDK + chunk * 8);
-      bf[i] = *reinterpret_cast<const bf16x8_t*>(b_lds + (wn * 32 + i * 16 + rc) * N_LDK + chunk * 8);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
-  }
-  const int col_in = lane & 15, row_in = (lane >> 4) * 4;
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint64_t gr = row0 + wm * 32 + i * 16 + row_in + e;
-        const uint64_t gc = col0 + wn * 32 + j * 16 + col_in;
-        if (gr < m && gc < n) c[gr * n + gc] = bf16_bits_from_f32(acc[i][j][e]);
-      }
+// ---- few output tiles, any alignment, any K ---------------------------------------------
+template <bool WIDE>
+__global__ void __launch_bounds__(gemm_direct::kThreads, WIDE ? 2 : 4) gemm_bf16_nt_direct_kernel(
+    int form, const uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
+    uint16_t* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t xcds) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  gemm_direct::run_form<gemm_direct::Bf16, WIDE>(
+      form, reinterpret_cast<const uint8_t*>(a), reinterpret_cast<const uint8_t*>(b), c, m, n, k,
+      1.0f, xcds, smem);
 }
 
 // ---- fast path ----------------------------------------------------------------------------
@@ -87,8 +45,8 @@ constexpr int kFastSmem = kStages * 2 * gemm_pipe::Geo<kRowBytes>::kTileBytes;  
 // stores only its valid rows and columns, element by element.
 //
 // KT: K is a multiple of 8 but not of 64; the last stage is partial and its
-// chunks past K load zeros (gemm_pipe::Rows MASK), the zero padding the
-// generic kernel gives its last k step, so C is bit-identical to it.
+// chunks past K load zeros (gemm_pipe::Rows MASK), so C is bit-identical to
+// that of operands zero-padded to whole stages.
 template <bool STAGED, bool EDGE, bool KT = false>
 __global__ void __launch_bounds__(256, 1) gemm_bf16_nt_256_kernel(const uint16_t* __restrict__ a,
                                                                    const uint16_t* __restrict__ b,
@@ -154,13 +112,6 @@ __global__ void __launch_bounds__(256, STAGES == 2 ? 2 : 1) gemm_bf16_nt_128_ker
                                    rows_a, rows_b);
 }
 
-// K = 0: C is all +0 (an empty sum).  A grid-stride fill kernel rather than
-// a memset node, so a caller may capture the launch in a HIP graph.
-__global__ void __launch_bounds__(256) zero_fill_bf16_kernel(uint16_t* __restrict__ c, uint64_t n) {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) c[i] = 0;
-}
-
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // kernels behind each entry point (fe2o3_kernel_resources)
@@ -186,8 +137,8 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_128_kernel<3, edge, k tail>", (const void*)gemm_bf16_nt_128_kernel<3, false, false, true>, 256, kSmallSmem<3>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_128_kernel<2, edge, tail, k tail>", (const void*)gemm_bf16_nt_128_kernel<2, false, true, true>, 256, kSmallSmem<2>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_128_kernel<3, edge, tail, k tail>", (const void*)gemm_bf16_nt_128_kernel<3, false, true, true>, 256, kSmallSmem<3>}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_generic_kernel", (const void*)gemm_bf16_nt_generic_kernel, 256, 0}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "zero_fill_bf16_kernel", (const void*)zero_fill_bf16_kernel, 256, 0})};
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel", (const void*)gemm_bf16_nt_direct_kernel<false>, gemm_direct::kThreads, gemm_direct::kLightSmem}),
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel<wide>", (const void*)gemm_bf16_nt_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem})};
 
 // Raises every fast-path kernel's dynamic-LDS limit once per process.
 int32_t set_fast_lds() {
@@ -273,6 +224,23 @@ int32_t launch_fast(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t 
 
 namespace {
 constexpr uint32_t kRepackMin = 128;  // outputs at least this in M and N repack
+
+int32_t launch_direct(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m, uint32_t n,
+                      uint32_t k, const tile_plan::Topology& topo, hipStream_t s) {
+  static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
+      {(const void*)gemm_bf16_nt_direct_kernel<true>,
+       (const void*)gemm_bf16_nt_direct_kernel<false>}, gemm_direct::kWideSmem);
+  if (lds_rc != FE2O3_OK) return lds_rc;
+  const gemm_direct::Launch l = gemm_direct::plan(m, n, k, 2u, topo.cus);
+  if (l.grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
+  if (l.wide)
+    gemm_bf16_nt_direct_kernel<true><<<(unsigned)l.grid, gemm_direct::kThreads, l.smem, s>>>(
+        l.form, a, b, c, m, n, k, topo.xcds);
+  else
+    gemm_bf16_nt_direct_kernel<false><<<(unsigned)l.grid, gemm_direct::kThreads, l.smem, s>>>(
+        l.form, a, b, c, m, n, k, topo.xcds);
+  return fe2o3_host::after_launch();
+}
 }  // namespace
 
 extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const uint16_t* b,
@@ -283,48 +251,39 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
     return FE2O3_ERR_LENGTH;
   if (c_len == 0) return FE2O3_OK;
   if ((a_len && !a) || (b_len && !b) || !c) return FE2O3_ERR_NULL;
-  if (k == 0) {
-    const uint64_t blocks = (c_len + 255) / 256;
-    zero_fill_bf16_kernel<<<(unsigned)(blocks < 4096u ? blocks : 4096u), 256, 0,
-                            (hipStream_t)stream>>>(c, c_len);
-    return fe2o3_host::after_launch();
-  }
+  tile_plan::Topology topo;
+  const int32_t topo_rc = fe2o3_host::device_topology(&topo);
+  if (topo_rc != FE2O3_OK) return topo_rc;
+  hipStream_t s = (hipStream_t)stream;
+  // Few output tiles, and K = 0 (the empty sum, +0): the direct kernel,
+  // whatever the operands' alignment.
+  if (k == 0 || (gemm_direct::k_fits(k, 2u) && gemm_direct::prefer(m, n, k, 2u, topo.cus)))
+    return launch_direct(a, b, c, m, n, k, topo, s);
   // fast path: 16-byte operand rows (K a multiple of 8), and a 256-row panel
   // (512 * k bytes) inside the 32-bit range of its buffer resource; whole
   // tiles with a 16-byte aligned C take the plain tile, any other M and N
   // the edge tile; K not a multiple of 64 the same tiles with a partial last
   // stage (KT)
   const bool fast = k % 8 == 0 && 512ull * k < (1ull << 31) && aligned16(a) && aligned16(b);
-  if (fast) {
-    const int32_t lds_rc = set_fast_lds();  // before any launch: a failure leaves C untouched
-    if (lds_rc != FE2O3_OK) return lds_rc;
-    tile_plan::Topology topo;
-    const int32_t topo_rc = fe2o3_host::device_topology(&topo);
-    if (topo_rc != FE2O3_OK) return topo_rc;
-    const tile_plan::Plan plan = tile_plan::plan(m, n, topo);
-    if (plan.grid > 0x7fffffffu || plan.tail_grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
-    if (k % gemm_pipe::Geo<kRowBytes>::kK16 != 0)
-      return launch_fast<true>(a, b, c, m, n, k, plan, topo.xcds, (hipStream_t)stream);
-    return launch_fast<false>(a, b, c, m, n, k, plan, topo.xcds, (hipStream_t)stream);
-  }
   // Rows the tile cannot read in place (K not a multiple of 8, or A or B two
   // bytes past a 16-byte boundary) are first copied into aligned rows of kp
   // = K rounded up to 8, zeros from K on, in stream-ordered scratch; the
   // tile then runs on kp, whose zeros fall where its partial last stage
   // puts zeros anyway, so an operand that is only misaligned gives the bits
   // of the aligned one.  Outputs below 128 x 128, and devices without
-  // stream-ordered scratch, take the generic kernel.
+  // stream-ordered scratch, take the direct kernel.
   const uint32_t kp = (k + 7u) & ~7u;
-  hipStream_t s = (hipStream_t)stream;
-  if (m >= kRepackMin && n >= kRepackMin && 512ull * kp < (1ull << 31)) {
-    const bool ra = k % 8 != 0 || !aligned16(a), rb = k % 8 != 0 || !aligned16(b);
-    const int32_t lds_rc = set_fast_lds();
+  if (fast || (m >= kRepackMin && n >= kRepackMin && 512ull * kp < (1ull << 31))) {
+    const int32_t lds_rc = set_fast_lds();  // before any launch: a failure leaves C untouched
     if (lds_rc != FE2O3_OK) return lds_rc;
-    tile_plan::Topology topo;
-    const int32_t topo_rc = fe2o3_host::device_topology(&topo);
-    if (topo_rc != FE2O3_OK) return topo_rc;
     const tile_plan::Plan plan = tile_plan::plan(m, n, topo);
     if (plan.grid > 0x7fffffffu || plan.tail_grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
+    if (fast) {
+      if (k % gemm_pipe::Geo<kRowBytes>::kK16 != 0)
+        return launch_fast<true>(a, b, c, m, n, k, plan, topo.xcds, s);
+      return launch_fast<false>(a, b, c, m, n, k, plan, topo.xcds, s);
+    }
+    const bool ra = k % 8 != 0 || !aligned16(a), rb = k % 8 != 0 || !aligned16(b);
     const uint64_t a_elems = ra ? (uint64_t)m * kp : 0, b_elems = rb ? (uint64_t)n * kp : 0;
     void* scratch = nullptr;
     if (fe2o3_host::scratch_alloc(&scratch, (a_elems + b_elems) * 2u, s) == FE2O3_OK) {
@@ -340,10 +299,7 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
       const int32_t free_rc = fe2o3_host::scratch_free(scratch, s);
       return rc != FE2O3_OK ? rc : free_rc;
     }
-    (void)hipGetLastError();  // no stream-ordered scratch: the generic kernel
+    (void)hipGetLastError();  // no stream-ordered scratch: the direct kernel
   }
-  dim3 grid((n + N_BN - 1) / N_BN, (m + N_BM - 1) / N_BM);
-  if (grid.y > 65535u) return FE2O3_ERR_SHAPE;
-  gemm_bf16_nt_generic_kernel<<<grid, 256, 0, s>>>(a, b, c, m, n, k);
-  return fe2o3_host::after_launch();
+  return launch_direct(a, b, c, m, n, k, topo, s);
 }

@@ -262,9 +262,11 @@ int32_t fe2o3_scalar_gemm_v1(const float *a, uint64_t a_len, const float *b,
  * rows that cannot be read in place are first copied into aligned rows of
  * k rounded up to 8 (zeros past k) in stream-ordered scratch from the
  * library's pool and the tile runs on them (an operand that is only
- * misaligned gives the aligned operand's bits).  Smaller outputs, and
- * devices without a pool, take a bounds-checked 64x64-tile kernel; k = 0
- * writes +0. */
+ * misaligned gives the aligned operand's bits).  Outputs with too few tiles
+ * to fill the device (at most 32 rows or columns, or about one round of
+ * 64x32 blocks), whatever the alignment, and devices without a pool, take a
+ * kernel that splits k over the waves of a workgroup and reads the operands
+ * at their own alignment; k = 0 writes +0. */
 int32_t fe2o3_gemm_bf16_nt(const uint16_t *a, uint64_t a_len,
                            const uint16_t *b, uint64_t b_len, uint16_t *c,
                            uint64_t c_len, uint32_t m, uint32_t n, uint32_t k,
@@ -486,10 +488,10 @@ int32_t fe2o3_quantize_e4m3(const float *x, uint64_t x_len, const float *scale,
  * or an unaligned C).  For other k or alignments, when m and n are at least
  * 128, the rows that cannot be read in place are first copied into aligned
  * rows of k rounded up to 16 (E4M3 +0 past k) in stream-ordered scratch
- * from the library's pool and the tile runs on them; smaller outputs, and
- * devices without a pool, take a bounds-checked kernel that widens E4M3 to
- * bf16 exactly and multiplies on bf16 MFMAs.  k = 0 writes +0.  The
- * products of two E4M3 values are exact in fp32 on every path. */
+ * from the library's pool and the tile runs on them; outputs with too few
+ * tiles to fill the device, and devices without a pool, take the kernel that
+ * splits k over a workgroup's waves (as fe2o3_gemm_bf16_nt).  k = 0 writes
+ * +0.  The products of two E4M3 values are exact in fp32 on every path. */
 int32_t fe2o3_gemm_fp8_nt(const uint8_t *a, uint64_t a_len, const uint8_t *b,
                           uint64_t b_len, const float *scale_a,
                           const float *scale_b, uint16_t *c, uint64_t c_len,

@@ -417,6 +417,40 @@ def test_gemm_bf16_nt_odd_k_repacked(gpu, oracle, m, n, k):
     _nt_case(gpu, oracle, m, n, k, seed=4)
 
 
+# The direct kernel (gemm_direct.hpp): every form's first and last rows and
+# columns, K of part of a piece, less than a unit, one unit per wave and one
+# more, several rounds and their remainders; the widest K takes 64-bit offsets
+@pytest.mark.parametrize("m,n,k", [(1, 1, 7), (3, 50, 9), (16, 16, 64), (17, 15, 63), (16, 700, 65),
+                                   (31, 513, 511), (32, 4200, 520), (33, 1000, 576), (64, 4096, 1088),
+                                   (64, 5000, 2056), (65, 2100, 1536), (130, 1100, 3000),
+                                   (1000, 20, 4100), (4100, 16, 1030), (16, 9000, 2048),
+                                   (1, 2, (1 << 25) + 3)])
+def test_gemm_bf16_nt_direct_forms(gpu, oracle, m, n, k):
+    """Against the oracle, and with A and B two bytes past a 16-byte boundary
+    bit for bit the aligned operands' C (inputs unchanged, guards intact)."""
+    a, b = _nt_case(gpu, oracle, m, n, k, seed=21)
+    prep = _kernels().gemm_bf16_nt_gpu.Kernel.load(gpu)
+    want = gpu.alloc(m * n, np.uint16)
+    prep.prepare(gpu.to_device(a), gpu.to_device(b), want, m, n, k).launch()
+    ga, gb = (Guarded(gpu, np.concatenate([np.zeros(1, np.uint16), h])) for h in (a, b))
+    got = Guarded(gpu, np.full(m * n + 1, 0x7FDE, np.uint16))  # C two bytes off as well
+    prep.prepare(ga.full.view(GUARD + 1, m * k), gb.full.view(GUARD + 1, n * k),
+                 got.body.view(1, m * n), m, n, k).launch()
+    assert got.guards_intact() and ga.unchanged() and gb.unchanged()
+    assert_same(got.download()[1:], want.download(), "2-byte offsets vs aligned")
+
+
+# Outputs just too large for the direct kernel: the 128x128 small-grid forms,
+# whole and edge tiles, one K step to several groups of three, partial last
+# stages, and repacked rows (K odd, 1600 x 1500: above the direct kernel's line
+# for those too)
+@pytest.mark.parametrize("m,n,k", [(1024, 1024, 64), (1024, 1024, 128), (1000, 1032, 192),
+                                   (1024, 1024, 320), (1024, 1024, 8), (1024, 1024, 72),
+                                   (1000, 1032, 1000), (1600, 1500, 77), (1600, 1500, 1003)])
+def test_gemm_bf16_nt_small_grid_tiles(gpu, oracle, m, n, k):
+    _nt_case(gpu, oracle, m, n, k, seed=22, rows=[0, 63, 127, 128, 511, 895, 897, m - 2, m - 1])
+
+
 # M or N not a multiple of 256 with whole 64-k stages: edge tiles of the
 # pipelined kernel (clamped operand rows, element-wise masked stores)
 @pytest.mark.parametrize("m,n,k", [(300, 520, 512), (257, 255, 128), (1, 1000, 64),

@@ -511,6 +511,43 @@ def test_gemm_fp8_any_shape(gpu, oracle, m, n, k):
     assert _fp8_case(gpu, oracle, m, n, k, (rr.ravel(), cc.ravel())) <= 1e-2
 
 
+# the direct kernel (gemm_direct.hpp): as for bf16, in units of 128 k; and the
+# 128x128 small-grid tiles, whole and edge, repacked rows among them
+@pytest.mark.parametrize("m,n,k", [(1, 1, 15), (3, 50, 17), (16, 700, 129), (31, 513, 1023),
+                                   (32, 4200, 1040), (33, 1000, 1152), (64, 4096, 2176),
+                                   (64, 5000, 4103), (65, 2100, 3072), (130, 1100, 6000),
+                                   (1000, 20, 8200), (4100, 16, 2061), (16, 9000, 4096),
+                                   (1024, 1024, 128), (1000, 1032, 384), (1024, 1024, 1040),
+                                   (1600, 1500, 77)])
+def test_gemm_fp8_direct_forms_and_small_grids(gpu, oracle, m, n, k):
+    """Random codes (no NaN) against the oracle on up to 20000 outputs, and
+    with every operand one byte (C two) past its boundary bit for bit the
+    same C."""
+    kern = _k()
+    rng = np.random.default_rng(m + 7 * n + k)
+    a, b = (rng.integers(0, 0x60, s, dtype=np.uint8) | (rng.integers(0, 2, s, dtype=np.uint8) << 7)
+            for s in (m * k, n * k))
+    sa = gpu.to_device(np.array([1.0 / 64], np.float32))
+    sb = gpu.to_device(np.array([1.0 / 32], np.float32))
+    c = Guarded(gpu, np.full(m * n, 0x7FDE, np.uint16))
+    kern.gemm_fp8_nt(gpu.to_device(a), gpu.to_device(b), sa, sb, c.body, m, n, k)
+    assert c.guards_intact()
+    got = c.download()
+    if m * n <= 20000:
+        rows, cols = (v.ravel() for v in np.meshgrid(np.arange(m), np.arange(n), indexing="ij"))
+    else:
+        rows, cols = rng.integers(0, m, 20000), rng.integers(0, n, 20000)
+        rows[:2], cols[:2] = (m - 1, 0), (n - 1, 0)
+    ref, _ = oracle.gemm_fp8_points(k, a.reshape(m, k)[rows], b.reshape(n, k)[cols], 1.0 / 2048)
+    assert rel_err(bf16_to_f32(got).reshape(m, n)[rows, cols], ref) <= 1e-2
+    ga, gb = (Guarded(gpu, np.concatenate([np.zeros(1, np.uint8), h])) for h in (a, b))
+    off = Guarded(gpu, np.full(m * n + 1, 0x7FDE, np.uint16))
+    kern.gemm_fp8_nt(ga.body.view(1, m * k), gb.body.view(1, n * k), sa, sb,
+                     off.body.view(1, m * n), m, n, k)
+    assert off.guards_intact() and ga.unchanged() and gb.unchanged()
+    assert_same(off.download()[1:], got, "offset operands vs aligned")
+
+
 # K a multiple of 16 but not of 128: the pipelined tiles with a partial last
 # stage (its chunks past K load zeros) on the 128x128 form (three and two
 # stages), the 256x256 tile and its tail round
