@@ -87,6 +87,20 @@ struct ScalarBase {
   }
 };
 
+// A 16-byte piece shifted down by `bits` (0 .. 127), zeros shifted in; 128 and
+// more leave it anyhow.
+FE2O3_DEVICE u32x4_t shift_down(u32x4_t v, uint32_t bits) {
+  uint64_t lo = v[0] | (uint64_t)v[1] << 32, hi = v[2] | (uint64_t)v[3] << 32;
+  if (bits >= 64u) {
+    lo = hi >> (bits & 63u);
+    hi = 0;
+  } else if (bits != 0u) {
+    lo = lo >> bits | hi << (64u - bits);
+    hi >>= bits;
+  }
+  return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
 // The 16-byte piece at byte `at` of a row of `bytes` bytes, zeros past its
 // end.  Nothing past the row is read: a piece that straddles the end comes
 // from the row's last 16 bytes, shifted down; a row shorter than that is read
@@ -96,30 +110,17 @@ FE2O3_DEVICE u32x4_t load_end(const uint8_t* row, Off at, Off bytes) {
   if (at >= bytes) return u32x4_t{0, 0, 0, 0};
   if (bytes - at >= 16u) return load16(row + at);
   const uint32_t left = (uint32_t)(bytes - at);
+  if (bytes >= 16u) return shift_down(load16(row + (bytes - 16u)), 8u * (16u - left));
   uint64_t lo = 0, hi = 0;
-  if (bytes >= 16u) {
-    const u32x4_t v = load16(row + (bytes - 16u));
-    lo = v[0] | (uint64_t)v[1] << 32;
-    hi = v[2] | (uint64_t)v[3] << 32;
-    const uint32_t sh = 8u * (16u - left);  // 8 .. 120
-    if (sh >= 64u) {
-      lo = hi >> (sh - 64u);
-      hi = 0;
-    } else {
-      lo = lo >> sh | hi << (64u - sh);
-      hi >>= sh;
-    }
-  } else {
-    // at most 15 bytes of a whole row: independent loads, no load waits
+  // at most 15 bytes of a whole row: independent loads, no load waits
 #pragma unroll
-    for (uint32_t i = 0; i < 16u; i += ELEM) {
-      if (i >= left) continue;
-      uint64_t v;
-      if constexpr (ELEM == 2) v = *reinterpret_cast<const uint16_t*>(row + at + i);
-      else v = row[at + i];
-      if (i < 8u) lo |= v << (8u * i);
-      else hi |= v << (8u * i - 64u);
-    }
+  for (uint32_t i = 0; i < 16u; i += ELEM) {
+    if (i >= left) continue;
+    uint64_t v;
+    if constexpr (ELEM == 2) v = *reinterpret_cast<const uint16_t*>(row + at + i);
+    else v = row[at + i];
+    if (i < 8u) lo |= v << (8u * i);
+    else hi |= v << (8u * i - 64u);
   }
   return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
 }

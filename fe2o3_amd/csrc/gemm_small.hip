@@ -3,14 +3,18 @@
 //   * tiled_gemm_lds_slice1 / moe_expert_gemm_bf16_m16_n16_k16: one 16x16x16
 //     bf16 tile, one wave64, LDS staging, one v_mfma_f32_16x16x32_bf16 with
 //     the upper K half zero;
-//   * tiled_gemm_general_v1: any m, n, k, strides, alpha/beta; 64x64 output
-//     tiles per 256-thread workgroup, guarded zero-filled loads, MFMA
-//     16x16x32 bf16, unfused alpha/beta epilogue;
+//   * tiled_gemm_general_v1: any m, n, k, strides, alpha/beta; the pipelined
+//     tiles of gemm_pipe.hpp, or 64x64 tiles through registers for small
+//     outputs and operands of any alignment; unfused alpha/beta epilogue.  The
+//     reference's two global-transfer schedules
+//     (crates/dialect-schedule/src/general_gemm.rs:13-38) are two entry points
+//     to the same kernels;
 //   * scalar_gemm_v1: f32, the reference's per-output sequential unfused
 //     recurrence, LDS-tiled and register-blocked (4x4 outputs per thread),
 //     bit-identical to the scalar oracle.
 #include "common.hpp"
 #include "gemm_core.hpp"
+#include "gemm_direct.hpp"
 #include "gemm_pipe.hpp"
 #include "internal.hpp"
 
@@ -101,107 +105,6 @@ __global__ void __launch_bounds__(256) zero_fill_kernel(float* __restrict__ c, u
     c[i] = 0.0f;
 }
 
-// ---- general bf16 GEMM with alpha/beta -----------------------------------------------
-// C[r*ldc+j] = alpha * (A B)[r][j] + beta * C[r*ldc+j] for r < m, j < n.
-// A row-major (lda), B row-major [k][n] (ldb).  Workgroup tile 64x64, K step
-// 32, four waves in a 2x2 arrangement each owning 32x32 (2x2 MFMA tiles).
-constexpr int G_BM = 64, G_BN = 64, G_BK = 32;
-constexpr int G_LDK = G_BK + 8;  // padded LDS row (bf16 elements), 80 bytes
-
-// Two global-transfer schedules of the same kernel, as the reference has two
-// (crates/dialect-schedule/src/general_gemm.rs:13-38): VEC_A = false stages
-// every A and B element with a masked scalar load; VEC_A = true loads each
-// full, in-range, 8-byte-aligned group of 4 A elements with one 8-byte load
-// and falls back to masked scalar loads for the rest (tails, misaligned
-// rows); B stays scalar.  The staged tiles, hence the results, are the same.
-template <bool VEC_A>
-__global__ void __launch_bounds__(256) gemm_general_kernel(
-    const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, float* __restrict__ c,
-    uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, float alpha,
-    float beta) {
-  __shared__ __attribute__((aligned(16))) uint16_t a_lds[G_BM * G_LDK];
-  __shared__ __attribute__((aligned(16))) uint16_t bt_lds[G_BN * G_LDK];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const uint64_t row0 = (uint64_t)blockIdx.y * G_BM, col0 = (uint64_t)blockIdx.x * G_BN;
-  f32x4_t acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const uint32_t phases = (k + G_BK - 1) / G_BK;
-  for (uint32_t ph = 0; ph < phases; ++ph) {
-    const uint64_t k0 = (uint64_t)ph * G_BK;
-    // A: thread t loads row t/4, depths (t%4)*8 .. +7 (zero outside m x k)
-    {
-      const int r = t >> 2, d0 = (t & 3) * 8;
-      const uint64_t gr = row0 + r;
-#pragma unroll
-      for (int v = 0; v < 2; ++v) {
-        const uint64_t gd0 = k0 + d0 + 4 * v;
-        const uint64_t idx = gr * lda + gd0;
-        if (VEC_A && gr < m && gd0 + 4 <= k && (((uintptr_t)(a + idx)) & 7u) == 0) {
-          *reinterpret_cast<uint2*>(a_lds + r * G_LDK + d0 + 4 * v) =
-              *reinterpret_cast<const uint2*>(a + idx);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const uint64_t gd = gd0 + e;
-            a_lds[r * G_LDK + d0 + 4 * v + e] = (gr < m && gd < k) ? a[gr * lda + gd] : (uint16_t)0;
-          }
-        }
-      }
-    }
-    // B: thread t loads depth t/8, columns (t%8)*8 .. +7, stored transposed
-    {
-      const int d = t >> 3, n0 = (t & 7) * 8;
-      const uint64_t gd = k0 + d;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint64_t gc = col0 + n0 + e;
-        bt_lds[(n0 + e) * G_LDK + d] = (gd < k && gc < n) ? b[gd * ldb + gc] : (uint16_t)0;
-      }
-    }
-    __syncthreads();
-    const int rc = lane & 15, chunk = lane >> 4;
-    bf16x8_t af[2], bf[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      af[i] = *reinterpret_cast<const bf16x8_t*>(a_lds + (wm * 32 + i * 16 + rc) * G_LDK + chunk * 8);
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      bf[j] = *reinterpret_cast<const bf16x8_t*>(bt_lds + (wn * 32 + j * 16 + rc) * G_LDK + chunk * 8);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
-  }
-  // epilogue: alpha * acc and beta * C rounded separately, then added
-  // (examples/tiled_gemm_v1/src/numerical_contract.rs:310-331 order).
-  {
-#pragma clang fp contract(off)
-    const int col_in = lane & 15, row_in = (lane >> 4) * 4;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint64_t gr = row0 + wm * 32 + i * 16 + row_in + e;
-          const uint64_t gc = col0 + wn * 32 + j * 16 + col_in;
-          if (gr < m && gc < n) {
-            float* p = c + gr * ldc + gc;
-            const float product = alpha * acc[i][j][e];
-            const float initial = beta * *p;
-            *p = product + initial;
-          }
-        }
-  }
-}
-
 // ---- scalar f32 GEMM (sequential, unfused) -----------------------------------------
 // Workgroup tile 16x16, 256 threads, one output per thread, whose accumulator
 // follows acc = acc + a*b over t = 0..k-1 in order.  One output per thread
@@ -281,8 +184,6 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_moe_expert_gemm_bf16_m16_n16_k16_v1", "tile16_bf16_kernel", (const void*)tile16_bf16_kernel, 64, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_tiled_gemm_v1", "tiled_v1_kernel", (const void*)tiled_v1_kernel, 64, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_tiled_gemm_v1", "zero_fill_kernel", (const void*)zero_fill_kernel, 256, 0}),
-    fe2o3_host::KernelRegistrar({"fe2o3_tiled_gemm_general_v1", "gemm_general_kernel<false>", (const void*)gemm_general_kernel<false>, 256, 0}),
-    fe2o3_host::KernelRegistrar({"fe2o3_tiled_gemm_general_vector_a_v1", "gemm_general_kernel<true>", (const void*)gemm_general_kernel<true>, 256, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_scalar_gemm_v1", "scalar_gemm_kernel", (const void*)scalar_gemm_kernel, 256, 0})};
 
 }  // namespace
@@ -352,56 +253,60 @@ namespace {
 constexpr int kGpRowBytes = 128, kGpStages = 2;
 constexpr int kGpSmem = kGpStages * 2 * gemm_pipe::Geo<kGpRowBytes>::kTileBytes;  // 128 KiB
 
-// C = alpha * acc + beta * C over one tile of TM x TN outputs (rows x cols
-// valid), accumulators Acc16T<RB, CB> of waves holding RPW rows by CPW
-// columns.  Per 16-row block: every C load of the lane first (one wait),
-// then the products and stores.  Whole-width tiles of a 16-byte aligned C
-// with ldc % 4 == 0 move 4 columns per access; otherwise element by element,
-// the loads of columns past n clamped to the last valid one (not stored).
+// C = alpha * acc + beta * C over one tile of TN columns (rows x cols valid),
+// accumulators Acc16T<RB, CB> of waves holding RPW rows by CPW columns.  Per
+// 16-row block: every C load of the lane first (one wait), then the products
+// and stores.  A lane's 4 columns move as one access of 16 bytes at C's own
+// 4-byte alignment (gfx950 global accesses of four dwords need no more).  In
+// a tile that the last column cuts, the group it cuts (and those past it)
+// moves element by element, loads clamped to that column.
+typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+
 template <int TN, int RPW, int CPW, class Acc>
 FE2O3_DEVICE void general_epilogue(const Acc& acc, float* c_tile, uint32_t rows, uint32_t cols,
-                                   uint32_t ldc, bool c_aligned, float alpha, float beta) {
+                                   uint32_t ldc, float alpha, float beta) {
 #pragma clang fp contract(off)
   constexpr int RB = RPW / 16, CB = CPW / 16;
   const uint32_t row0 = gemm_pipe::acc16_row0<RPW>(), col0 = gemm_pipe::acc16_col0<CPW>();
-  const bool vec = cols == (uint32_t)TN && ldc % 4u == 0u && c_aligned;
+  auto combined = [&](int i, int j, const f32x4_t& cv) {
+    f32x4_t y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float product = alpha * acc.v[i][j][e];
+      const float initial = beta * cv[e];
+      y[e] = product + initial;
+    }
+    return y;
+  };
 #pragma unroll
   for (int i = 0; i < RB; ++i) {
     const uint32_t r = row0 + 16u * i;
     if (r >= rows) continue;
     float* out = c_tile + (uint64_t)r * ldc;
-    if (vec) {
-      f32x4_t cv[CB];
+    f32x4_t cv[CB];
+    if (cols == (uint32_t)TN) {
 #pragma unroll
-      for (int j = 0; j < CB; ++j) cv[j] = *reinterpret_cast<const f32x4_t*>(out + col0 + 16u * j);
+      for (int j = 0; j < CB; ++j)
+        cv[j] = *reinterpret_cast<const f32x4_any_t*>(out + col0 + 16u * j);
+#pragma unroll
+      for (int j = 0; j < CB; ++j)
+        *reinterpret_cast<f32x4_any_t*>(out + col0 + 16u * j) = combined(i, j, cv[j]);
+    } else {
 #pragma unroll
       for (int j = 0; j < CB; ++j) {
-        f32x4_t y;
+        const uint32_t col = col0 + 16u * j;
+        if (col + 4u <= cols) {
+          *reinterpret_cast<f32x4_any_t*>(out + col) =
+              combined(i, j, *reinterpret_cast<const f32x4_any_t*>(out + col));
+        } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float product = alpha * acc.v[i][j][e];
-          const float initial = beta * cv[j][e];
-          y[e] = product + initial;
+          for (int e = 0; e < 4; ++e) cv[j][e] = out[min(col + e, cols - 1u)];
+          const f32x4_t y = combined(i, j, cv[j]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col + e < cols) out[col + e] = y[e];
         }
-        *reinterpret_cast<f32x4_t*>(out + col0 + 16u * j) = y;
       }
-    } else {
-      float cv[CB][4];
-#pragma unroll
-      for (int j = 0; j < CB; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) cv[j][e] = out[min(col0 + 16u * j + e, cols - 1u)];
-#pragma unroll
-      for (int j = 0; j < CB; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t col = col0 + 16u * j + e;
-          if (col < cols) {
-            const float product = alpha * acc.v[i][j][e];
-            const float initial = beta * cv[j][e];
-            out[col] = product + initial;
-          }
-        }
     }
   }
 }
@@ -409,7 +314,7 @@ FE2O3_DEVICE void general_epilogue(const Acc& acc, float* c_tile, uint32_t rows,
 // k: A's k extent and the K loop's; kb: B's rows (its k extent), at most k
 // and more than k - 64.  KT: k or kb is not a multiple of 64; A's chunks
 // past k and B's rows past kb load zeros (gemm_pipe::Rows MASK), so each
-// accumulator gets the staged kernel's zero-padded 32-k blocks.
+// accumulator gets the register tiles' zero-padded 32-k blocks.
 template <bool KT = false>
 __global__ void __launch_bounds__(256, 1) gemm_general_pipe_kernel(
     const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, float* __restrict__ c,
@@ -426,7 +331,7 @@ __global__ void __launch_bounds__(256, 1) gemm_general_pipe_kernel(
   gemm_pipe::Acc16 acc;
   gemm_pipe::mainloop<gemm_pipe::Bf16MmaKN, kGpRowBytes, kGpStages, KT>(ar, br, k, smem, acc);
   general_epilogue<256, 128, 128>(acc, c + (uint64_t)tm * 256u * ldc + (uint64_t)tn * 256u, rows,
-                                  cols, ldc, ((uintptr_t)c & 15u) == 0u, alpha, beta);
+                                  cols, ldc, alpha, beta);
 }
 
 // The same GEMM on 128 x 128 tiles (Bf16MmaKN64), for problems whose
@@ -462,7 +367,210 @@ __global__ void __launch_bounds__(256, STAGES == 2 ? 2 : 1) gemm_general_pipe128
   gemm_pipe::Bf16MmaKN64::Acc acc;
   gemm_pipe::mainloop<gemm_pipe::Bf16MmaKN64, kGpRowBytes, STAGES, KT>(ar, br, k, smem, acc);
   general_epilogue<128, 64, 64>(acc, c + (uint64_t)tm * 128u * ldc + (uint64_t)tn * 128u, rows,
-                                cols, ldc, ((uintptr_t)c & 15u) == 0u, alpha, beta);
+                                cols, ldc, alpha, beta);
+}
+
+// ---- 64 x 64 tiles through registers: any alignment, any K ------------------------------
+// For outputs too small for the pipelined tiles to fill the device, and for
+// operands they would need repacked: 16-byte loads at the operand's own
+// alignment into registers, kGsDepth steps of 64 k ahead, then through LDS
+// (two buffers, one barrier per step).  Four waves, 2 x 2, own 32 x 32
+// outputs each.  B's [k][n] rows are read back with the transposing LDS read,
+// as in gemm_pipe::Bf16MmaKN.  Every accumulator gets the MFMAs of the
+// pipelined tiles in the same k order over the same zero-padded 32-k blocks,
+// so C is bit-identical to theirs.
+//
+// Bound by LDS, which moves three bytes per byte loaded at this tile (two
+// steps of 64 k take 0.6 us alone on a CU); against the masked scalar loads
+// it replaces 2000 x 100 x 2000 takes 18.6 us for 177.7, and against
+// repacking for the pipelined tile 1000 x 1500 x 700 takes 15.1 for 30.1.
+constexpr int kGsThreads = 256, kGsDepth = 4;
+constexpr uint32_t kGsBuf = 64 * 128;  // bytes of one operand's step: 64 rows of 128
+
+// 16-byte piece position of B's k row in LDS: the rows that one half wave of
+// a transposing read touches (8g + q, g < 2, q < 4) fall on distinct banks
+FE2O3_DEVICE uint32_t gs_swz_b(uint32_t krow) {
+  return 2u * (((krow >> 1) & 1u) | (((krow >> 3) & 1u) << 1));
+}
+
+// How a tile reads B's columns: all 64 valid; cut by the last column; or a
+// row of B shorter than a 16-byte piece.
+enum class Cols { whole, cut, narrow };
+
+template <Cols MODE>
+FE2O3_DEVICE void general_tile(const uint16_t* __restrict__ a, const uint16_t* __restrict__ b,
+                               float* __restrict__ c, uint32_t n, uint32_t k, uint32_t lda,
+                               uint32_t ldb, uint32_t ldc, float alpha, float beta, uint32_t tm,
+                               uint32_t tn, uint32_t rows, uint32_t cols, uint8_t* smem) {
+  using G = gemm_pipe::Geo<128>;
+  using gemm_direct::load16;
+  using gemm_direct::load_end;
+  const uint32_t t = threadIdx.x, lane = t & 63u;
+  const uint32_t wave = gemm_pipe::wave_id();
+  // this thread's pieces of a step: place pc of rows pr and pr + 32 of A's
+  // 64 (rows past m repeat the last) and of B's 64 k rows.  A piece that the
+  // last column cuts is read 8 columns before it and shifted down; one past
+  // it reads the same, and its columns are not stored.
+  const uint32_t pr = t >> 3, pc = t & 7u;
+  const uint32_t b_first = tn * 64u + 8u * pc;
+  const uint32_t b_read = MODE == Cols::whole ? b_first
+                          : MODE == Cols::cut ? min(b_first, n - 8u) : 0u;
+  const uint32_t b_shift = 16u * (b_first - b_read);  // bits
+  const uint8_t* row_a[2];
+  const uint8_t* ap[2];
+  const uint8_t* bp[2];
+  uint32_t aw[2], bw[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t r = pr + 32u * h;
+    row_a[h] = reinterpret_cast<const uint8_t*>(
+        a + ((uint64_t)tm * 64u + min(r, rows - 1u)) * lda);
+    ap[h] = row_a[h] + 16u * pc;
+    bp[h] = reinterpret_cast<const uint8_t*>(b + (uint64_t)r * ldb + b_read);
+    aw[h] = r * 128u + ((pc ^ G::swz(r)) << 4);
+    bw[h] = 2u * kGsBuf + r * 128u + ((pc ^ gs_swz_b(r)) << 4);
+  }
+  const uint64_t b_step = (uint64_t)ldb * 128u;
+  const uint32_t steps = k / 64u, k_rest = k % 64u;
+  // the partial last step, fetched first, without a branch, and kept: A's
+  // pieces that K cuts (or that lie past it) are read 16 bytes before the
+  // row's end, B's rows past K repeat the last; end_a and end_b make of them
+  // what the step needs, zeros past K
+  u32x4_t last_a[2], last_b[2];
+  const bool short_row = k < 8u || MODE == Cols::narrow;  // no whole piece in a row
+  const uint64_t a_at = (uint64_t)steps * 128u + 16u * pc;
+  const uint64_t a_last = min(a_at, (uint64_t)k * 2u - 16u);
+  if (k_rest != 0u && !short_row) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t r = pr + 32u * h, rb = min(r, k_rest - 1u);
+      last_a[h] = load16(row_a[h] + a_last);
+      last_b[h] = load16(bp[h] + steps * b_step - (uint64_t)(r - rb) * ldb * 2u);
+    }
+  }
+  auto end_a = [&](int h) {
+    if (short_row) return load_end<2, uint64_t>(row_a[h], a_at, (uint64_t)k * 2u);
+    const uint64_t past = a_at - a_last;
+    return past < 16u ? gemm_direct::shift_down(last_a[h], 8u * (uint32_t)past) : u32x4_t{};
+  };
+  auto end_b = [&](int h) {
+    const uint32_t r = pr + 32u * h;
+    if (r >= k_rest) return u32x4_t{};
+    if (short_row)
+      return load_end<2, uint64_t>(
+          reinterpret_cast<const uint8_t*>(b + ((uint64_t)steps * 64u + r) * ldb),
+          (uint64_t)b_first * 2u, (uint64_t)n * 2u);
+    return MODE == Cols::cut ? gemm_direct::shift_down(last_b[h], b_shift) : last_b[h];
+  };
+
+  gemm_pipe::Acc16T<2, 2> acc;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc.v[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  constexpr int D = MODE == Cols::narrow ? 2 : kGsDepth;
+  u32x4_t ra[D][2], rb[D][2];
+  uint32_t loaded = 0;  // the next step to load; the last one is loaded again past it
+  auto load = [&](int s) {
+    __builtin_amdgcn_sched_barrier(0);
+    const bool more = loaded + 1u < steps;
+    ++loaded;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      ra[s][h] = load16(ap[h]);
+      if constexpr (MODE == Cols::narrow)
+        rb[s][h] = load_end<2, uint64_t>(bp[h], (uint64_t)b_first * 2u, (uint64_t)n * 2u);
+      else
+        rb[s][h] = load16(bp[h]);
+      ap[h] += more ? 128u : 0u;
+      bp[h] += more ? b_step : 0u;
+    }
+  };
+  auto put = [&](uint32_t buf, int h, u32x4_t pa, u32x4_t pb) {
+    *reinterpret_cast<u32x4_t*>(smem + buf * kGsBuf + aw[h]) = pa;
+    *reinterpret_cast<u32x4_t*>(smem + buf * kGsBuf + bw[h]) = pb;
+  };
+  auto put_set = [&](uint32_t buf, int s) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      put(buf, h, ra[s][h],
+          MODE == Cols::cut ? gemm_direct::shift_down(rb[s][h], b_shift) : rb[s][h]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // fragments: wave rows wm * 32, columns wn * 32
+  const uint32_t wm = wave >> 1, wn = wave & 1u, lr = lane & 15u, g = lane >> 4;
+  auto compute = [&](uint32_t buf) {
+    const uint8_t* la = smem + buf * kGsBuf;
+    const uint8_t* lb = la + 2u * kGsBuf;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8_t fa[2], fb[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint32_t r = wm * 32u + 16u * i + lr;
+        fa[i] =
+            *reinterpret_cast<const bf16x8_t*>(la + r * 128u + (((4u * ks + g) ^ G::swz(r)) << 4));
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const uint32_t kr = 32u * ks + 8u * g + (lr >> 2);
+        const uint32_t piece = wn * 4u + 2u * j + ((lr & 3u) >> 1), off = (lr & 1u) * 8u;
+        const bf16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+            (lds_bf16x4_t*)(lb + kr * 128u + ((piece ^ gs_swz_b(kr)) << 4) + off));
+        const bf16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(
+            (lds_bf16x4_t*)(lb + (kr + 4u) * 128u + ((piece ^ gs_swz_b(kr + 4u)) << 4) + off));
+        fb[j] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc.v[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc.v[i][j], 0, 0, 0);
+    }
+  };
+  // Step t is in buffer t % 2 when its turn comes.  It writes step t + 1 into
+  // the other buffer, which every wave left at the barrier before, and loads
+  // step t + D into the set that step t came from.
+  if (steps != 0u) {
+#pragma unroll
+    for (int s = 0; s < D; ++s) load(s);
+    put_set(0, 0);
+    lds_barrier();
+    for (uint32_t t0 = 0; t0 < steps; t0 += D) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        if (t0 + s >= steps) break;
+        put_set((s + 1) & 1, (s + 1) % D);
+        load(s);
+        compute(s & 1);
+        lds_barrier();
+      }
+    }
+  }
+  if (k_rest != 0u) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) put(steps & 1u, h, end_a(h), end_b(h));
+    lds_barrier();
+    compute(steps & 1u);
+  }
+  general_epilogue<64, 32, 32>(acc, c + (uint64_t)tm * 64u * ldc + (uint64_t)tn * 64u, rows, cols,
+                               ldc, alpha, beta);
+}
+
+__global__ void __launch_bounds__(kGsThreads, 3) gemm_general_kernel(
+    const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, float* __restrict__ c,
+    uint32_t m, uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb, uint32_t ldc, float alpha,
+    float beta, uint32_t xcds) {
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[4 * kGsBuf];  // A0 A1 B0 B1
+  uint32_t tm, tn;
+  gemm_core::xcd_tile_order(blockIdx.x, (m + 63u) / 64u, (n + 63u) / 64u, xcds, &tm, &tn);
+  const uint32_t rows = min(64u, m - tm * 64u), cols = min(64u, n - tn * 64u);
+  if (n < 8u)
+    general_tile<Cols::narrow>(a, b, c, n, k, lda, ldb, ldc, alpha, beta, tm, tn, rows, cols, smem);
+  else if (cols < 64u)
+    general_tile<Cols::cut>(a, b, c, n, k, lda, ldb, ldc, alpha, beta, tm, tn, rows, cols, smem);
+  else
+    general_tile<Cols::whole>(a, b, c, n, k, lda, ldb, ldc, alpha, beta, tm, tn, rows, cols, smem);
 }
 
 // ---- operands the pipelined tile cannot read directly ---------------------------
@@ -511,6 +619,7 @@ __global__ void __launch_bounds__(256) repack_rows_kernel(const uint16_t* __rest
   fe2o3_host::KernelRegistrar({entry, "gemm_general_pipe128_kernel<3, k tail>", (const void*)gemm_general_pipe128_kernel<3, false, true>, 256, kGp64Smem<3>}), \
   fe2o3_host::KernelRegistrar({entry, "gemm_general_pipe128_kernel<2, tail, k tail>", (const void*)gemm_general_pipe128_kernel<2, true, true>, 256, kGp64Smem<2>}), \
   fe2o3_host::KernelRegistrar({entry, "gemm_general_pipe128_kernel<3, tail, k tail>", (const void*)gemm_general_pipe128_kernel<3, true, true>, 256, kGp64Smem<3>}), \
+  fe2o3_host::KernelRegistrar({entry, "gemm_general_kernel", (const void*)gemm_general_kernel, kGsThreads, 0}), \
   fe2o3_host::KernelRegistrar({entry, "repack_rows_kernel", (const void*)repack_rows_kernel, 256, 0})
 
 const fe2o3_host::KernelRegistrar kRegisteredPipe[] = {
@@ -586,11 +695,26 @@ bool b_direct(const uint16_t* b, uint32_t k, uint32_t ldb) {
 }
 
 // Operands the tile cannot read in place are repacked (repack_rows_kernel)
-// when M and N are at least one 128 x 128 tile; smaller problems stay on
-// the staged kernel.
+// when M and N are at least one 128 x 128 tile; smaller problems, and those
+// below register_tiles' line, stay on the register tiles.
 constexpr uint32_t kRepackMin = 128;
 
-template <bool VEC_A>
+// Whether the 64 x 64 register tiles take a GEMM that the pipelined tiles
+// could run, in place (`in_place`) or on repacked operands.  Both sides in us
+// (pipelined, register); `rounds` is what the busiest CU walks, in steps.
+//   in place       1024 x 1024 x 1024  11.2, 10.2    1024 x 512 x 2048   15.7, 15.9
+//                  1200 x 1200 x 256    9.3,  7.7    1024 x 2048 x 512    9.4,  9.8
+//                  512^3                7.6,  5.4    1024 x 1024 x 4096  26.3, 28.9
+//   repacked       1000 x 1500 x 700   30.3, 15.1    1500^3              31.9, 32.9
+//                  2048 x 2048 x 512   27.6, 21.7    2000 x 2000 x 1000  30.1, 32.2
+//                  1024 x 1024 x 4096  40.9, 35.3    512 x 512 x 8192    62.2, 63.9
+bool register_tiles(uint32_t m, uint32_t n, uint32_t k, bool in_place, uint32_t cus) {
+  const uint64_t tiles = (((uint64_t)m + 63u) / 64u) * (((uint64_t)n + 63u) / 64u);
+  const uint64_t rounds = (tiles + cus - 1u) / cus * (((uint64_t)k + 63u) / 64u);
+  if (in_place) return 2u * tiles <= 3ull * cus && rounds <= 32u;
+  return rounds <= 48u || (tiles <= cus && rounds <= 96u);
+}
+
 int32_t general_gemm(const uint16_t* a, uint64_t a_len, const uint16_t* b, uint64_t b_len,
                      float* c, uint64_t c_len, uint32_t m, uint32_t n, uint32_t k, uint32_t lda,
                      uint32_t ldb, uint32_t ldc, float alpha, float beta, void* stream) {
@@ -607,14 +731,14 @@ int32_t general_gemm(const uint16_t* a, uint64_t a_len, const uint16_t* b, uint6
   if ((ea && !a) || (eb && !b) || !c) return FE2O3_ERR_NULL;
   const bool ad = k != 0 && a_direct(a, k, lda), bd = k != 0 && b_direct(b, k, ldb);
   const bool repack = k != 0 && (!ad || !bd) && m >= kRepackMin && n >= kRepackMin;
-  if (k != 0 && ((ad && bd) || repack)) {
+  tile_plan::Topology topo;
+  const int32_t topo_rc = fe2o3_host::device_topology(&topo);
+  if (topo_rc != FE2O3_OK) return topo_rc;
+  if (k != 0 && ((ad && bd) || repack) && !register_tiles(m, n, k, ad && bd, topo.cus)) {
     // every kernel's LDS limit is raised before anything is launched, so a
     // failure leaves C untouched
     const int32_t lds_rc = set_general_lds();
     if (lds_rc != FE2O3_OK) return lds_rc;
-    tile_plan::Topology topo;
-    const int32_t topo_rc = fe2o3_host::device_topology(&topo);
-    if (topo_rc != FE2O3_OK) return topo_rc;
     const tile_plan::Plan plan = tile_plan::plan(m, n, topo);
     if (plan.grid > 0x7fffffffu || plan.tail_grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
     hipStream_t s = (hipStream_t)stream;
@@ -635,10 +759,10 @@ int32_t general_gemm(const uint16_t* a, uint64_t a_len, const uint16_t* b, uint6
     void* scratch = nullptr;
     int32_t rc = fe2o3_host::scratch_alloc(&scratch, (a_elems + b_elems) * 2, s);
     if (rc != FE2O3_OK) {
-      // no stream-ordered scratch on this device or process: the staged
+      // no stream-ordered scratch on this device or process: the register
       // kernel reads the operands as they are
       (void)hipGetLastError();
-      goto staged;
+      goto in_registers;
     }
     uint16_t* ap = static_cast<uint16_t*>(scratch);
     uint16_t* bp = ap + a_elems;
@@ -666,11 +790,11 @@ int32_t general_gemm(const uint16_t* a, uint64_t a_len, const uint16_t* b, uint6
     const int32_t free_rc = fe2o3_host::scratch_free(scratch, s);
     return rc != FE2O3_OK ? rc : free_rc;
   }
-staged:
-  dim3 grid((n + G_BN - 1) / G_BN, (m + G_BM - 1) / G_BM);
-  if (grid.y > 65535u) return FE2O3_ERR_SHAPE;
-  gemm_general_kernel<VEC_A><<<grid, 256, 0, (hipStream_t)stream>>>(a, b, c, m, n, k, lda, ldb,
-                                                                    ldc, alpha, beta);
+in_registers:
+  const uint64_t tiles = (((uint64_t)m + 63u) / 64u) * (((uint64_t)n + 63u) / 64u);
+  if (((uint64_t)m + 63u) / 64u > 65535u || tiles > 0x7fffffffu) return FE2O3_ERR_SHAPE;
+  gemm_general_kernel<<<(unsigned)tiles, kGsThreads, 0, (hipStream_t)stream>>>(
+      a, b, c, m, n, k, lda, ldb, ldc, alpha, beta, topo.xcds);
   return fe2o3_host::after_launch();
 }
 
@@ -695,7 +819,7 @@ int32_t fe2o3_tiled_gemm_general_v1(const uint16_t* a, uint64_t a_len, const uin
                                     uint32_t n, uint32_t k, uint32_t lda, uint32_t ldb,
                                     uint32_t ldc, float alpha, float beta, void* stream) {
   FE2O3_ENTRY("fe2o3_tiled_gemm_general_v1");
-  return general_gemm<false>(a, a_len, b, b_len, c, c_len, m, n, k, lda, ldb, ldc, alpha, beta,
+  return general_gemm(a, a_len, b, b_len, c, c_len, m, n, k, lda, ldb, ldc, alpha, beta,
                              stream);
 }
 
@@ -705,7 +829,7 @@ int32_t fe2o3_tiled_gemm_general_vector_a_v1(const uint16_t* a, uint64_t a_len,
                                              uint32_t lda, uint32_t ldb, uint32_t ldc,
                                              float alpha, float beta, void* stream) {
   FE2O3_ENTRY("fe2o3_tiled_gemm_general_vector_a_v1");
-  return general_gemm<true>(a, a_len, b, b_len, c, c_len, m, n, k, lda, ldb, ldc, alpha, beta,
+  return general_gemm(a, a_len, b, b_len, c, c_len, m, n, k, lda, ldb, ldc, alpha, beta,
                             stream);
 }
 

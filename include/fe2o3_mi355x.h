@@ -228,10 +228,10 @@ int32_t fe2o3_tiled_gemm_general_v1(const uint16_t *a, uint64_t a_len,
  * schedule, VectorizedAOnlyBf16GlobalTransferV1
  * (crates/dialect-schedule/src/general_gemm.rs:13-38; the hardware harness
  * runs both schedules on the same seven profiles,
- * examples/tiled_gemm_general_v1/hardware-harness/src/lib.rs:135-253): A is
- * staged with one 8-byte load per full, in-range, 8-byte-aligned group of 4
- * elements and masked scalar loads elsewhere; B stays scalar.  Results are
- * bit-identical to fe2o3_tiled_gemm_general_v1. */
+ * examples/tiled_gemm_general_v1/hardware-harness/src/lib.rs:135-253).  The
+ * schedules differ in how operand elements are transferred, not in any
+ * result; here both entry points run the same kernels, which move whole
+ * 16-byte pieces of A and B. */
 int32_t fe2o3_tiled_gemm_general_vector_a_v1(const uint16_t *a, uint64_t a_len,
                                              const uint16_t *b, uint64_t b_len,
                                              float *c, uint64_t c_len, uint32_t m,

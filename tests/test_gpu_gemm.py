@@ -220,6 +220,20 @@ def test_general_pipelined_tile_matches_staged_kernel(gpu, oracle, dims, strides
     assert rel_err(rows, out) <= 1e-5
 
 
+# the 64x64 register tiles: rows and columns of less than a piece, cut tiles,
+# K from part of a piece to several rounds of the load ring and its remainders;
+# and outputs just past the line where the pipelined tiles take over, in place
+# and repacked (their strips run on the register tiles)
+@pytest.mark.parametrize("dims,strides", [
+    ((70, 5, 100), (103, 6, 5)), ((65, 8, 7), (8, 8, 9)), ((33, 1, 1), (1, 1, 1)),
+    ((64, 63, 63), (64, 64, 64)), ((129, 65, 65), (70, 67, 66)), ((66, 71, 129), (131, 72, 71)),
+    ((100, 200, 256), (256, 200, 200)), ((100, 200, 321), (323, 205, 203)),
+    ((130, 72, 450), (450, 75, 72)), ((200, 7, 333), (335, 7, 7)),
+    ((1300, 1300, 1096), (1104, 1304, 1310)), ((1300, 1310, 2051), (2055, 1311, 1313))])
+def test_general_register_tiles(gpu, oracle, dims, strides):
+    test_general_pipelined_tile_matches_staged_kernel(gpu, oracle, dims, strides, 1.25, -0.5)
+
+
 @pytest.mark.parametrize("m,n,k", [(6144, 6144, 128), (6000, 6100, 192)])
 def test_general_tail_round_matches_row_blocks(gpu, m, n, k):
     """576 tiles of 256x256 (the last 64 as 128x128 quarters after two full
