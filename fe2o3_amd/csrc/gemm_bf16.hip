@@ -42,7 +42,7 @@ constexpr int kFastSmem = kStages * 2 * gemm_pipe::Geo<kRowBytes>::kTileBytes;  
 // EDGE: M or N is not a multiple of 256; the grid covers ceil(M/256) x
 // ceil(N/256) tiles, operand rows past M (N) repeat the last valid row
 // (their products reach only outputs that are not stored), and each tile
-// stores only its valid rows and columns, element by element.
+// stores only its valid rows and columns (gemm_pipe::store_bf16_edge).
 //
 // KT: K is a multiple of 8 but not of 64; the last stage is partial and its
 // chunks past K load zeros (gemm_pipe::Rows MASK), so C is bit-identical to

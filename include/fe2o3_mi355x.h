@@ -257,7 +257,7 @@ int32_t fe2o3_scalar_gemm_v1(const float *a, uint64_t a_len, const float *b,
  * (128x128 for small grids) runs whenever k is a multiple of 8 (k*512 <
  * 2^31) and A and B are 16-byte aligned, with a partial last k stage when k
  * is not a multiple of 64: whole tiles when m and n are multiples of 256
- * and C is 16-byte aligned, edge tiles (element-wise masked stores)
+ * and C is 16-byte aligned, edge tiles (masked stores at any alignment)
  * otherwise.  For other k or alignments, when m and n are at least 128, the
  * rows that cannot be read in place are first copied into aligned rows of
  * k rounded up to 8 (zeros past k) in stream-ordered scratch from the

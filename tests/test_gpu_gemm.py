@@ -460,7 +460,9 @@ def test_gemm_bf16_nt_direct_forms(gpu, oracle, m, n, k):
 # for those too)
 @pytest.mark.parametrize("m,n,k", [(1024, 1024, 64), (1024, 1024, 128), (1000, 1032, 192),
                                    (1024, 1024, 320), (1024, 1024, 8), (1024, 1024, 72),
-                                   (1000, 1032, 1000), (1600, 1500, 77), (1600, 1500, 1003)])
+                                   (1000, 1032, 1000), (1600, 1500, 77), (1600, 1500, 1003),
+                                   # a last column that cuts an 8-column store, on both tiles
+                                   (1001, 1035, 200), (2500, 4099, 136)])
 def test_gemm_bf16_nt_small_grid_tiles(gpu, oracle, m, n, k):
     _nt_case(gpu, oracle, m, n, k, seed=22, rows=[0, 63, 127, 128, 511, 895, 897, m - 2, m - 1])
 

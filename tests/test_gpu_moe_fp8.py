@@ -518,7 +518,7 @@ def test_gemm_fp8_any_shape(gpu, oracle, m, n, k):
                                    (64, 5000, 4103), (65, 2100, 3072), (130, 1100, 6000),
                                    (1000, 20, 8200), (4100, 16, 2061), (16, 9000, 4096),
                                    (1024, 1024, 128), (1000, 1032, 384), (1024, 1024, 1040),
-                                   (1600, 1500, 77)])
+                                   (1600, 1500, 77), (1001, 1035, 208), (2500, 4099, 144)])
 def test_gemm_fp8_direct_forms_and_small_grids(gpu, oracle, m, n, k):
     """Random codes (no NaN) against the oracle on up to 20000 outputs, and
     with every operand one byte (C two) past its boundary bit for bit the
