@@ -36,6 +36,8 @@
 //    * Both MFMA runs alternate accumulators (S^T: the two key blocks; PV:
 //      the four d blocks), and each LDS operand is read two MFMAs ahead of
 //      its MFMA (+3% over the scheduler's read-just-before-use).
+//    * Calls with few query tiles split the keys over the waves of a
+//      workgroup (flash_fwd_split_kernel).
 //    * Causal: a workgroup runs query tiles r and nq-1-r of one head in
 //      turn, so every workgroup does nq+1 key tiles; a wave skips the
 //      MFMAs of key tiles that lie entirely above its rows and masks the
@@ -72,8 +74,7 @@ constexpr int BKV = 64;        // keys per tile
 constexpr int TILE_BYTES = BKV * D * 2;     // 16 KiB: 64 rows of 256 B
 constexpr int STAGE_BYTES = 2 * TILE_BYTES; // K tile then V tile
 constexpr int SMEM_BYTES = 2 * STAGE_BYTES; // 64 KiB: two stages
-constexpr float RESCALE_SLACK = 8.0f;       // log2 units: p may reach 2^8 before a rescale
-constexpr float kLazyBound = 256.0f;          // 2^RESCALE_SLACK
+constexpr float kLazyBound = 256.0f;        // p may reach 2^8 before a rescale
 
 // Both tiles are [64 keys][128 d] bf16 rows of 256 B holding 16 chunks of
 // 16 B.  K chunk c of row r sits at c ^ (r & 15): the S^T operand reads (32
@@ -166,12 +167,11 @@ FE2O3_DEVICE bf16x8_t read_vt(const uint8_t* vt, uint32_t db, uint32_t kb, uint3
 
 // RAGGED: seq is not a multiple of 64, so the last key tile is partial and
 // its copies mask the rows past seq (copy_load).
-template <bool CAUSAL, bool RAGGED = false>
-__global__ void __launch_bounds__(THREADS, 8 / WAVES) flash_fwd_kernel(
-    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-    const uint16_t* __restrict__ v, uint16_t* __restrict__ o, float* __restrict__ lse,
-    uint32_t seq, uint32_t heads, float scale_log2, uint32_t paired, uint32_t xcds) {
-  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+template <bool CAUSAL, bool RAGGED>
+FE2O3_DEVICE void flash_block(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                              const uint16_t* __restrict__ v, uint16_t* __restrict__ o,
+                              float* __restrict__ lse, uint32_t seq, uint32_t heads,
+                              float scale_log2, uint32_t paired, uint32_t xcds, uint8_t* smem) {
   const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
   const uint32_t lr = lane & 31u, g = lane >> 5;
   // Workgroup order.  Workgroup id i runs on XCD i % xcds (the device's XCD
@@ -400,13 +400,299 @@ __global__ void __launch_bounds__(THREADS, 8 / WAVES) flash_fwd_kernel(
   }  // item
 }
 
+template <bool CAUSAL>
+__global__ void __launch_bounds__(THREADS, 8 / WAVES) flash_fwd_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+    const uint16_t* __restrict__ v, uint16_t* __restrict__ o, float* __restrict__ lse,
+    uint32_t seq, uint32_t heads, float scale_log2, uint32_t paired, uint32_t xcds) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  flash_block<CAUSAL, false>(q, k, v, o, lse, seq, heads, scale_log2, paired, xcds, smem);
+}
+
+__global__ void __launch_bounds__(THREADS, 8 / WAVES) flash_fwd_ragged_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+    const uint16_t* __restrict__ v, uint16_t* __restrict__ o, float* __restrict__ lse,
+    uint32_t seq, uint32_t heads, float scale_log2, uint32_t paired, uint32_t xcds,
+    uint32_t causal) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  if (causal)
+    flash_block<true, true>(q, k, v, o, lse, seq, heads, scale_log2, paired, xcds, smem);
+  else
+    flash_block<false, true>(q, k, v, o, lse, seq, heads, scale_log2, paired, xcds, smem);
+}
+
+// ---- few query tiles: keys split over a workgroup's waves ----------------------------------
+// With fewer 128-row tiles than the device holds workgroups (two per CU), the
+// time is one workgroup's walk over its key tiles, of which a causal head's
+// last rows have the most.  Here a workgroup of four waves takes 64 query
+// rows: SG groups of SQ waves, every group the same rows and every SG-th key
+// tile (32 keys, double-buffered LDS of the group's own), and the groups' sums
+// meet in LDS at the end: each group gathers its share of the head's d, weights
+// the groups by exp2(m_group - m) and stores it.  A walk is half as many steps
+// of half the keys, and twice the workgroups spread over the CUs.
+// Bound by the walk (0.6 us a step with one wave per SIMD, a chain of S^T,
+// softmax and O^T): 32 heads x 1000 causal 28.0 -> 19.0 us, 8 x 500 19.2 ->
+// 9.9.  Four groups in workgroups of eight waves: 25.6 and 9.8 (one per CU
+// then, and the second round pays the start and the merge again).
+constexpr int SQ = 2, SG = 2, SK = 32;
+constexpr int S_ROWS = 32 * SQ, S_THREADS = 64 * SQ * SG;
+constexpr uint32_t S_TILE = SK * D * 2, S_STAGE = 2 * S_TILE, S_GROUP = 2 * S_STAGE;
+constexpr uint32_t S_ACC = SQ * SG * 64u * 64u * 4u;  // the sums, 128 KiB (the tiles' LDS reused)
+constexpr int S_SMEM = (int)(S_ACC + SQ * SG * 64u * 8u);
+static_assert(SG * S_GROUP <= S_ACC, "the sums reuse the tiles' LDS");
+constexpr int S_DB = 4 / SG;  // 32-wide d blocks that a group gathers
+
+template <bool CAUSAL, bool RAGGED>
+FE2O3_DEVICE void flash_split_block(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+                                    const uint16_t* __restrict__ v, uint16_t* __restrict__ o,
+                                    float* __restrict__ lse, uint32_t seq, uint32_t heads,
+                                    float scale_log2, uint32_t xcds, uint32_t cus,
+                                    uint8_t* smem) {
+  const uint32_t lane = threadIdx.x & 63u, lr = lane & 31u, g = lane >> 5;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t group = wave / SQ, wq = wave % SQ;
+  // workgroup order as in flash_block: XCD x walks whole heads, heaviest
+  // causal tile first
+  const uint32_t nq = (seq + S_ROWS - 1u) / S_ROWS;
+  uint32_t bh, rank, first;  // first: the head's first workgroup
+  if (xcds > 1u && heads % xcds == 0u) {
+    const uint32_t xcd = blockIdx.x % xcds, slot = blockIdx.x / xcds;
+    bh = (slot / nq) * xcds + xcd;
+    rank = slot % nq;
+    first = slot / nq * nq * xcds + xcd;
+  } else {
+    bh = blockIdx.x / nq;
+    rank = blockIdx.x % nq;
+    first = bh * nq;
+  }
+  // workgroup i + cus shares a CU with workgroup i: the heads of every second
+  // `cus` workgroups start at the light end, so that a CU's two add up to
+  // about the same work
+  const uint32_t qt = CAUSAL && (first / cus & 1u) == 0u ? nq - 1u - rank : rank;
+  const uint64_t head = (uint64_t)bh * seq * D;
+  const uint32_t head_bytes = seq * (uint32_t)(D * 2);
+  const __amdgpu_buffer_rsrc_t ksrc = head_rsrc(k + head, head_bytes);
+  const __amdgpu_buffer_rsrc_t vsrc = head_rsrc(v + head, head_bytes);
+  const uint32_t q_row0 = qt * S_ROWS + wq * 32u, my_q = q_row0 + lr;
+  const uint32_t q_load = my_q < seq ? my_q : seq - 1u;
+  bf16x8_t qf[8];
+#pragma unroll
+  for (int ds = 0; ds < 8; ++ds)
+    qf[ds] = *reinterpret_cast<const bf16x8_t*>(q + head + (uint64_t)q_load * D + ds * 16 + g * 8);
+
+  // tile copies: 8 loads of 4 rows, the group's wave wq loads rows
+  // 4 (2j + wq) .. +3; the K swizzle depends on the row mod 16, so odd and
+  // even j have an offset each, V's on the row mod 4
+  const uint32_t crow = 4u * wq + (lane >> 4), cpos = lane & 15u;
+  const uint32_t k_off[2] = {crow * 256u + ((cpos ^ swz_k(crow)) << 4),
+                             crow * 256u + ((cpos ^ swz_k(crow + 8u)) << 4)};
+  const uint32_t v_off = crow * 256u + ((cpos ^ swz_v(crow)) << 4);
+  uint8_t* own = smem + group * S_GROUP;
+  // copy n (0 .. 7: K then V) of the tile at byte `tile` into `stage`
+  auto copy = [&](int n, uint32_t tile, uint8_t* stage) {
+    const int j = n & 3;
+    const bool is_v = n >= 4;
+    const uint32_t soff = tile + 2048u * j, voff = is_v ? v_off : k_off[j & 1];
+    const uint32_t off = !RAGGED || voff + soff < head_bytes ? voff : kKeyOutOfRange;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        is_v ? vsrc : ksrc,
+        (lds_void_t*)(stage + (is_v ? S_TILE : 0u) + (2u * j + wq) * 1024u), 16, off, soff, 0, 0);
+  };
+
+  f32x16_t acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
+  float m_ref = -INFINITY, l_run = 0.0f;  // as in flash_block
+
+  const uint32_t kv_tiles = (seq + SK - 1u) / SK;
+  const uint32_t n_kv = CAUSAL ? min((qt + 1u) * (uint32_t)(S_ROWS / SK), kv_tiles) : kv_tiles;
+  const uint32_t turns = (n_kv + SG - 1u) / SG;
+  // the byte offset of the group's tile of turn t; turns it has no tile in
+  // copy the last tile into a buffer that is not read
+  auto tile_of = [&](uint32_t t) {
+    return __builtin_amdgcn_readfirstlane(min(t * SG + group, n_kv - 1u) * S_TILE);
+  };
+#pragma unroll
+  for (int n = 0; n < 8; ++n) copy(n, tile_of(0), own);
+  wait_vmcnt0();
+  lds_barrier();
+  for (uint32_t t = 0; t < turns; ++t) {
+    const uint8_t* cur = own + (t & 1u) * S_STAGE;
+    uint8_t* nxt = own + ((t + 1u) & 1u) * S_STAGE;
+    const uint32_t nt = tile_of(t + 1u), j = t * SG + group, key0 = j * SK;
+    const bool active = j < n_kv && (!CAUSAL || key0 <= q_row0 + 31u);
+    if (!active) {
+#pragma unroll
+      for (int n = 0; n < 8; ++n) copy(n, nt, nxt);
+    } else {
+      auto kread = [&](int i) {
+        return *reinterpret_cast<const bf16x8_t*>(
+            cur + lr * 256u + (((2u * (uint32_t)i + g) ^ swz_k(lr)) << 4));
+      };
+      f32x16_t s;
+      bf16x8_t kf[8];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) kf[i] = kread(i);
+      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, kAhead, 0);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i + kAhead < 8) kf[i + kAhead] = kread(i + kAhead);
+        s = i == 0 ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[0], f32x16_t{}, 0, 0, 0)
+                   : __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i], s, 0, 0, 0);
+        copy(i, nt, nxt);
+        if (i + kAhead < 8) __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(kSchedVmemRead, 1, 0);
+      }
+      if (!CAUSAL && key0 + (uint32_t)SK > seq) {  // keys past seq
+        const int lim = (int)(seq - key0) - 4 * (int)g;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (8 * (e >> 2) + (e & 3) >= lim) s[e] = -INFINITY;
+      }
+      if (CAUSAL && key0 + SK - 1u > q_row0) {  // the diagonal tile
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (key0 + 8u * (e >> 2) + 4u * g + (e & 3) > my_q) s[e] = -INFINITY;
+      }
+      bf16x8_t pf[2];
+      float psum;
+      auto probabilities = [&] {
+        psum = 0.0f;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float pv[8];
+#pragma unroll
+          for (int jj = 0; jj < 8; ++jj) {
+            pv[jj] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[h * 8 + jj], scale_log2, -m_ref));
+            psum += pv[jj];
+          }
+#pragma unroll
+          for (int jj = 0; jj < 8; ++jj) pf[h][jj] = (__bf16)pv[jj];
+        }
+      };
+      probabilities();
+      if (__any(!(psum <= kLazyBound))) {  // raise the reference, as in flash_block
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mloc = fmaxf(mloc, s[e]);
+        mloc = fmaxf(mloc, swap_half(mloc)) * scale_log2;
+        const float m_new = fmaxf(m_ref, mloc);
+        const float alpha = __builtin_amdgcn_exp2f(m_ref - m_new);
+        m_ref = m_new;
+        l_run *= alpha;
+#pragma unroll
+        for (int db = 0; db < 4; ++db)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[db][e] *= alpha;
+        probabilities();
+      }
+      l_run += psum;
+      const uint8_t* vt = cur + S_TILE;
+      __builtin_amdgcn_s_setprio(1);
+      auto vread = [&](int i) { return read_vt(vt, (uint32_t)(i & 3), 0u, (uint32_t)(i >> 2)); };
+      bf16x8_t vf[8];
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) vf[i] = vread(i);
+      __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2 * kAhead, 1);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i + kAhead < 8) vf[i + kAhead] = vread(i + kAhead);
+        acc[i & 3] =
+            __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], pf[i >> 2], acc[i & 3], 0, 0, 0);
+        if (i + kAhead < 8) __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 2, 1);
+        __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 1);
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
+    wait_vmcnt0();
+    lds_barrier();
+  }
+
+  // sums [wave][db][4 of 16][lane] and each lane's reference and row sum
+  f32x4_t* sums = reinterpret_cast<f32x4_t*>(smem);
+  f32x2_t* stats = reinterpret_cast<f32x2_t*>(smem + S_ACC);
+  const float l_own = l_run + swap_half(l_run);
+#pragma unroll
+  for (int db = 0; db < 4; ++db)
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4)
+      sums[((wave * 4u + db) * 4u + e4) * 64u + lane] = f32x4_t{
+          acc[db][4 * e4], acc[db][4 * e4 + 1], acc[db][4 * e4 + 2], acc[db][4 * e4 + 3]};
+  stats[wave * 64u + lane] = f32x2_t{m_ref, l_own};
+  __syncthreads();
+  // a group without an active tile has m = -inf, l = 0: weight 0.  A row's
+  // first key is always some group's, so the largest m is finite.
+  f32x2_t st[SG];
+  float m = -INFINITY, l = 0.0f, weight[SG];
+#pragma unroll
+  for (int x = 0; x < SG; ++x) {
+    st[x] = stats[(x * SQ + wq) * 64u + lane];
+    m = fmaxf(m, st[x][0]);
+  }
+#pragma unroll
+  for (int x = 0; x < SG; ++x) {
+    weight[x] = __builtin_amdgcn_exp2f(st[x][0] - m);
+    l += weight[x] * st[x][1];
+  }
+  const float inv = 1.0f / l;
+  if (my_q >= seq) return;
+  uint16_t* out = o + head + (uint64_t)my_q * D + 4u * g;
+#pragma unroll
+  for (int x4 = 0; x4 < 4 * S_DB; ++x4) {
+    const uint32_t db = group * S_DB + x4 / 4, e4 = x4 % 4;
+    f32x4_t y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < SG; ++x)
+      y += weight[x] * sums[(((x * SQ + wq) * 4u + db) * 4u + e4) * 64u + lane];
+    u32x2_t packed;
+    packed[0] = pack_bf16x2(y[0] * inv, y[1] * inv);
+    packed[1] = pack_bf16x2(y[2] * inv, y[3] * inv);
+    *reinterpret_cast<u32x2_t*>(out + db * 32u + 8u * e4) = packed;
+  }
+  if (lse != nullptr && group == 0 && g == 0)
+    lse[(uint64_t)bh * seq + my_q] = (m + __log2f(l)) * 0.69314718055994531f;
+}
+
+// Whether a call runs on it, from the 64-row query tiles in all.  Non-causal
+// while they fit one per CU; causal, whose tiles are unequal, two per CU, for
+// sequences of several turns (us, 128-row workgroups against this kernel;
+// heads x seq):
+//   non-causal  8 x 500    13.1, 10.1    16 x 1024  19.5, 16.0   32 x 512   12.9, 10.7
+//               32 x 1000  26.0, 26.2    16 x 2048  39.0, 40.2
+//   causal      8 x 500    19.2,  9.9    32 x 1000  28.0, 19.0   16 x 2048  40.2, 30.2
+//               8 x 4096   67.9, 54.2    64 x 300   10.6, 11.0   64 x 1024  29.9, 35.5
+// A single key tile per row is not worth the merge (8 x 64: 5.1, 5.3).
+bool split_keys(uint64_t tiles, uint32_t seq, bool causal, uint32_t cus) {
+  if (tiles <= cus) return seq > 64u;
+  return causal && tiles <= 2ull * cus && seq >= 512u;
+}
+
+__global__ void __launch_bounds__(S_THREADS, 2) flash_fwd_split_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
+    const uint16_t* __restrict__ v, uint16_t* __restrict__ o, float* __restrict__ lse,
+    uint32_t seq, uint32_t heads, float scale_log2, uint32_t xcds, uint32_t cus, uint32_t causal) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  const bool ragged = seq % SK != 0u;
+  if (causal && ragged)
+    flash_split_block<true, true>(q, k, v, o, lse, seq, heads, scale_log2, xcds, cus, smem);
+  else if (causal)
+    flash_split_block<true, false>(q, k, v, o, lse, seq, heads, scale_log2, xcds, cus, smem);
+  else if (ragged)
+    flash_split_block<false, true>(q, k, v, o, lse, seq, heads, scale_log2, xcds, cus, smem);
+  else
+    flash_split_block<false, false>(q, k, v, o, lse, seq, heads, scale_log2, xcds, cus, smem);
+}
+
 // kernels behind each entry point (fe2o3_kernel_resources)
 const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_flash_attention_causal_f32_b1_h1_n8_d16_v1", "flash_profile_kernel", (const void*)flash_profile_kernel, 64, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_flash_attention_fwd", "flash_fwd_kernel<false>", (const void*)flash_fwd_kernel<false>, THREADS, SMEM_BYTES}),
     fe2o3_host::KernelRegistrar({"fe2o3_flash_attention_fwd", "flash_fwd_kernel<true>", (const void*)flash_fwd_kernel<true>, THREADS, SMEM_BYTES}),
-    fe2o3_host::KernelRegistrar({"fe2o3_flash_attention_fwd", "flash_fwd_kernel<false, ragged>", (const void*)flash_fwd_kernel<false, true>, THREADS, SMEM_BYTES}),
-    fe2o3_host::KernelRegistrar({"fe2o3_flash_attention_fwd", "flash_fwd_kernel<true, ragged>", (const void*)flash_fwd_kernel<true, true>, THREADS, SMEM_BYTES})};
+    fe2o3_host::KernelRegistrar({"fe2o3_flash_attention_fwd", "flash_fwd_ragged_kernel", (const void*)flash_fwd_ragged_kernel, THREADS, SMEM_BYTES}),
+    fe2o3_host::KernelRegistrar({"fe2o3_flash_attention_fwd", "flash_fwd_split_kernel", (const void*)flash_fwd_split_kernel, S_THREADS, S_SMEM})};
 
 }  // namespace
 
@@ -447,32 +733,42 @@ int32_t fe2o3_flash_attention_fwd(const uint16_t* q, uint64_t q_len, const uint1
     return FE2O3_ERR_ALIGNMENT;
   if (!(scale > 0.0f) || !__builtin_isfinite(scale)) return FE2O3_ERR_SHAPE;
   const float scale_log2 = scale * 1.4426950408889634f;
-  static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
-      {(const void*)flash_fwd_kernel<true>, (const void*)flash_fwd_kernel<false>,
-       (const void*)flash_fwd_kernel<true, true>, (const void*)flash_fwd_kernel<false, true>},
-      SMEM_BYTES);
+  static const int32_t lds_rc = [] {
+    const int32_t rc = fe2o3_host::set_dynamic_lds(
+        {(const void*)flash_fwd_kernel<true>, (const void*)flash_fwd_kernel<false>,
+         (const void*)flash_fwd_ragged_kernel},
+        SMEM_BYTES);
+    return rc != FE2O3_OK
+               ? rc
+               : fe2o3_host::set_dynamic_lds({(const void*)flash_fwd_split_kernel}, S_SMEM);
+  }();
   if (lds_rc != FE2O3_OK) return lds_rc;
-  // one linear workgroup id per (query tile, batch*head); see the kernel
-  // causal: pairs of query tiles per workgroup (every workgroup the same
-  // work) when the tile count is even; non-causal tiles are equal already
-  const uint32_t nq = (seq + BQ - 1u) / BQ;  // query tiles per head, the last maybe partial
-  const uint32_t paired = causal && nq % 2u == 0u ? 1u : 0u;
-  const uint64_t wgs = (uint64_t)nq / (paired ? 2u : 1u) * bh;
-  if (wgs > 0x7fffffffu) return FE2O3_ERR_SHAPE;
   tile_plan::Topology topo;
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
+  // one linear workgroup id per (query tile, batch*head); see the kernel
+  // causal: pairs of query tiles per workgroup (every workgroup the same
+  // work) when the tile count is even; non-causal tiles are equal already.
+  // Heads of up to four tiles that fit the device at once run unpaired (8 x 32
+  // heads x 256: 20.3 -> 16.2 us; 16 x 4096, more tiles a head: 75 -> 92).
+  const uint32_t nq = (seq + BQ - 1u) / BQ;  // query tiles per head, the last maybe partial
+  const bool at_once = nq <= 4u && nq * bh <= 2ull * topo.cus;
+  const uint32_t paired = causal && nq % 2u == 0u && !at_once ? 1u : 0u;
+  const uint64_t wgs = (uint64_t)nq / (paired ? 2u : 1u) * bh;
+  if (wgs > 0x7fffffffu) return FE2O3_ERR_SHAPE;
   const dim3 grid((unsigned)wgs);
   hipStream_t s = (hipStream_t)stream;
-  const bool ragged = seq % BKV != 0u;  // a partial last key tile
-  if (causal && ragged)
-    flash_fwd_kernel<true, true><<<grid, THREADS, SMEM_BYTES, s>>>(
-        q, k, v, o, lse, seq, (uint32_t)bh, scale_log2, paired, topo.xcds);
+  const uint64_t split_wgs = ((uint64_t)seq + S_ROWS - 1u) / S_ROWS * bh;
+  if (split_keys(split_wgs, seq, causal != 0, topo.cus)) {
+    flash_fwd_split_kernel<<<(unsigned)split_wgs, S_THREADS, S_SMEM, s>>>(
+        q, k, v, o, lse, seq, (uint32_t)bh, scale_log2, topo.xcds, topo.cus, causal != 0);
+    return fe2o3_host::after_launch();
+  }
+  if (seq % BKV != 0u)  // a partial last key tile
+    flash_fwd_ragged_kernel<<<grid, THREADS, SMEM_BYTES, s>>>(
+        q, k, v, o, lse, seq, (uint32_t)bh, scale_log2, paired, topo.xcds, causal != 0);
   else if (causal)
     flash_fwd_kernel<true><<<grid, THREADS, SMEM_BYTES, s>>>(
-        q, k, v, o, lse, seq, (uint32_t)bh, scale_log2, paired, topo.xcds);
-  else if (ragged)
-    flash_fwd_kernel<false, true><<<grid, THREADS, SMEM_BYTES, s>>>(
         q, k, v, o, lse, seq, (uint32_t)bh, scale_log2, paired, topo.xcds);
   else
     flash_fwd_kernel<false><<<grid, THREADS, SMEM_BYTES, s>>>(

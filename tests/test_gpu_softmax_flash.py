@@ -411,3 +411,42 @@ def test_flash_partial_key_tile_ignores_stale_lds(gpu, oracle):
         rc, ref, _ = oracle.flash_attention_rows_bf16(*host, s, 128, causal, 0.125, bh, rows)
         assert rc == 0
         assert rel_err(got, ref) <= 1e-2
+
+
+@pytest.mark.parametrize("causal", [False, True])
+# the kernel that splits the keys over wave groups: one key tile in each group
+# and less, turns that one group sits out, partial key and query tiles, two
+# workgroups per CU in both workgroup orders (36 and 40 heads)
+@pytest.mark.parametrize("b,h,s", [(1, 3, 65), (2, 1, 96), (1, 2, 97), (1, 9, 161), (1, 1, 1111),
+                                   (1, 36, 520), (1, 40, 520)])
+def test_flash_split_keys_all_rows(gpu, oracle, b, h, s, causal):
+    test_flash_any_seq_all_rows(gpu, oracle, b, h, s, causal)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("pattern", ["normal", "ramp", "jump"])
+@pytest.mark.parametrize("s", [37, 64, 200, 256, 300, 512, 640])
+def test_flash_wide_kernels_all_rows(gpu, oracle, pattern, s, causal):
+    """Two heads repeated over 640, more query tiles than the split kernel
+    takes: whole and partial tiles, paired and unpaired, with references that
+    rise at every key tile or jump.  Every repeat bit for bit the first, whose
+    rows and LSE match the f64 oracle."""
+    rep, rng = 320, np.random.default_rng(s)
+    t = {"normal": 0.0, "ramp": np.arange(s) / 64.0,
+         "jump": np.where(np.arange(s) >= s // 2, 14.0, 0.0)}[pattern] * np.ones(s)
+    n = 2 * s
+    q = rng.standard_normal((n, 128)) if pattern == "normal" else \
+        1.0 + 0.05 * rng.standard_normal((n, 128))
+    k = rng.standard_normal((n, 128)) if pattern == "normal" else \
+        np.tile(t, 2)[:, None] + 0.1 * rng.standard_normal((n, 128))
+    v = rng.standard_normal((n, 128))
+    one = [oracle.bf16_from_f32(np.ascontiguousarray(x, np.float32).ravel()) for x in (q, k, v)]
+    _, out, lse, scale = _flash(gpu, 1, 2 * rep, s, causal, seed=0,
+                                qkv=[np.tile(x, rep) for x in one])
+    out, lse = out.reshape(rep, -1), lse.reshape(rep, -1)
+    assert np.all(out == out[0]) and np.all(lse == lse[0])
+    bh, rows = np.repeat(np.arange(2, dtype=np.uint32), s), np.tile(np.arange(s, dtype=np.uint32), 2)
+    rc, ref, ref_lse = oracle.flash_attention_rows_bf16(*one, s, 128, causal, scale, bh, rows)
+    assert rc == 0
+    assert rel_err(out[0].reshape(-1, 128), ref) <= 1e-2
+    assert rel_err(lse[0], ref_lse) <= 1e-5  # fp32 output: the 1e-5 bar
