@@ -6,6 +6,7 @@
 //      id (kernel.rs:25-33); route r = 2*token + rank; gating weights
 //      w0 = 1/(1+exp(l1-l0)), w1 = 1 - w0 (w0 in [0.5,1], so the pair sums to
 //      exactly 1 as examples/moe_expert_v1/src/pipeline.rs:137-148 requires).
+//      Up to 512 routes both steps run in one workgroup (route_small).
 //   2. route_assign: one workgroup per 512 routes; requested = per-expert
 //      totals, admitted = min(requested, capacity), offsets = exclusive scan
 //      of admitted with the terminal total; each route gets rank = number of
@@ -54,48 +55,66 @@ FE2O3_DEVICE float logit_at<uint16_t>(const uint16_t* p, uint64_t i) {
   return f32_from_bf16_bits(p[i]);
 }
 
-// A token with a NaN or infinite logit is written as top2 = (DROP, DROP)
-// and marks the contract-status word; route_assign then rejects the whole
-// launch (see there), as the reference's kernel traps on any non-finite
-// logit (kernel.rs:118-128).
+// The two best experts of one token and their gating weights, in one pass
+// over its logits, loaded eight at a time (one memory wait per eight).  A
+// token with a NaN or infinite logit is written as top2 = (DROP, DROP) and
+// marks the contract-status word; the assignment then rejects the whole
+// launch (see there), as the reference's kernel traps on any non-finite logit
+// (kernel.rs:118-128).
+template <typename T>
+FE2O3_DEVICE void select_token(const T* __restrict__ row, uint32_t experts,
+                               uint32_t* __restrict__ top2, float* __restrict__ weights,
+                               uint32_t* __restrict__ status, uint32_t* best_out,
+                               uint32_t* second_out) {
+#pragma clang fp contract(off)
+  uint32_t best = DROP, second = DROP;
+  float bs = 0.0f, ss = 0.0f, probe = 0.0f;
+  for (uint32_t e0 = 0; e0 < experts; e0 += 8u) {
+    float v[8];
+#pragma unroll
+    for (uint32_t q = 0; q < 8; ++q) v[q] = logit_at(row, min(e0 + q, experts - 1u));
+#pragma unroll
+    for (uint32_t q = 0; q < 8; ++q) {
+      const uint32_t e = e0 + q;
+      if (e >= experts) break;
+      const float s = v[q];
+      probe = finite_probe(probe, s);
+      if (best == DROP || s > bs || (s == bs && e < best)) {
+        second = best;
+        ss = bs;
+        best = e;
+        bs = s;
+      } else if (second == DROP || s > ss || (s == ss && e < second)) {
+        second = e;
+        ss = s;
+      }
+    }
+  }
+  if (probe != probe) {
+    mark_nonfinite(status);
+    best = second = DROP;
+  } else if (weights != nullptr) {
+    const float w0 = 1.0f / (1.0f + expf(ss - bs));
+    weights[0] = w0;
+    weights[1] = 1.0f - w0;
+  }
+  top2[0] = best;
+  top2[1] = second;
+  *best_out = best;
+  *second_out = second;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) route_select_kernel(const T* __restrict__ logits,
                                                            uint32_t tokens, uint32_t experts,
                                                            uint32_t* __restrict__ top2,
                                                            float* __restrict__ weights,
                                                            uint32_t* __restrict__ status) {
-#pragma clang fp contract(off)
   const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= tokens) return;
-  const T* row = logits + (uint64_t)t * experts;
-  uint32_t best = DROP, second = DROP;
-  float bs = 0.0f, ss = 0.0f, probe = 0.0f;
-  for (uint32_t e = 0; e < experts; ++e) probe = finite_probe(probe, logit_at(row, e));
-  if (probe != probe) {
-    mark_nonfinite(status);
-    top2[2ull * t] = DROP;
-    top2[2ull * t + 1] = DROP;
-    return;
-  }
-  for (uint32_t e = 0; e < experts; ++e) {
-    const float s = logit_at(row, e);
-    if (best == DROP || s > bs || (s == bs && e < best)) {
-      second = best;
-      ss = bs;
-      best = e;
-      bs = s;
-    } else if (second == DROP || s > ss || (s == ss && e < second)) {
-      second = e;
-      ss = s;
-    }
-  }
-  top2[2ull * t] = best;
-  top2[2ull * t + 1] = second;
-  if (weights != nullptr) {
-    const float w0 = 1.0f / (1.0f + expf(ss - bs));
-    weights[2ull * t] = w0;
-    weights[2ull * t + 1] = 1.0f - w0;
-  }
+  uint32_t best, second;
+  select_token(logits + (uint64_t)t * experts, experts, top2 + 2ull * t,
+               weights ? weights + 2ull * t : nullptr, status, &best, &second);
 }
 
 // Slot assignment, one workgroup per RA_ROUTES consecutive routes (one route
@@ -132,113 +151,166 @@ FE2O3_DEVICE void for_each_expert(uint32_t e, Fn&& fn) {
   }
 }
 
-// PREFIXED: the per-expert counts before this workgroup and the totals come
-// from route_scan_kernel (prefix: (experts + 1) words per workgroup, the
-// last unused here; totals: experts words, then the number of workgroups
-// that saw a rejected entry) instead of from counting all of top2 here.
-template <bool PREFIXED>
-__global__ void __launch_bounds__(RA_THREADS) route_assign_kernel(
-    uint32_t* __restrict__ top2, uint32_t routes, uint32_t experts, uint32_t capacity,
-    uint32_t* __restrict__ requested, uint32_t* __restrict__ admitted,
-    uint32_t* __restrict__ offsets, uint32_t* __restrict__ slots,
-    uint32_t* __restrict__ permutation, uint32_t* __restrict__ inverse,
-    float* __restrict__ weights, const uint32_t* __restrict__ prefix,
-    const uint32_t* __restrict__ totals) {
-  __shared__ uint32_t total[MAX_EXPERTS], before[MAX_EXPERTS], off_s[MAX_EXPERTS + 1];
-  __shared__ uint32_t wave_cnt[RA_WAVES][MAX_EXPERTS];
+struct RouteOut {
+  uint32_t *top2, *requested, *admitted, *offsets, *slots, *permutation, *inverse;
+  float* weights;
+};
+
+struct AssignLds {
+  uint32_t total[MAX_EXPERTS], before[MAX_EXPERTS], off_s[MAX_EXPERTS + 1];
+  uint32_t wave_cnt[RA_WAVES][MAX_EXPERTS];
+};
+
+// The outputs of this workgroup's routes (thread t: route r = start + t of
+// expert e, DROP for none), once lds.total and lds.before hold the counts.
+// first: the workgroup that writes the per-expert outputs.
+FE2O3_DEVICE void assign_routes(uint32_t e, uint32_t r, uint32_t routes, uint32_t experts,
+                                uint32_t capacity, bool rejected, bool first, const RouteOut& out,
+                                AssignLds& lds) {
   const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
-  const uint32_t start = blockIdx.x * (uint32_t)RA_ROUTES;
   const uint64_t lt = (1ull << lane) - 1ull;
-  if constexpr (PREFIXED) {
-    if (t < experts) {
-      total[t] = totals[t];
-      before[t] = prefix[(uint64_t)blockIdx.x * (experts + 1u) + t];
-    }
-  } else {
-    if (t < experts) total[t] = before[t] = 0;
-  }
-  for (uint32_t i = t; i < RA_WAVES * MAX_EXPERTS; i += RA_THREADS) (&wave_cnt[0][0])[i] = 0;
-  __syncthreads();
-  // counts over all of top2, 64 routes per wave and chunk; the loads of
-  // eight chunks are issued together, then counted
-  constexpr int kBatch = 8;
-  int rejected = PREFIXED && totals[experts] != 0u;
-  for (uint32_t base0 = wave * 64u; !PREFIXED && base0 < routes;
-       base0 += kBatch * RA_THREADS) {
-    uint32_t ev[kBatch];
-#pragma unroll
-    for (int q = 0; q < kBatch; ++q) {
-      const uint32_t r = base0 + q * RA_THREADS + lane;
-      ev[q] = r < routes ? top2[r] : DROP;
-      rejected |= r < routes && ev[q] >= experts;
-      if (ev[q] >= experts) ev[q] = DROP;  // not an expert: counted nowhere
-    }
-#pragma unroll
-    for (int q = 0; q < kBatch; ++q) {
-      const uint32_t base = base0 + q * RA_THREADS;
-      for_each_expert(ev[q], [&](uint32_t x, uint64_t mask) {
-        if (lane == 0) {
-          const uint32_t c = (uint32_t)__builtin_popcountll(mask);
-          atomicAdd(&total[x], c);
-          if (base < start) atomicAdd(&before[x], c);
-        }
-      });
-    }
-  }
-  const uint32_t r = start + t;
   if (__syncthreads_or(rejected)) {
     if (r < routes) {
-      top2[r] = DROP;
-      slots[r] = DROP;
-      inverse[r] = DROP;
-      permutation[r] = DROP;
-      if (weights != nullptr) weights[r] = 0.0f;
+      out.top2[r] = DROP;
+      out.slots[r] = DROP;
+      out.inverse[r] = DROP;
+      out.permutation[r] = DROP;
+      if (out.weights != nullptr) out.weights[r] = 0.0f;
     }
-    if (blockIdx.x == 0) {
-      if (t < experts) requested[t] = admitted[t] = offsets[t] = 0;
-      if (t == 0) offsets[experts] = 0;
+    if (first) {
+      if (t < experts) out.requested[t] = out.admitted[t] = out.offsets[t] = 0;
+      if (t == 0) out.offsets[experts] = 0;
     }
     return;
   }
   if (t == 0) {  // admitted counts and their exclusive scan (at most 64 experts)
     uint32_t run = 0;
     for (uint32_t x = 0; x < experts; ++x) {
-      off_s[x] = run;
-      run += total[x] < capacity ? total[x] : capacity;
+      lds.off_s[x] = run;
+      run += lds.total[x] < capacity ? lds.total[x] : capacity;
     }
-    off_s[experts] = run;
+    lds.off_s[experts] = run;
   }
   // ranks within this wave, and this wave's count per expert
-  const uint32_t e = r < routes ? top2[r] : DROP;
   uint32_t rank = 0;
   for_each_expert(e, [&](uint32_t x, uint64_t mask) {
     if (e == x) rank = (uint32_t)__builtin_popcountll(mask & lt);
-    if (lane == 0) wave_cnt[wave][x] = (uint32_t)__builtin_popcountll(mask);
+    if (lane == 0) lds.wave_cnt[wave][x] = (uint32_t)__builtin_popcountll(mask);
   });
   __syncthreads();
-  if (blockIdx.x == 0) {
+  if (first) {
     if (t < experts) {
-      requested[t] = total[t];
-      admitted[t] = total[t] < capacity ? total[t] : capacity;
-      offsets[t] = off_s[t];
+      out.requested[t] = lds.total[t];
+      out.admitted[t] = lds.total[t] < capacity ? lds.total[t] : capacity;
+      out.offsets[t] = lds.off_s[t];
     }
-    if (t == 0) offsets[experts] = off_s[experts];
+    if (t == 0) out.offsets[experts] = lds.off_s[experts];
   }
   if (r >= routes) return;
-  rank += before[e];
-  for (uint32_t w = 0; w < wave; ++w) rank += wave_cnt[w][e];
+  rank += lds.before[e];
+  for (uint32_t w = 0; w < wave; ++w) rank += lds.wave_cnt[w][e];
   if (rank < capacity) {
-    const uint32_t slot = off_s[e] + rank;
-    slots[r] = slot;
-    inverse[r] = slot;
-    permutation[slot] = r;
+    const uint32_t slot = lds.off_s[e] + rank;
+    out.slots[r] = slot;
+    out.inverse[r] = slot;
+    out.permutation[slot] = r;
   } else {
-    slots[r] = DROP;
-    inverse[r] = DROP;
+    out.slots[r] = DROP;
+    out.inverse[r] = DROP;
   }
   // slots below the accepted total are each written by their route; the rest
   // of the permutation holds the sentinel
-  if (r >= off_s[experts]) permutation[r] = DROP;
+  if (r >= lds.off_s[experts]) out.permutation[r] = DROP;
+}
+
+// PREFIXED: the per-expert counts before this workgroup and the totals come
+// from route_scan_kernel (prefix: (experts + 1) words per workgroup, the
+// last unused here; totals: experts words, then the number of workgroups
+// that saw a rejected entry) instead of from counting all of top2 here.
+// Counting: lane x of a wave keeps expert x's count, one ballot and one
+// conditional add per expert and 64 routes; a list of the experts present in
+// each 64, counted by LDS atomics, took 24.8 us at 4096 tokens of 8 experts
+// where this takes 12.3 (28.6 and 13.6 at 2753 tokens of 16).
+template <bool PREFIXED>
+__global__ void __launch_bounds__(RA_THREADS) route_assign_kernel(
+    RouteOut out, uint32_t routes, uint32_t experts, uint32_t capacity,
+    const uint32_t* __restrict__ prefix, const uint32_t* __restrict__ totals) {
+  __shared__ AssignLds lds;
+  const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+  const uint32_t start = blockIdx.x * (uint32_t)RA_ROUTES;
+  if constexpr (PREFIXED) {
+    if (t < experts) {
+      lds.total[t] = totals[t];
+      lds.before[t] = prefix[(uint64_t)blockIdx.x * (experts + 1u) + t];
+    }
+  } else {
+    if (t < experts) lds.total[t] = lds.before[t] = 0;
+  }
+  for (uint32_t i = t; i < RA_WAVES * MAX_EXPERTS; i += RA_THREADS) (&lds.wave_cnt[0][0])[i] = 0;
+  __syncthreads();
+  // counts over all of top2, 64 routes per wave and chunk; the loads of
+  // eight chunks are issued together, then counted
+  constexpr int kBatch = 8;
+  int rejected = PREFIXED && totals[experts] != 0u;
+  uint32_t all = 0, earlier = 0;  // of expert `lane`
+  for (uint32_t base0 = wave * 64u; !PREFIXED && base0 < routes;
+       base0 += kBatch * RA_THREADS) {
+    uint32_t ev[kBatch];
+#pragma unroll
+    for (int q = 0; q < kBatch; ++q) {
+      const uint32_t r = base0 + q * RA_THREADS + lane;
+      ev[q] = r < routes ? out.top2[r] : DROP;
+      rejected |= r < routes && ev[q] >= experts;
+    }
+#pragma unroll
+    for (int q = 0; q < kBatch; ++q) {
+      const uint32_t base = base0 + q * RA_THREADS;
+      if (base >= routes) break;
+      uint32_t here = 0;
+      for (uint32_t x0 = 0; x0 < experts; x0 += 4u) {  // no entry names an expert past the last
+        uint32_t c[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+          c[i] = (uint32_t)__builtin_popcountll(__ballot(ev[q] == x0 + i));
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) here = lane == x0 + i ? c[i] : here;
+      }
+      all += here;
+      if (base < start) earlier += here;
+    }
+  }
+  if (!PREFIXED && lane < experts) {
+    if (all) atomicAdd(&lds.total[lane], all);
+    if (earlier) atomicAdd(&lds.before[lane], earlier);
+  }
+  const uint32_t r = start + t;
+  const uint32_t e = r < routes ? out.top2[r] : DROP;
+  assign_routes(e, r, routes, experts, capacity, rejected, blockIdx.x == 0, out, lds);
+}
+
+// Router of at most RA_ROUTES routes: selection and assignment in one
+// workgroup and one launch (a decoding step's 32 tokens: two launches of 4.8
+// and 4.0 us, against one of 4.9).
+template <typename T>
+__global__ void __launch_bounds__(RA_THREADS) route_small_kernel(
+    const T* __restrict__ logits, RouteOut out, uint32_t tokens, uint32_t experts,
+    uint32_t capacity, uint32_t* __restrict__ status) {
+  __shared__ AssignLds lds;
+  __shared__ uint32_t chosen[RA_ROUTES];
+  const uint32_t t = threadIdx.x, lane = t & 63u, routes = 2u * tokens;
+  if (t < experts) lds.total[t] = lds.before[t] = 0;
+  for (uint32_t i = t; i < RA_WAVES * MAX_EXPERTS; i += RA_THREADS) (&lds.wave_cnt[0][0])[i] = 0;
+  if (t < tokens)
+    select_token(logits + (uint64_t)t * experts, experts, out.top2 + 2u * t,
+                 out.weights ? out.weights + 2u * t : nullptr, status, &chosen[2u * t],
+                 &chosen[2u * t + 1u]);
+  __syncthreads();
+  const uint32_t e = t < routes ? chosen[t] : DROP;
+  for_each_expert(e, [&](uint32_t x, uint64_t mask) {
+    if (lane == 0) atomicAdd(&lds.total[x], (uint32_t)__builtin_popcountll(mask));
+  });
+  // a rejected token's entries are DROP
+  assign_routes(e, t, routes, experts, capacity, t < routes && e == DROP, true, out, lds);
 }
 
 // Slot assignment for many routes, in three kernels whose work is linear in
@@ -722,7 +794,17 @@ int32_t route(const void* logits, uint64_t logits_len, uint32_t dtype, uint32_t*
   hipStream_t s = (hipStream_t)stream;
   uint32_t* status = fe2o3_host::status_word();
   if (status == nullptr) return (int32_t)hipErrorInvalidSymbol;
-  if (tokens) {
+  const RouteOut out = {top2, requested, admitted, offsets, slots, permutation, inverse, weights};
+  if (routes <= RA_ROUTES) {
+    if (dtype == 0)
+      route_small_kernel<float><<<1, RA_THREADS, 0, s>>>((const float*)logits, out, tokens,
+                                                         experts, capacity, status);
+    else
+      route_small_kernel<uint16_t><<<1, RA_THREADS, 0, s>>>((const uint16_t*)logits, out, tokens,
+                                                            experts, capacity, status);
+    return fe2o3_host::after_launch();
+  }
+  {
     const unsigned blocks = (tokens + 255u) / 256u;
     if (dtype == 0)
       route_select_kernel<float><<<blocks, 256, 0, s>>>((const float*)logits, tokens, experts,
@@ -745,17 +827,15 @@ int32_t route(const void* logits, uint64_t logits_len, uint32_t dtype, uint32_t*
                                                                counts);
       route_scan_kernel<<<1, RS_THREADS, 0, s>>>(counts, assign_blocks, experts, totals);
       route_assign_kernel<true><<<assign_blocks, RA_THREADS, 0, s>>>(
-          top2, (uint32_t)routes, experts, capacity, requested, admitted, offsets, slots,
-          permutation, inverse, weights, counts, totals);
+          out, (uint32_t)routes, experts, capacity, counts, totals);
       const int32_t rc = fe2o3_host::after_launch();
       const int32_t free_rc = fe2o3_host::scratch_free(scratch, s);
       return rc != FE2O3_OK ? rc : free_rc;
     }
     (void)hipGetLastError();
   }
-  route_assign_kernel<false><<<assign_blocks, RA_THREADS, 0, s>>>(
-      top2, (uint32_t)routes, experts, capacity, requested, admitted, offsets, slots, permutation,
-      inverse, weights, nullptr, nullptr);
+  route_assign_kernel<false><<<assign_blocks, RA_THREADS, 0, s>>>(out, (uint32_t)routes, experts,
+                                                                  capacity, nullptr, nullptr);
   return fe2o3_host::after_launch();
 }
 
@@ -1086,8 +1166,9 @@ __global__ void __launch_bounds__(RS_THREADS) check_reduce_kernel(
 
 // kernels behind each entry point (fe2o3_kernel_resources)
 const fe2o3_host::KernelRegistrar kRegistered[] = {
-    fe2o3_host::KernelRegistrar({"fe2o3_moe_top2_route_f32_t8_e4_k2_c4_v1", "route_select_kernel<float>", (const void*)route_select_kernel<float>, 256, 0}),
-    fe2o3_host::KernelRegistrar({"fe2o3_moe_top2_route_f32_t8_e4_k2_c4_v1", "route_assign_kernel", (const void*)route_assign_kernel<false>, RA_THREADS, 0}),
+    fe2o3_host::KernelRegistrar({"fe2o3_moe_top2_route_f32_t8_e4_k2_c4_v1", "route_small_kernel<float>", (const void*)route_small_kernel<float>, RA_THREADS, 0}),
+    fe2o3_host::KernelRegistrar({"fe2o3_moe_top2_route", "route_small_kernel<float>", (const void*)route_small_kernel<float>, RA_THREADS, 0}),
+    fe2o3_host::KernelRegistrar({"fe2o3_moe_top2_route", "route_small_kernel<uint16_t>", (const void*)route_small_kernel<uint16_t>, RA_THREADS, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_moe_top2_route", "route_select_kernel<float>", (const void*)route_select_kernel<float>, 256, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_moe_top2_route", "route_select_kernel<uint16_t>", (const void*)route_select_kernel<uint16_t>, 256, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_moe_top2_route", "route_assign_kernel", (const void*)route_assign_kernel<false>, RA_THREADS, 0}),
@@ -1112,34 +1193,6 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_moe_routing_check", "route_scan_kernel", (const void*)route_scan_kernel, RS_THREADS, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_moe_routing_check", "check_verify_kernel", (const void*)check_verify_kernel, RA_THREADS, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_moe_routing_check", "check_reduce_kernel", (const void*)check_reduce_kernel, RS_THREADS, 0})};
-
-// The expert FFN's second stream, one per device, created on first use and
-// kept for the life of the process (default priority, non-blocking so that it
-// also runs beside a caller's null stream).
-struct SideStream {
-  std::mutex mu;
-  hipStream_t stream = nullptr;
-  hipEvent_t ready = nullptr, done = nullptr;
-  bool ok = false;
-};
-
-SideStream* side_stream() {
-  static constexpr int kMaxDevices = 64;
-  static SideStream sides[kMaxDevices];
-  static std::mutex create_mu;
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
-  SideStream& sd = sides[dev];
-  std::lock_guard<std::mutex> lock(create_mu);
-  if (!sd.ok) {
-    if (hipStreamCreateWithFlags(&sd.stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&sd.ready, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&sd.done, hipEventDisableTiming) != hipSuccess)
-      return nullptr;
-    sd.ok = true;
-  }
-  return &sd;
-}
 
 }  // namespace
 
@@ -1218,10 +1271,13 @@ uint32_t down_k_parts(uint64_t routes, uint32_t experts, uint32_t hidden, uint32
   return 2u * rounds1 <= rounds2 ? 1u : 2u;
 }
 
-// The expert FFN behind both C-ABI entry points.  `split_streams` runs the
-// second half of the experts on the per-device side stream (created on
-// first use); without it every kernel runs on the caller's stream and the
-// call creates nothing.
+// The expert FFN behind both C-ABI entry points: every kernel on the caller's
+// stream, all experts in each launch.  (Two halves of the experts on two
+// streams, each half's partly filled last round filled by the other's tiles,
+// cost more in the events that join them -- the combine started 10 us after
+// the last down tile -- than the rounds gave: 8 experts, hidden 4096, ffn
+// 14336, 535 us against 511 at 32 tokens, 692 against 665 at 512, 1195 against
+// 1172 at 2048, 2168 against 2157 at 4096.)
 int32_t ffn_top2(const uint16_t* x, uint64_t x_len, const uint16_t* w_gate, uint64_t w_gate_len,
                  const uint16_t* w_up, uint64_t w_up_len, const uint16_t* w_down,
                  uint64_t w_down_len, uint64_t top2_len, const uint32_t* expert_offsets,
@@ -1229,7 +1285,7 @@ int32_t ffn_top2(const uint16_t* x, uint64_t x_len, const uint16_t* w_gate, uint
                  const uint32_t* inverse, uint64_t inverse_len, const float* route_weights,
                  uint64_t weights_len, uint16_t* out, uint64_t out_len, void* workspace,
                  uint64_t workspace_bytes, uint32_t tokens, uint32_t hidden, uint32_t ffn,
-                 uint32_t experts, bool split_streams, void* stream) {
+                 uint32_t experts, void* stream) {
   if (experts < 1 || experts > MAX_EXPERTS) return FE2O3_ERR_SHAPE;
   // hidden: 256-column output blocks of the down GEMM; ffn: 128-wide gate/up
   // blocks, and each k-half of the down GEMM a whole number of 64-k stages
@@ -1261,60 +1317,34 @@ int32_t ffn_top2(const uint16_t* x, uint64_t x_len, const uint16_t* w_gate, uint
       kSmem);
   if (lds_rc != FE2O3_OK) return lds_rc;
   hipStream_t s = (hipStream_t)stream;
-  // the most m-tiles any routing yields for experts [b, e): routes/288
-  // rounded up, plus one partial tile per expert
+  // grids for the most m-tiles any routing yields: routes/288 rounded up,
+  // plus one partial tile per expert
   tile_plan::Topology topo;
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
   const uint32_t xcds = topo.xcds;
   const uint32_t kparts = down_k_parts(routes, experts, hidden, topo.cus);
-  auto grids = [&](uint32_t n_experts, uint64_t* gu, uint64_t* dn) {
-    *gu = expert_grid(routes, n_experts, ffn / 128u, xcds);
-    *dn = expert_grid(routes, n_experts, kparts * (hidden / 256u), xcds);
-    return *gu <= 0x7fffffffu && *dn <= 0x7fffffffu;
-  };
+  const uint64_t gu = expert_grid(routes, experts, ffn / 128u, xcds);
+  const uint64_t dn = expert_grid(routes, experts, kparts * (hidden / 256u), xcds);
+  if (gu > 0x7fffffffu || dn > 0x7fffffffu) return FE2O3_ERR_SHAPE;
   // The gate/up tiles read the token rows in place, through the permutation,
   // when x fits the 32-bit range of a buffer resource; otherwise from rows
   // gathered into the workspace first.
   const uint64_t x_bytes = (uint64_t)tokens * hidden * 2u;
   const bool tokens_direct = x_bytes < (1ull << 31);
-  auto experts_ffn = [&](uint32_t b, uint32_t e, hipStream_t st) {
-    uint64_t gu, dn;
-    grids(e - b, &gu, &dn);
-    if (tokens_direct)
-      gate_up_kernel<true><<<(unsigned)gu, 256, kSmem, st>>>(
-          x, (uint32_t)x_bytes, permutation, w_gate, w_up, expert_offsets, b, e, hidden, ffn,
-          (uint32_t)routes, ws.hc, xcds);
-    else
-      gate_up_kernel<false><<<(unsigned)gu, 256, kSmem, st>>>(
-          ws.xc, 0u, permutation, w_gate, w_up, expert_offsets, b, e, hidden, ffn,
-          (uint32_t)routes, ws.hc, xcds);
-    down_kernel<<<(unsigned)dn, 256, kSmem, st>>>(ws.hc, w_down, expert_offsets, b, e, hidden,
-                                                  ffn, routes, kparts, ws.yc, xcds);
-  };
-  uint64_t gu_all, dn_all;
-  if (!grids(experts, &gu_all, &dn_all)) return FE2O3_ERR_SHAPE;
   if (!tokens_direct)
     gather_kernel<<<(unsigned)routes, 256, 0, s>>>(x, permutation, expert_offsets, experts, hidden,
                                                   (uint32_t)routes, ws.xc);
-  // Two halves of the experts, each gate/up then down, on the caller's
-  // stream and on a side stream: each grouped GEMM ends in a partly filled
-  // round of tiles, which the other half's tiles fill.
-  SideStream* side = split_streams && experts >= 2 ? side_stream() : nullptr;
-  if (side != nullptr) {
-    std::lock_guard<std::mutex> lock(side->mu);  // keeps one call's event waits its own
-    const uint32_t half = experts / 2u;
-    hipError_t e = hipEventRecord(side->ready, s);
-    if (e == hipSuccess) e = hipStreamWaitEvent(side->stream, side->ready, 0);
-    if (e != hipSuccess) return (int32_t)e;
-    experts_ffn(0u, half, s);
-    experts_ffn(half, experts, side->stream);
-    e = hipEventRecord(side->done, side->stream);
-    if (e == hipSuccess) e = hipStreamWaitEvent(s, side->done, 0);
-    if (e != hipSuccess) return (int32_t)e;
-  } else {
-    experts_ffn(0u, experts, s);
-  }
+  if (tokens_direct)
+    gate_up_kernel<true><<<(unsigned)gu, 256, kSmem, s>>>(
+        x, (uint32_t)x_bytes, permutation, w_gate, w_up, expert_offsets, 0u, experts, hidden, ffn,
+        (uint32_t)routes, ws.hc, xcds);
+  else
+    gate_up_kernel<false><<<(unsigned)gu, 256, kSmem, s>>>(
+        ws.xc, 0u, permutation, w_gate, w_up, expert_offsets, 0u, experts, hidden, ffn,
+        (uint32_t)routes, ws.hc, xcds);
+  down_kernel<<<(unsigned)dn, 256, kSmem, s>>>(ws.hc, w_down, expert_offsets, 0u, experts, hidden,
+                                              ffn, routes, kparts, ws.yc, xcds);
   const uint64_t threads = (uint64_t)tokens * (hidden / 4u);
   combine_kernel<<<(unsigned)((threads + 255u) / 256u), 256, 0, s>>>(ws.yc, inverse, route_weights,
                                                                     tokens, hidden, routes, kparts,
@@ -1364,7 +1394,7 @@ int32_t fe2o3_moe_ffn_top2(const uint16_t* x, uint64_t x_len, const uint16_t* w_
   return ffn_top2(x, x_len, w_gate, w_gate_len, w_up, w_up_len, w_down, w_down_len, top2_len,
                   expert_offsets, offsets_len, permutation, permutation_len, inverse, inverse_len,
                   route_weights, weights_len, out, out_len, workspace, workspace_bytes, tokens,
-                  hidden, ffn, experts, true, stream);
+                  hidden, ffn, experts, stream);
 }
 
 int32_t fe2o3_moe_ffn_top2_noalloc(const uint16_t* x, uint64_t x_len, const uint16_t* w_gate,
@@ -1387,7 +1417,7 @@ int32_t fe2o3_moe_ffn_top2_noalloc(const uint16_t* x, uint64_t x_len, const uint
   return ffn_top2(x, x_len, w_gate, w_gate_len, w_up, w_up_len, w_down, w_down_len, top2_len,
                   expert_offsets, offsets_len, permutation, permutation_len, inverse, inverse_len,
                   route_weights, weights_len, out, out_len, ws, kNoAllocScratchBytes, tokens,
-                  hidden, ffn, experts, false, stream);
+                  hidden, ffn, experts, stream);
 }
 
 int32_t fe2o3_moe_routing_check(const uint32_t* top2_experts, uint64_t top2_len,
