@@ -20,6 +20,7 @@
 #include "gemm_pipe.hpp"
 #include "internal.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -28,44 +29,59 @@ using namespace fe2o3;
 
 __global__ void zero_f32_kernel(float* p) { *p = 0.0f; }
 
-// A workgroup step covers 4096 elements as 1024 units of four (unit 256w + t
-// for thread t, w = 0..3): four 16-byte loads in flight per thread, each wave
-// access 1 KiB contiguous.  The rest
-// (fewer than 4096 elements) runs one unit, then one element, per thread.
+// A workgroup step of the quantization covers 4096 elements as 1024 units of
+// four (unit 256w + t for thread t, w = 0..3): four 16-byte loads in flight
+// per thread, each wave access 1 KiB contiguous.  The rest (fewer than 4096
+// elements) runs one unit, then one element, per thread.
 constexpr uint64_t kStepUnits = 1024;
 
-__global__ void __launch_bounds__(256) amax_kernel(const float* __restrict__ x, uint64_t n,
-                                                   float* __restrict__ amax) {
+// amax: workgroups of 16 waves, one per CU, and an atomic only from a
+// workgroup whose maximum is above what the result holds by then.  Atomics on
+// one address serialize (about 10 ns each): with one from each of 1024
+// workgroups of four waves, amax, scale and quantization of 2^22 elements took
+// 23.3 us for 17.4, of 2^24 42.9 for 35.9.
+constexpr int kAmaxThreads = 1024;
+constexpr uint64_t kAmaxStepUnits = 4ull * kAmaxThreads;
+
+__global__ void __launch_bounds__(kAmaxThreads) amax_kernel(const float* __restrict__ x,
+                                                            uint64_t n,
+                                                            float* __restrict__ amax) {
   float m = 0.0f;
   const uint64_t t = threadIdx.x;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  const uint64_t units = n / 4, steps = units / kStepUnits;
+  // whole steps only where every workgroup has one; else a unit per thread
+  const uint64_t units = n / 4, whole = units / kAmaxStepUnits;
+  const uint64_t steps = whole >= gridDim.x ? whole : 0;
   const f32x4_t* x4 = reinterpret_cast<const f32x4_t*>(x);
   auto max4 = [](f32x4_t v) {
     return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
   };
   for (uint64_t st = blockIdx.x; st < steps; st += gridDim.x) {
-    const uint64_t u0 = st * kStepUnits + t;
+    const uint64_t u0 = st * kAmaxStepUnits + t;
     f32x4_t v[4];
 #pragma unroll
-    for (int w = 0; w < 4; ++w) v[w] = __builtin_nontemporal_load(x4 + u0 + 256 * w);
+    for (int w = 0; w < 4; ++w) v[w] = __builtin_nontemporal_load(x4 + u0 + kAmaxThreads * w);
 #pragma unroll
     for (int w = 0; w < 4; ++w) m = fmaxf(m, max4(v[w]));
   }
-  for (uint64_t u = steps * kStepUnits + blockIdx.x * blockDim.x + t; u < units; u += stride)
+  for (uint64_t u = steps * kAmaxStepUnits + blockIdx.x * blockDim.x + t; u < units; u += stride)
     m = fmaxf(m, max4(x4[u]));
   for (uint64_t i = units * 4 + blockIdx.x * blockDim.x + t; i < n; i += stride)
     m = fmaxf(m, fabsf(x[i]));
-  // One device-scope atomic per workgroup: atomics on one address from every
-  // wave serialize and cost more than the read of the tensor.
-  __shared__ float wave_m[4];
+  __shared__ float wave_m[kAmaxThreads / 64];
   m = wave_max(m);
   if ((threadIdx.x & 63u) == 0) wave_m[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
-    m = fmaxf(fmaxf(wave_m[0], wave_m[1]), fmaxf(wave_m[2], wave_m[3]));
-    // |x| >= 0, so the IEEE bit patterns order like unsigned integers
-    atomicMax(reinterpret_cast<unsigned int*>(amax), __float_as_uint(m));
+#pragma unroll
+    for (int w = 1; w < kAmaxThreads / 64; ++w) m = fmaxf(m, wave_m[w]);
+    // |x| >= 0, so the IEEE bit patterns order like unsigned integers; the
+    // result only grows, so a stale value read here costs an atomic, never one
+    // that was due
+    unsigned int* out = reinterpret_cast<unsigned int*>(amax);
+    const unsigned int bits = __float_as_uint(m);
+    if (bits > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(out, bits);
   }
 }
 
@@ -74,7 +90,7 @@ __global__ void scale_kernel(const float* amax, float* scale) {
   *scale = a / 448.0f;
 }
 
-// Same step layout as amax_kernel: four units (16 elements) in flight per
+// Four units (16 elements) in flight per
 // thread, 16-byte loads and 4-byte stores of codes, each wave access
 // contiguous.
 __global__ void __launch_bounds__(256) quantize_kernel(const float* __restrict__ x, uint64_t n,
@@ -83,7 +99,9 @@ __global__ void __launch_bounds__(256) quantize_kernel(const float* __restrict__
   const float s = *scale;
   const uint64_t t = threadIdx.x;
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  const uint64_t units = n / 4, steps = units / kStepUnits;
+  // whole steps only where most workgroups have one; else a unit per thread
+  const uint64_t units = n / 4, whole = units / kStepUnits;
+  const uint64_t steps = 2 * whole >= gridDim.x ? whole : 0;
   const f32x4_t* x4 = reinterpret_cast<const f32x4_t*>(x);
   uint32_t* q4 = reinterpret_cast<uint32_t*>(q);
   auto code4 = [s](f32x4_t v) {
@@ -273,17 +291,16 @@ int32_t launch_direct(const uint8_t* a, const uint8_t* b, const float* sa, const
   return fe2o3_host::after_launch();
 }
 
-// one workgroup per 4096-element step, at most 8192 striding over the rest
-unsigned grid_for(uint64_t n) {
-  uint64_t b = (n + 4095) / 4096;
-  if (b == 0) b = 1;
-  return (unsigned)(b < 8192 ? b : 8192);
+// one workgroup per `elements`, at most `most` striding over the rest
+unsigned grid_for(uint64_t n, uint64_t elements, uint64_t most) {
+  const uint64_t b = (n + elements - 1) / elements;
+  return (unsigned)std::min(std::max<uint64_t>(b, 1), most);
 }
 
 // kernels behind each entry point (fe2o3_kernel_resources)
 const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_amax_f32", "zero_f32_kernel", (const void*)zero_f32_kernel, 1, 0}),
-    fe2o3_host::KernelRegistrar({"fe2o3_amax_f32", "amax_kernel", (const void*)amax_kernel, 256, 0}),
+    fe2o3_host::KernelRegistrar({"fe2o3_amax_f32", "amax_kernel", (const void*)amax_kernel, kAmaxThreads, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_fp8_scale_from_amax", "scale_kernel", (const void*)scale_kernel, 1, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_quantize_e4m3", "quantize_kernel", (const void*)quantize_kernel, 256, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_kernel", (const void*)gemm_fp8_kernel<false, false>, 256, kFp8Smem}),
@@ -401,9 +418,15 @@ int32_t fe2o3_amax_f32(const float* x, uint64_t x_len, float* amax, void* stream
   if (!amax || (x_len && !x)) return FE2O3_ERR_NULL;
   if (((uintptr_t)x & 15u) != 0) return FE2O3_ERR_ALIGNMENT;
   hipStream_t s = (hipStream_t)stream;
+  tile_plan::Topology topo;
+  const int32_t topo_rc = fe2o3_host::device_topology(&topo);
+  if (topo_rc != FE2O3_OK) return topo_rc;
   zero_f32_kernel<<<1, 1, 0, s>>>(amax);
-  // at most 1024 workgroups (4 per CU), each striding over the tensor
-  if (x_len) amax_kernel<<<std::min(grid_for(x_len), 1024u), 256, 0, s>>>(x, x_len, amax);
+  // one workgroup per 4096 elements, at most one per CU (two from 256 MiB on,
+  // where the stream is worth more than the atomics: a linear of 8192^3 took
+  // 490 us before and 488 with them)
+  const unsigned most = topo.cus * (x_len >= (1u << 26) ? 2u : 1u);
+  if (x_len) amax_kernel<<<grid_for(x_len, 4096, most), kAmaxThreads, 0, s>>>(x, x_len, amax);
   return fe2o3_host::after_launch();
 }
 
@@ -421,7 +444,11 @@ int32_t fe2o3_quantize_e4m3(const float* x, uint64_t x_len, const float* scale, 
   if (x_len == 0) return FE2O3_OK;
   if (!x || !scale || !q) return FE2O3_ERR_NULL;
   if (((uintptr_t)x & 15u) != 0 || ((uintptr_t)q & 3u) != 0) return FE2O3_ERR_ALIGNMENT;
-  quantize_kernel<<<grid_for(x_len), 256, 0, (hipStream_t)stream>>>(x, x_len, scale, q);
+  // a step per workgroup; up to 2^20 elements (a decoding step's activations) a
+  // unit per thread, which occupies four times the CUs: a linear of 32 x 8192 x
+  // 8192 took 21.1 us, and 22.7 with steps here and in amax
+  const unsigned grid = grid_for(x_len, x_len <= (1u << 20) ? 1024 : 4096, 8192);
+  quantize_kernel<<<grid, 256, 0, (hipStream_t)stream>>>(x, x_len, scale, q);
   return fe2o3_host::after_launch();
 }
 

@@ -461,6 +461,22 @@ def test_amax_scale_and_quantize_bit_exact(gpu, oracle):
     assert_same(q.download(), oracle.quantize_e4m3(xh, float(s_ref)), "quantized")
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 4095, 4097, 16383, 16384, 16389, 65537, 1 << 20,
+                               (1 << 22) + 7])
+def test_amax_any_length_any_place(gpu, oracle, n):
+    """The largest magnitude first, last, in the middle, negative, and twice
+    on one output (a second call starts from zero again)."""
+    x = (np.random.default_rng(n).random(n) * 2 - 1).astype(np.float32)
+    amax = gpu.alloc(1, np.float32)
+    for at, value in ((0, 5.0), (n - 1, -7.0), (n // 2, 3.0)):
+        y = x.copy()
+        y[at] = value
+        _k().amax_f32(gpu.to_device(y), amax)
+        assert amax.download()[0] == np.float32(abs(value))
+    _k().amax_f32(gpu.to_device(x), amax)
+    assert amax.download()[0] == np.float32(oracle.amax_f32(x))
+
+
 def _fp8_case(gpu, oracle, m, n, k, points, block=None):
     """rel-err of the device GEMM at `points` (rows, cols); the outputs of
     whole rows block[0]..block[1]-1 among them come from the row-block form
