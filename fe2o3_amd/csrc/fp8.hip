@@ -282,11 +282,12 @@ int32_t launch_direct(const uint8_t* a, const uint8_t* b, const float* sa, const
   if (lds_rc != FE2O3_OK) return lds_rc;
   const gemm_direct::Launch l = gemm_direct::plan(m, n, k, 1u, topo.cus);
   if (l.grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
+  const dim3 grid = gemm_direct::list_grid(l.grid);
   if (l.wide)
-    gemm_fp8_direct_kernel<true><<<(unsigned)l.grid, gemm_direct::kThreads, l.smem, s>>>(
+    gemm_fp8_direct_kernel<true><<<grid, gemm_direct::kThreads, l.smem, s>>>(
         l.form, a, b, sa, sb, c, m, n, k, topo.xcds);
   else
-    gemm_fp8_direct_kernel<false><<<(unsigned)l.grid, gemm_direct::kThreads, l.smem, s>>>(
+    gemm_fp8_direct_kernel<false><<<grid, gemm_direct::kThreads, l.smem, s>>>(
         l.form, a, b, sa, sb, c, m, n, k, topo.xcds);
   return fe2o3_host::after_launch();
 }
@@ -464,15 +465,16 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   tile_plan::Topology topo;
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
-  // Few output tiles, and K = 0 (the empty sum, +0): the direct kernel,
-  // whatever the operands' alignment.
-  if (k == 0 || (gemm_direct::k_fits(k, 1u) && gemm_direct::prefer(m, n, k, 1u, topo.cus)))
-    return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
   // fast path: 16-byte operand rows (K a multiple of 16) and a 256-row fp8
   // panel (256 * k bytes) within its buffer resource's 32-bit range; K not a
   // multiple of 128 takes the edge tiles with a partial last stage
   const bool aligned_a = ((uintptr_t)a & 15u) == 0, aligned_b = ((uintptr_t)b & 15u) == 0;
   const bool fast = k % 16 == 0 && 256ull * k < (1ull << 31) && aligned_a && aligned_b;
+  // Few output tiles, and K = 0 (the empty sum, +0): the direct kernel,
+  // whatever the operands' alignment.
+  if (k == 0 || ((fast || gemm_direct::rows_ok(m)) && gemm_direct::k_fits(k, 1u) &&
+                 gemm_direct::prefer(m, n, k, 1u, topo.cus)))
+    return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
   // Rows the tile cannot read in place (K not a multiple of 16, or A or B
   // off a 16-byte boundary) are first copied into aligned rows of kp = K
   // rounded up to 16, zeros from K on, in stream-ordered scratch; the tile
@@ -491,8 +493,10 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
       scratch = nullptr;
     }
   }
-  if (!fast && scratch == nullptr)
+  if (!fast && scratch == nullptr) {
+    if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
     return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
+  }
   // every kernel's LDS limit is raised before anything is launched, so a
   // failure leaves C untouched
   int32_t rc = set_fp8_lds();

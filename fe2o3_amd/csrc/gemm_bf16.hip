@@ -233,11 +233,12 @@ int32_t launch_direct(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_
   if (lds_rc != FE2O3_OK) return lds_rc;
   const gemm_direct::Launch l = gemm_direct::plan(m, n, k, 2u, topo.cus);
   if (l.grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
+  const dim3 grid = gemm_direct::list_grid(l.grid);
   if (l.wide)
-    gemm_bf16_nt_direct_kernel<true><<<(unsigned)l.grid, gemm_direct::kThreads, l.smem, s>>>(
+    gemm_bf16_nt_direct_kernel<true><<<grid, gemm_direct::kThreads, l.smem, s>>>(
         l.form, a, b, c, m, n, k, topo.xcds);
   else
-    gemm_bf16_nt_direct_kernel<false><<<(unsigned)l.grid, gemm_direct::kThreads, l.smem, s>>>(
+    gemm_bf16_nt_direct_kernel<false><<<grid, gemm_direct::kThreads, l.smem, s>>>(
         l.form, a, b, c, m, n, k, topo.xcds);
   return fe2o3_host::after_launch();
 }
@@ -255,16 +256,17 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
   hipStream_t s = (hipStream_t)stream;
-  // Few output tiles, and K = 0 (the empty sum, +0): the direct kernel,
-  // whatever the operands' alignment.
-  if (k == 0 || (gemm_direct::k_fits(k, 2u) && gemm_direct::prefer(m, n, k, 2u, topo.cus)))
-    return launch_direct(a, b, c, m, n, k, topo, s);
   // fast path: 16-byte operand rows (K a multiple of 8), and a 256-row panel
   // (512 * k bytes) inside the 32-bit range of its buffer resource; whole
   // tiles with a 16-byte aligned C take the plain tile, any other M and N
   // the edge tile; K not a multiple of 64 the same tiles with a partial last
   // stage (KT)
   const bool fast = k % 8 == 0 && 512ull * k < (1ull << 31) && aligned16(a) && aligned16(b);
+  // Few output tiles, and K = 0 (the empty sum, +0): the direct kernel,
+  // whatever the operands' alignment.
+  if (k == 0 || ((fast || gemm_direct::rows_ok(m)) && gemm_direct::k_fits(k, 2u) &&
+                 gemm_direct::prefer(m, n, k, 2u, topo.cus)))
+    return launch_direct(a, b, c, m, n, k, topo, s);
   // Rows the tile cannot read in place (K not a multiple of 8, or A or B two
   // bytes past a 16-byte boundary) are first copied into aligned rows of kp
   // = K rounded up to 8, zeros from K on, in stream-ordered scratch; the
@@ -301,5 +303,6 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
     }
     (void)hipGetLastError();  // no stream-ordered scratch: the direct kernel
   }
+  if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
   return launch_direct(a, b, c, m, n, k, topo, s);
 }

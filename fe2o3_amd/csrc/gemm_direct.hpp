@@ -125,6 +125,16 @@ FE2O3_DEVICE u32x4_t load_end(const uint8_t* row, Off at, Off bytes) {
   return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
 }
 
+// HIP refuses a grid of 2^32 threads or more in one dimension, so the ids of a
+// list of workgroups continue in y from kGridX on; the last row of the grid
+// may run past the list.
+constexpr uint32_t kGridX = 1u << 22;
+inline dim3 list_grid(uint64_t workgroups) {
+  return dim3((unsigned)(workgroups < kGridX ? workgroups : kGridX),
+              (unsigned)((workgroups + kGridX - 1u) / kGridX));
+}
+FE2O3_DEVICE uint32_t list_id() { return blockIdx.y * kGridX + blockIdx.x; }
+
 // Output block (tm, tn) of workgroup `id`: each XCD takes a contiguous run of
 // the list (as tile_plan::xcd_tile_order does), block rows fastest, so that
 // the blocks that read the same rows of B run together behind one L2.
@@ -146,9 +156,10 @@ FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict
                         uint32_t xcds, uint8_t* smem) {
   const uint32_t lane = threadIdx.x & 63u, lr = lane & 15u, g = lane >> 4;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t tiles_m = (m - 1u) / (16u * MB) + 1u, tiles_n = (n - 1u) / (16u * NB) + 1u;
+  if (list_id() >= tiles_m * tiles_n) return;
   uint32_t tm, tn;
-  block_of(blockIdx.x, (m + 16u * MB - 1u) / (16u * MB), (n + 16u * NB - 1u) / (16u * NB), xcds,
-           &tm, &tn);
+  block_of(list_id(), tiles_m, tiles_n, xcds, &tm, &tn);
   const uint32_t row0 = tm * 16u * MB, col0 = tn * 16u * NB;
   const Off kbytes = (Off)k * T::kBytes;
   // this lane's rows as offsets from the block's first; rows past the end
@@ -349,6 +360,10 @@ inline bool prefer(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes, uint
   choose(m, n, cus, &cost);
   return cost <= (kbytes % 16u == 0u ? 10u : 18u);
 }
+// Operands that the pipelined tiles cannot read in place are taken up to 65535
+// blocks of 64 rows of A; more are a shape error.
+inline bool rows_ok(uint32_t m) { return ((uint64_t)m + 63u) / 64u <= 65535u; }
+
 // 64 rows of K within 32-bit byte offsets, as the chosen forms need
 inline bool k_fits(uint32_t k, uint32_t elem_bytes) { return 64ull * k * elem_bytes < (1ull << 32); }
 

@@ -563,7 +563,9 @@ __global__ void __launch_bounds__(kGsThreads, 3) gemm_general_kernel(
     float beta, uint32_t xcds) {
   __shared__ __attribute__((aligned(1024))) uint8_t smem[4 * kGsBuf];  // A0 A1 B0 B1
   uint32_t tm, tn;
-  gemm_core::xcd_tile_order(blockIdx.x, (m + 63u) / 64u, (n + 63u) / 64u, xcds, &tm, &tn);
+  const uint32_t tiles_m = (m - 1u) / 64u + 1u, tiles_n = (n - 1u) / 64u + 1u;
+  if (gemm_direct::list_id() >= tiles_m * tiles_n) return;
+  gemm_core::xcd_tile_order(gemm_direct::list_id(), tiles_m, tiles_n, xcds, &tm, &tn);
   const uint32_t rows = min(64u, m - tm * 64u), cols = min(64u, n - tn * 64u);
   if (n < 8u)
     general_tile<Cols::narrow>(a, b, c, n, k, lda, ldb, ldc, alpha, beta, tm, tn, rows, cols, smem);
@@ -793,7 +795,7 @@ int32_t general_gemm(const uint16_t* a, uint64_t a_len, const uint16_t* b, uint6
 in_registers:
   const uint64_t tiles = (((uint64_t)m + 63u) / 64u) * (((uint64_t)n + 63u) / 64u);
   if (((uint64_t)m + 63u) / 64u > 65535u || tiles > 0x7fffffffu) return FE2O3_ERR_SHAPE;
-  gemm_general_kernel<<<(unsigned)tiles, kGsThreads, 0, (hipStream_t)stream>>>(
+  gemm_general_kernel<<<gemm_direct::list_grid(tiles), kGsThreads, 0, (hipStream_t)stream>>>(
       a, b, c, m, n, k, lda, ldb, ldc, alpha, beta, topo.xcds);
   return fe2o3_host::after_launch();
 }

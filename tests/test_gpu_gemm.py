@@ -454,6 +454,26 @@ def test_gemm_bf16_nt_direct_forms(gpu, oracle, m, n, k):
     assert_same(got.download()[1:], want.download(), "2-byte offsets vs aligned")
 
 
+def test_gemm_bf16_nt_direct_limits(gpu):
+    """More workgroups than a grid's x dimension takes (2^32 threads, 512 a
+    workgroup, 64 columns each): C = 1 * B exactly; and the shape error for
+    operands off the 16-byte rows with more than 65535 blocks of 64 rows."""
+    kern = _kernels()
+    prep = kern.gemm_bf16_nt_gpu.Kernel.load(gpu)
+    n = (1 << 29) + 100
+    pattern = (np.arange(28_673, dtype=np.uint32) * 40503 >> 3).astype(np.uint16) & 0x3EFF | 0x0100
+    b = np.resize(pattern, n)  # finite, normal, positive
+    c = gpu.alloc(n, np.uint16)
+    prep.prepare(gpu.to_device(np.array([0x3F80], np.uint16)), gpu.to_device(b), c, 1, n, 1).launch()
+    assert np.array_equal(c.download(), b)
+    m = 65535 * 64 + 1
+    a = gpu.to_device(np.zeros(m * 9, np.uint16))
+    with pytest.raises(RuntimeError) as refused:
+        prep.prepare(a, gpu.to_device(np.zeros(9, np.uint16)), gpu.alloc(m, np.uint16),
+                     m, 1, 9).launch()
+    assert refused.value.status == -3
+
+
 # Outputs just too large for the direct kernel: the 128x128 small-grid forms,
 # whole and edge tiles, one K step to several groups of three, partial last
 # stages, and repacked rows (K odd, 1600 x 1500: above the direct kernel's line
