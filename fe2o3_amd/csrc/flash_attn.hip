@@ -437,7 +437,7 @@ __global__ void __launch_bounds__(THREADS, 8 / WAVES) flash_fwd_ragged_kernel(
 constexpr int SQ = 2, SG = 2, SK = 32;
 constexpr int S_ROWS = 32 * SQ, S_THREADS = 64 * SQ * SG;
 constexpr uint32_t S_TILE = SK * D * 2, S_STAGE = 2 * S_TILE, S_GROUP = 2 * S_STAGE;
-constexpr uint32_t S_ACC = SQ * SG * 64u * 64u * 4u;  // the sums, 128 KiB (the tiles' LDS reused)
+constexpr uint32_t S_ACC = SQ * SG * 64u * 64u * 4u;  // the sums, 64 KiB (the tiles' LDS reused)
 constexpr int S_SMEM = (int)(S_ACC + SQ * SG * 64u * 8u);
 static_assert(SG * S_GROUP <= S_ACC, "the sums reuse the tiles' LDS");
 constexpr int S_DB = 4 / SG;  // 32-wide d blocks that a group gathers
