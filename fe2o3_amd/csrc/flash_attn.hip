@@ -504,7 +504,10 @@ FE2O3_DEVICE void flash_split_block(const uint16_t* __restrict__ q, const uint16
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
-  float m_ref = -INFINITY, l_run = 0.0f;  // as in flash_block
+  // As in flash_block, but from the lowest finite value on: a group's own first
+  // tile may hold only scores of -inf (keys that the caller shut out), whose
+  // exponentials against -inf would be NaN and against this are 0.
+  float m_ref = -__FLT_MAX__, l_run = 0.0f;
 
   const uint32_t kv_tiles = (seq + SK - 1u) / SK;
   const uint32_t n_kv = CAUSAL ? min((qt + 1u) * (uint32_t)(S_ROWS / SK), kv_tiles) : kv_tiles;
@@ -623,8 +626,8 @@ FE2O3_DEVICE void flash_split_block(const uint16_t* __restrict__ q, const uint16
           acc[db][4 * e4], acc[db][4 * e4 + 1], acc[db][4 * e4 + 2], acc[db][4 * e4 + 3]};
   stats[wave * 64u + lane] = f32x2_t{m_ref, l_own};
   __syncthreads();
-  // a group without an active tile has m = -inf, l = 0: weight 0.  A row's
-  // first key is always some group's, so the largest m is finite.
+  // a group without an active tile, or with scores of -inf alone, has the
+  // lowest m, l = 0 and sums of 0; a row of nothing else divides 0 by 0
   f32x2_t st[SG];
   float m = -INFINITY, l = 0.0f, weight[SG];
 #pragma unroll

@@ -423,6 +423,25 @@ def test_flash_split_keys_all_rows(gpu, oracle, b, h, s, causal):
     test_flash_any_seq_all_rows(gpu, oracle, b, h, s, causal)
 
 
+@pytest.mark.parametrize("causal,first", [(False, 0), (False, 32), (True, 32)])
+@pytest.mark.parametrize("s", [96, 200])
+def test_flash_split_keys_shut_out_tile(gpu, oracle, s, causal, first):
+    """32 keys whose scores are all -inf (one infinite channel), which are the
+    first tile of one wave group: they take no part, the other keys give the
+    f64 oracle's rows and LSE."""
+    h, rng = 2, np.random.default_rng(s + first)
+    q, k, v = (rng.standard_normal((h, s, 128)).astype(np.float32) for _ in range(3))
+    q[:, :, 0] = 1.0
+    k[:, first:first + 32, 0] = -np.inf
+    qkv = [oracle.bf16_from_f32(np.ascontiguousarray(x).ravel()) for x in (q, k, v)]
+    host, out, lse, scale = _flash(gpu, 1, h, s, causal, seed=0, qkv=qkv)
+    bh, rows = np.repeat(np.arange(h, dtype=np.uint32), s), np.tile(np.arange(s, dtype=np.uint32), h)
+    rc, ref, ref_lse = oracle.flash_attention_rows_bf16(*host, s, 128, causal, scale, bh, rows)
+    assert rc == 0 and np.all(np.isfinite(ref))
+    assert rel_err(out.reshape(-1, 128), ref) <= 1e-2
+    assert rel_err(lse, ref_lse) <= 1e-5  # fp32 output: the 1e-5 bar
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("pattern", ["normal", "ramp", "jump"])
 @pytest.mark.parametrize("s", [37, 64, 200, 256, 300, 512, 640])
