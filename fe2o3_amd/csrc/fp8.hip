@@ -12,8 +12,8 @@
 // is 128 bytes of k per row, i.e. 128 fp8 values, each taken by one
 // v_mfma_f32_16x16x128_f8f6f4 (5.0 PFLOP/s dense peak).  Any M
 // and N run on it (edge tiles store only their valid rows and columns).
-// Outputs of few tiles, at any alignment and K (K = 0 writes +0), take the
-// direct kernel (gemm_direct.hpp).
+// Outputs of few tiles, at any alignment and K, take the direct kernel
+// (gemm_direct.hpp); K = 0 writes +0.
 #include "common.hpp"
 #include "gemm_core.hpp"
 #include "gemm_direct.hpp"
@@ -327,7 +327,8 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_128_kernel<3, edge, tail, k tail>", (const void*)gemm_fp8_128_kernel<3, false, true, true>, 256, kFp8SmallSmem<3>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel", (const void*)gemm_fp8_direct_kernel<false>, gemm_direct::kThreads, gemm_direct::kLightSmem}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "repack_bytes_kernel", (const void*)repack_bytes_kernel, 256, 0}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel<wide>", (const void*)gemm_fp8_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem})};
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel<wide>", (const void*)gemm_fp8_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem}),
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "zero_fill_kernel", (const void*)gemm_core::zero_fill_kernel<uint16_t>, 256, 0})};
 
 }  // namespace
 
@@ -462,6 +463,10 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   if (c_len == 0) return FE2O3_OK;
   if ((a_len && !a) || (b_len && !b) || !c || !scale_a || !scale_b) return FE2O3_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
+  if (k == 0) {  // the empty sum: +0 whatever the scales, which are not read
+    gemm_core::zero_fill_kernel<<<gemm_core::zero_fill_grid(c_len), 256, 0, s>>>(c, c_len);
+    return fe2o3_host::after_launch();
+  }
   tile_plan::Topology topo;
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
@@ -470,10 +475,9 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   // multiple of 128 takes the edge tiles with a partial last stage
   const bool aligned_a = ((uintptr_t)a & 15u) == 0, aligned_b = ((uintptr_t)b & 15u) == 0;
   const bool fast = k % 16 == 0 && 256ull * k < (1ull << 31) && aligned_a && aligned_b;
-  // Few output tiles, and K = 0 (the empty sum, +0): the direct kernel,
-  // whatever the operands' alignment.
-  if (k == 0 || ((fast || gemm_direct::rows_ok(m)) && gemm_direct::k_fits(k, 1u) &&
-                 gemm_direct::prefer(m, n, k, 1u, topo.cus)))
+  // few output tiles: the direct kernel, whatever the operands' alignment
+  if ((fast || gemm_direct::rows_ok(m)) && gemm_direct::k_fits(k, 1u) &&
+      gemm_direct::prefer(m, n, k, 1u, topo.cus))
     return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
   // Rows the tile cannot read in place (K not a multiple of 16, or A or B
   // off a 16-byte boundary) are first copied into aligned rows of kp = K

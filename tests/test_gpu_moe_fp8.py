@@ -673,6 +673,19 @@ def test_gemm_fp8_k0_writes_positive_zero(gpu):
     assert c.guards_intact() and c.download().tolist() == [0] * 63
 
 
+@pytest.mark.parametrize("sa,sb", [(-1.0, 1.0), (0.5, -2.0), (np.inf, 1.0), (1.0, -np.inf),
+                                   (np.nan, 1.0), (3e38, 3e38), (np.inf, 0.0)])
+@pytest.mark.parametrize("m,n", [(7, 9), (300, 520)])
+def test_gemm_fp8_k0_is_positive_zero_for_any_scales(gpu, m, n, sa, sb):
+    """The empty sum is +0 bit for bit whatever the scales: negative, infinite
+    (an amax over data that holds an infinity), NaN, or overflowing together."""
+    scales = [gpu.to_device(np.array([x], np.float32)) for x in (sa, sb)]
+    empty = gpu.alloc(0, np.uint8)
+    c = Guarded(gpu, np.full(m * n, 0xFFFF, np.uint16))
+    _k().gemm_fp8_nt(empty, empty, *scales, c.body, m, n, 0)
+    assert c.guards_intact() and not c.download().any()
+
+
 def test_gemm_fp8_config4_sampled(gpu, oracle):
     """8192^3 e4m3 with amax/448 per-tensor scales; one
     whole 128-row block (rows 4096..4223, all 8192 columns: 1M outputs at
