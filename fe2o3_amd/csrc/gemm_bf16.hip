@@ -138,7 +138,8 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_128_kernel<2, edge, tail, k tail>", (const void*)gemm_bf16_nt_128_kernel<2, false, true, true>, 256, kSmallSmem<2>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_128_kernel<3, edge, tail, k tail>", (const void*)gemm_bf16_nt_128_kernel<3, false, true, true>, 256, kSmallSmem<3>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel", (const void*)gemm_bf16_nt_direct_kernel<false>, gemm_direct::kThreads, gemm_direct::kLightSmem}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel<wide>", (const void*)gemm_bf16_nt_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem})};
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel<wide>", (const void*)gemm_bf16_nt_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem}),
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "zero_fill_kernel", (const void*)gemm_core::zero_fill_kernel<uint16_t>, 256, 0})};
 
 // Raises every fast-path kernel's dynamic-LDS limit once per process.
 int32_t set_fast_lds() {
@@ -252,20 +253,23 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
     return FE2O3_ERR_LENGTH;
   if (c_len == 0) return FE2O3_OK;
   if ((a_len && !a) || (b_len && !b) || !c) return FE2O3_ERR_NULL;
+  hipStream_t s = (hipStream_t)stream;
+  if (k == 0) {
+    gemm_core::zero_fill_kernel<<<gemm_core::zero_fill_grid(c_len), 256, 0, s>>>(c, c_len);
+    return fe2o3_host::after_launch();
+  }
   tile_plan::Topology topo;
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
-  hipStream_t s = (hipStream_t)stream;
   // fast path: 16-byte operand rows (K a multiple of 8), and a 256-row panel
   // (512 * k bytes) inside the 32-bit range of its buffer resource; whole
   // tiles with a 16-byte aligned C take the plain tile, any other M and N
   // the edge tile; K not a multiple of 64 the same tiles with a partial last
   // stage (KT)
   const bool fast = k % 8 == 0 && 512ull * k < (1ull << 31) && aligned16(a) && aligned16(b);
-  // Few output tiles, and K = 0 (the empty sum, +0): the direct kernel,
-  // whatever the operands' alignment.
-  if (k == 0 || ((fast || gemm_direct::rows_ok(m)) && gemm_direct::k_fits(k, 2u) &&
-                 gemm_direct::prefer(m, n, k, 2u, topo.cus)))
+  // few output tiles: the direct kernel, whatever the operands' alignment
+  if ((fast || gemm_direct::rows_ok(m)) && gemm_direct::k_fits(k, 2u) &&
+      gemm_direct::prefer(m, n, k, 2u, topo.cus))
     return launch_direct(a, b, c, m, n, k, topo, s);
   // Rows the tile cannot read in place (K not a multiple of 8, or A or B two
   // bytes past a 16-byte boundary) are first copied into aligned rows of kp

@@ -1,6 +1,6 @@
 // gemm_direct.hpp -- GEMMs with too few output tiles for the pipelined tile
 // (gemm_pipe.hpp) to fill the device: a decoding step's few activation rows,
-// small outputs, and operands at any alignment with any K.
+// small outputs, and operands at any alignment with any K above 0.
 //
 // C[m][n] = A[m][k] B[n][k]^T, both operands k-contiguous.  A workgroup of 8
 // waves owns an output block of 16 MB x 16 NB and splits K over its waves:
@@ -147,7 +147,7 @@ FE2O3_DEVICE void block_of(uint32_t id, uint32_t tiles_m, uint32_t tiles_n, uint
 }
 
 // One output block.  T: Bf16 or Fp8.  D: units in flight per wave.  smem:
-// kWaves * max(MB * NB, 2 (MB + NB)) KiB.  c: m x n bf16, rows n apart.  k may be 0 (C is +0).
+// kWaves * max(MB * NB, 2 (MB + NB)) KiB.  c: m x n bf16, rows n apart.
 // Off: of byte offsets within the block's rows (uint32_t while 64 rows of K
 // fit it).
 template <class T, int MB, int NB, int D, class Off = uint32_t>
