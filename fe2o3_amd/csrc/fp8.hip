@@ -260,8 +260,6 @@ int32_t repack_bytes(const uint8_t* src, uint32_t rows, uint32_t cols, uint8_t* 
   return fe2o3_host::after_launch();
 }
 
-constexpr uint32_t kRepackMin = 128;  // outputs at least this in M and N repack
-
 // ---- few output tiles, any alignment, any K ----------------------------------------------
 template <bool WIDE>
 __global__ void __launch_bounds__(gemm_direct::kThreads, WIDE ? 2 : 4) gemm_fp8_direct_kernel(
@@ -271,6 +269,28 @@ __global__ void __launch_bounds__(gemm_direct::kThreads, WIDE ? 2 : 4) gemm_fp8_
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   gemm_direct::run_form<gemm_direct::Fp8, WIDE>(form, a, b, c, m, n, k, scale_a[0] * scale_b[0],
                                                 xcds, smem);
+}
+
+__global__ void __launch_bounds__(gemm_direct::kThreads, 2) gemm_fp8_in_order_kernel(
+    const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
+    const float* __restrict__ scale_a, const float* __restrict__ scale_b,
+    uint16_t* __restrict__ c, uint32_t m, uint32_t n, uint32_t k) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  gemm_direct::in_order_block<gemm_direct::Fp8>(a, b, c, m, n, k, scale_a[0] * scale_b[0], smem);
+}
+
+int32_t launch_in_order(const uint8_t* a, const uint8_t* b, const float* sa, const float* sb,
+                        uint16_t* c, uint32_t m, uint32_t n, uint32_t k, hipStream_t s) {
+  static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
+      {(const void*)gemm_fp8_in_order_kernel}, gemm_direct::kLightSmem);
+  if (lds_rc != FE2O3_OK) return lds_rc;
+  const uint64_t blocks = gemm_direct::in_order_blocks(m, n);
+  if (blocks > 0x7fffffffu) return FE2O3_ERR_SHAPE;
+  const dim3 grid =
+      gemm_direct::list_grid((blocks + gemm_direct::kWaves - 1u) / gemm_direct::kWaves);
+  gemm_fp8_in_order_kernel<<<grid, gemm_direct::kThreads, gemm_direct::kLightSmem, s>>>(
+      a, b, sa, sb, c, m, n, k);
+  return fe2o3_host::after_launch();
 }
 
 int32_t launch_direct(const uint8_t* a, const uint8_t* b, const float* sa, const float* sb,
@@ -328,6 +348,7 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel", (const void*)gemm_fp8_direct_kernel<false>, gemm_direct::kThreads, gemm_direct::kLightSmem}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "repack_bytes_kernel", (const void*)repack_bytes_kernel, 256, 0}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel<wide>", (const void*)gemm_fp8_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem}),
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_in_order_kernel", (const void*)gemm_fp8_in_order_kernel, gemm_direct::kThreads, gemm_direct::kLightSmem}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "zero_fill_kernel", (const void*)gemm_core::zero_fill_kernel<uint16_t>, 256, 0})};
 
 }  // namespace
@@ -484,10 +505,11 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   // rounded up to 16, zeros from K on, in stream-ordered scratch; the tile
   // then runs on kp, whose zeros fall where its partial last stage puts
   // zeros anyway, so an operand that is only misaligned gives the bits of
-  // the aligned one.  Outputs below 128 x 128, and devices without
-  // stream-ordered scratch, take the direct kernel.
+  // the aligned one.  Smaller outputs, and devices without stream-ordered
+  // scratch, take the direct kernel, in K order where the tile could run the
+  // sizes (gemm_direct::tile_sizes).
   const uint32_t kp = (k + 15u) & ~15u;
-  const bool repack = !fast && m >= kRepackMin && n >= kRepackMin && 256ull * kp < (1ull << 31);
+  const bool repack = !fast && gemm_direct::repack(m, n, k, 1u);
   void* scratch = nullptr;
   if (repack) {
     const bool ra = k % 16 != 0 || !aligned_a, rb = k % 16 != 0 || !aligned_b;
@@ -499,6 +521,8 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   }
   if (!fast && scratch == nullptr) {
     if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
+    if (gemm_direct::tile_sizes(m, n, k, 1u))
+      return launch_in_order(a, b, scale_a, scale_b, c, m, n, k, s);
     return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
   }
   // every kernel's LDS limit is raised before anything is launched, so a

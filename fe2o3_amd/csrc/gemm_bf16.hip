@@ -31,6 +31,15 @@ __global__ void __launch_bounds__(gemm_direct::kThreads, WIDE ? 2 : 4) gemm_bf16
       1.0f, xcds, smem);
 }
 
+__global__ void __launch_bounds__(gemm_direct::kThreads, 4) gemm_bf16_nt_in_order_kernel(
+    const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
+    uint32_t m, uint32_t n, uint32_t k) {
+  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+  gemm_direct::in_order_block<gemm_direct::Bf16>(reinterpret_cast<const uint8_t*>(a),
+                                                 reinterpret_cast<const uint8_t*>(b), c, m, n, k,
+                                                 1.0f, smem);
+}
+
 // ---- fast path ----------------------------------------------------------------------------
 // 256x256 tiles, 64 k per LDS stage (128-byte rows), two stages, 16x16x32
 // MFMAs in a fixed issue order (gemm_pipe.hpp).
@@ -139,6 +148,7 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_128_kernel<3, edge, tail, k tail>", (const void*)gemm_bf16_nt_128_kernel<3, false, true, true>, 256, kSmallSmem<3>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel", (const void*)gemm_bf16_nt_direct_kernel<false>, gemm_direct::kThreads, gemm_direct::kLightSmem}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel<wide>", (const void*)gemm_bf16_nt_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem}),
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_in_order_kernel", (const void*)gemm_bf16_nt_in_order_kernel, gemm_direct::kThreads, gemm_direct::kLightSmem}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "zero_fill_kernel", (const void*)gemm_core::zero_fill_kernel<uint16_t>, 256, 0})};
 
 // Raises every fast-path kernel's dynamic-LDS limit once per process.
@@ -224,8 +234,6 @@ int32_t launch_fast(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t 
 }  // namespace
 
 namespace {
-constexpr uint32_t kRepackMin = 128;  // outputs at least this in M and N repack
-
 int32_t launch_direct(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m, uint32_t n,
                       uint32_t k, const tile_plan::Topology& topo, hipStream_t s) {
   static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
@@ -241,6 +249,20 @@ int32_t launch_direct(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_
   else
     gemm_bf16_nt_direct_kernel<false><<<grid, gemm_direct::kThreads, l.smem, s>>>(
         l.form, a, b, c, m, n, k, topo.xcds);
+  return fe2o3_host::after_launch();
+}
+
+int32_t launch_in_order(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m, uint32_t n,
+                        uint32_t k, hipStream_t s) {
+  static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
+      {(const void*)gemm_bf16_nt_in_order_kernel}, gemm_direct::kLightSmem);
+  if (lds_rc != FE2O3_OK) return lds_rc;
+  const uint64_t blocks = gemm_direct::in_order_blocks(m, n);
+  if (blocks > 0x7fffffffu) return FE2O3_ERR_SHAPE;
+  const dim3 grid =
+      gemm_direct::list_grid((blocks + gemm_direct::kWaves - 1u) / gemm_direct::kWaves);
+  gemm_bf16_nt_in_order_kernel<<<grid, gemm_direct::kThreads, gemm_direct::kLightSmem, s>>>(
+      a, b, c, m, n, k);
   return fe2o3_host::after_launch();
 }
 }  // namespace
@@ -276,10 +298,11 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
   // = K rounded up to 8, zeros from K on, in stream-ordered scratch; the
   // tile then runs on kp, whose zeros fall where its partial last stage
   // puts zeros anyway, so an operand that is only misaligned gives the bits
-  // of the aligned one.  Outputs below 128 x 128, and devices without
-  // stream-ordered scratch, take the direct kernel.
+  // of the aligned one.  Smaller outputs, and devices without stream-ordered
+  // scratch, take the direct kernel, in K order where the tile could run the
+  // sizes (gemm_direct::tile_sizes).
   const uint32_t kp = (k + 7u) & ~7u;
-  if (fast || (m >= kRepackMin && n >= kRepackMin && 512ull * kp < (1ull << 31))) {
+  if (fast || gemm_direct::repack(m, n, k, 2u)) {
     const int32_t lds_rc = set_fast_lds();  // before any launch: a failure leaves C untouched
     if (lds_rc != FE2O3_OK) return lds_rc;
     const tile_plan::Plan plan = tile_plan::plan(m, n, topo);
@@ -308,5 +331,6 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
     (void)hipGetLastError();  // no stream-ordered scratch: the direct kernel
   }
   if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
+  if (gemm_direct::tile_sizes(m, n, k, 2u)) return launch_in_order(a, b, c, m, n, k, s);
   return launch_direct(a, b, c, m, n, k, topo, s);
 }

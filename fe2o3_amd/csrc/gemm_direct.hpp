@@ -16,6 +16,11 @@
 // (bf16 16 x 4096 x 14336: 34.1 us against 24.7; 128 x 4096 x 4096: 23.9
 // against 13.6).
 //
+// The in-order form (in_order_block) gives every wave an output block of its
+// own and all of K instead: C's bits are then those of the pipelined tile, for
+// the calls that would take the tile if their operands could be read in place
+// or copied.
+//
 // What bounds it: with one block row (m <= 16 MB) the weights' HBM stream,
 // else the 64 bytes a clock that a CU loads (16 (MB + NB) rows of K per
 // block).  bf16 16 x 4096 x 4096 runs at 4.4 TB/s, fp8 32 x 8192 x 8192 at 5.4;
@@ -40,13 +45,16 @@ typedef uint32_t u32x8_t __attribute__((ext_vector_type(8)));
 // One 16-row block's unit, two 16-byte pieces per lane.  As loaded: of rows
 // l / 8 (words 0-3) and 8 + l / 8 (words 4-7) the piece l % 8.  As an MFMA
 // operand: of row l % 16 the pieces l / 16 (words 0-3) and 4 + l / 16 (words
-// 4-7); both operands use the same assignment, so every k meets its own.
+// 4-7); both operands use the same assignment, so every k meets its own.  (In
+// the in-order form the pieces that the pipelined tile's MFMA takes from that
+// lane: for fp8 2 (l / 16) and the next.)
 typedef u32x8_t Frag;
 
 struct Bf16 {
   static constexpr uint32_t kBytes = 2;  // per element
   static constexpr bool kScaled = false;
   static constexpr int kDeep = 3;  // units in flight of the widest forms
+  static FE2O3_DEVICE uint32_t tile_piece(uint32_t g, uint32_t h) { return 4u * h + g; }
   static FE2O3_DEVICE void mma(const Frag& b, const Frag& a, f32x4_t& acc) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -63,6 +71,7 @@ struct Fp8 {
   static constexpr uint32_t kBytes = 1;
   static constexpr bool kScaled = true;
   static constexpr int kDeep = 2;
+  static FE2O3_DEVICE uint32_t tile_piece(uint32_t g, uint32_t h) { return 2u * g + h; }
   static FE2O3_DEVICE void mma(const Frag& b, const Frag& a, f32x4_t& acc) {
     acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
         __builtin_bit_cast(i32x8_t, b), __builtin_bit_cast(i32x8_t, a), acc, 0, 0, 0, 0, 0, 0);
@@ -146,20 +155,23 @@ FE2O3_DEVICE void block_of(uint32_t id, uint32_t tiles_m, uint32_t tiles_n, uint
   *tn = id / tiles_m;
 }
 
-// One output block.  T: Bf16 or Fp8.  D: units in flight per wave.  smem:
-// kWaves * max(MB * NB, 2 (MB + NB)) KiB.  c: m x n bf16, rows n apart.
-// Off: of byte offsets within the block's rows (uint32_t while 64 rows of K
-// fit it).
-template <class T, int MB, int NB, int D, class Off = uint32_t>
+// One output block per workgroup, or (IN_ORDER) per wave.  T: Bf16 or Fp8.  D:
+// units in flight per wave.  smem: kWaves * max(MB * NB, 2 (MB + NB)) KiB.  c:
+// m x n bf16, rows n apart.  Off: of byte offsets within the block's rows
+// (uint32_t while 64 rows of K fit it).
+template <class T, int MB, int NB, int D, class Off = uint32_t, bool IN_ORDER = false>
 FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
                         uint16_t* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, float scale,
                         uint32_t xcds, uint8_t* smem) {
   const uint32_t lane = threadIdx.x & 63u, lr = lane & 15u, g = lane >> 4;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t tiles_m = (m - 1u) / (16u * MB) + 1u, tiles_n = (n - 1u) / (16u * NB) + 1u;
-  if (list_id() >= tiles_m * tiles_n) return;
+  // IN_ORDER: a workgroup's waves take neighbouring blocks of the list, and
+  // share nothing, so a wave past its end just leaves
+  const uint32_t id = IN_ORDER ? list_id() * kWaves + wave : list_id();
+  if (id >= tiles_m * tiles_n) return;
   uint32_t tm, tn;
-  block_of(list_id(), tiles_m, tiles_n, xcds, &tm, &tn);
+  block_of(id, tiles_m, tiles_n, IN_ORDER ? 1u : xcds, &tm, &tn);
   const uint32_t row0 = tm * 16u * MB, col0 = tn * 16u * NB;
   const Off kbytes = (Off)k * T::kBytes;
   // this lane's rows as offsets from the block's first; rows past the end
@@ -178,8 +190,9 @@ FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict
   uint8_t* own = smem + wave * (uint32_t)(MB + NB) * 2048u;
   const uint32_t wr0 = pr * 128u + ((pc ^ G::swz(pr)) << 4);
   const uint32_t wr1 = (8u + pr) * 128u + ((pc ^ G::swz(8u + pr)) << 4);
-  const uint32_t rd0 = lr * 128u + ((g ^ G::swz(lr)) << 4);
-  const uint32_t rd1 = lr * 128u + (((4u + g) ^ G::swz(lr)) << 4);
+  auto piece = [&](uint32_t h) { return IN_ORDER ? T::tile_piece(g, h) : 4u * h + g; };
+  const uint32_t rd0 = lr * 128u + ((piece(0) ^ G::swz(lr)) << 4);
+  const uint32_t rd1 = lr * 128u + ((piece(1) ^ G::swz(lr)) << 4);
 
   f32x4_t acc[MB][NB];
 #pragma unroll
@@ -187,10 +200,12 @@ FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   u32x4_t af[D][2 * MB], bf[D][2 * NB];
+  constexpr uint32_t kStride = IN_ORDER ? 1u : kWaves;  // units between the wave's own
+  const uint32_t first_unit = IN_ORDER ? 0u : wave;
   // the wave's unit u into set s
   auto load = [&](int s, uint32_t u) {
     __builtin_amdgcn_sched_barrier(0);  // not before the set's last use: it has no second one
-    const uint64_t at = ((uint64_t)u * kWaves + wave) * kUnit;
+    const uint64_t at = ((uint64_t)u * kStride + first_unit) * kUnit;
     const ScalarBase pa(a0 + at), pb(b0 + at);
 #pragma unroll
     for (int j = 0; j < 2 * NB; ++j) bf[s][j] = pb.load16(bo[j]);
@@ -229,7 +244,8 @@ FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict
     __builtin_amdgcn_sched_barrier(0);
   };
   const uint32_t units = (uint32_t)(kbytes / kUnit);  // whole ones
-  const uint32_t mine = units > wave ? (units - wave + kWaves - 1u) / kWaves : 0u;
+  const uint32_t mine =
+      units > first_unit ? (units - first_unit + kStride - 1u) / kStride : 0u;
   if (mine >= (uint32_t)D) {
 #pragma unroll
     for (int s = 0; s < D; ++s) load(s, s);
@@ -261,7 +277,7 @@ FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict
     for (int s = 0; s < D; ++s)
       if ((uint32_t)s < mine) mma(s);
   }
-  if (kbytes % kUnit != 0u && units % kWaves == wave) {  // the partial last unit
+  if (kbytes % kUnit != 0u && units % kStride == first_unit) {  // the partial last unit
     const Off at = (Off)units * kUnit + 16u * pc;
     auto row_of = [](const uint8_t* base, Off off) {
       __builtin_amdgcn_sched_barrier(0);  // one piece at a time: registers, not latency
@@ -276,25 +292,12 @@ FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict
     mma(0);
   }
 
-  __syncthreads();  // the partial sums take the LDS of all waves' units
-  // partial sums [wave][block][lane], then one thread per 4 columns of a row
-  // adds the waves' in order
-  f32x4_t* part = reinterpret_cast<f32x4_t*>(smem);
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j) part[(wave * MB * NB + i * NB + j) * 64u + lane] = acc[i][j];
-  __syncthreads();
   const bool vec = n % 4u == 0u && ((uintptr_t)c & 7u) == 0u;
-#pragma unroll
-  for (uint32_t t = threadIdx.x; t < MB * NB * 64u; t += kThreads) {
-    f32x4_t sum = part[t];
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w) sum += part[w * MB * NB * 64u + t];
-    const uint32_t blk = t >> 6, l = t & 63u;
+  // lane l's 4 columns of 16 x 16 block blk (i * NB + j)
+  auto store = [&](uint32_t blk, uint32_t l, f32x4_t sum) {
     const uint32_t row = row0 + 16u * (blk / NB) + (l & 15u);
     const uint32_t col = col0 + 16u * (blk % NB) + 4u * (l >> 4);
-    if (row >= m || col >= n) continue;
+    if (row >= m || col >= n) return;
     uint16_t* out = c + (uint64_t)row * n + col;
     if constexpr (T::kScaled)
 #pragma unroll
@@ -307,6 +310,29 @@ FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict
       for (int e = 0; e < 4; ++e)
         if (col + e < n) out[e] = bf16_bits_from_f32(sum[e]);
     }
+  };
+  if constexpr (IN_ORDER) {
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) store(i * NB + j, lane, acc[i][j]);
+    return;
+  }
+  __syncthreads();  // the partial sums take the LDS of all waves' units
+  // partial sums [wave][block][lane], then one thread per 4 columns of a row
+  // adds the waves' in order
+  f32x4_t* part = reinterpret_cast<f32x4_t*>(smem);
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) part[(wave * MB * NB + i * NB + j) * 64u + lane] = acc[i][j];
+  __syncthreads();
+#pragma unroll
+  for (uint32_t t = threadIdx.x; t < MB * NB * 64u; t += kThreads) {
+    f32x4_t sum = part[t];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) sum += part[w * MB * NB * 64u + t];
+    store(t >> 6, t & 63u, sum);
   }
 }
 
@@ -364,6 +390,28 @@ inline bool prefer(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes, uint
 // blocks of 64 rows of A; more are a shape error.
 inline bool rows_ok(uint32_t m) { return ((uint64_t)m + 63u) / 64u <= 65535u; }
 
+// A call past prefer's line whose operands the tile cannot read in place, but
+// could at these sizes at another alignment or after a copy: its C has the
+// tile's bits on every way there.
+//   tile_sizes: outputs from 128 x 128 on (any K, copied into rows of whole
+//     pieces), and smaller ones whose rows are whole pieces.
+//   repack: they are copied into scratch for the tile; small ones only when
+//     K is long, else the in-order form, which also serves without scratch
+//     (us, copies and tile against in order: bf16 100 x 8192 x 4096 53 | 114,
+//     fp8 38 | 59; bf16 127 x 9000 x 1024 29 | 31, fp8 29 | 17; bf16 16 x 40000
+//     x 256 25 | 10).
+constexpr uint32_t kRepackMin = 128;
+inline bool tile_sizes(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) {
+  const uint64_t kbytes = (uint64_t)k * elem_bytes, padded = (kbytes + 15u) / 16u * 16u;
+  return 256ull * padded < (1ull << 31) &&
+         (padded == kbytes || (m >= kRepackMin && n >= kRepackMin));
+}
+inline bool repack(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) {
+  return tile_sizes(m, n, k, elem_bytes) &&
+         ((m >= kRepackMin && n >= kRepackMin) ||
+          ((uint64_t)k * elem_bytes > 2048u && rows_ok(m)));
+}
+
 // 64 rows of K within 32-bit byte offsets, as the chosen forms need
 inline bool k_fits(uint32_t k, uint32_t elem_bytes) { return 64ull * k * elem_bytes < (1ull << 32); }
 
@@ -380,6 +428,11 @@ inline Launch plan(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes, uint
   const int form = k_fits(k, elem_bytes) ? choose(m, n, cus) : kNumForms;
   const Form f = form < kNumForms ? kForms[form] : Form{1, 4, true};
   return {form, f.wide, grid_of(f, m, n), smem_of(f.mb, f.nb)};
+}
+
+// the in-order form's blocks, one per wave
+inline uint64_t in_order_blocks(uint32_t m, uint32_t n) {
+  return grid_of(Form{2, 2, false}, m, n);
 }
 
 constexpr int kLightSmem = (int)smem_of(2, 2), kWideSmem = (int)smem_of(4, 2);
@@ -406,6 +459,12 @@ FE2O3_DEVICE void run_form(int form, const uint8_t* a, const uint8_t* b, uint16_
     }
   }
 #undef FE2O3_DIRECT
+}
+
+template <class T>
+FE2O3_DEVICE void in_order_block(const uint8_t* a, const uint8_t* b, uint16_t* c, uint32_t m,
+                                 uint32_t n, uint32_t k, float scale, uint8_t* smem) {
+  block<T, 2, 2, 2, uint32_t, true>(a, b, c, m, n, k, scale, 1u, smem);
 }
 
 }  // namespace gemm_direct

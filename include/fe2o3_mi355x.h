@@ -258,15 +258,16 @@ int32_t fe2o3_scalar_gemm_v1(const float *a, uint64_t a_len, const float *b,
  * 2^31) and A and B are 16-byte aligned, with a partial last k stage when k
  * is not a multiple of 64: whole tiles when m and n are multiples of 256
  * and C is 16-byte aligned, edge tiles (masked stores at any alignment)
- * otherwise.  For other k or alignments, when m and n are at least 128, the
- * rows that cannot be read in place are first copied into aligned rows of
- * k rounded up to 8 (zeros past k) in stream-ordered scratch from the
- * library's pool and the tile runs on them (an operand that is only
- * misaligned gives the aligned operand's bits).  Outputs with too few tiles
- * to fill the device (at most 32 rows or columns, or about one round of
- * 64x32 blocks), whatever the alignment, and devices without a pool, take a
- * kernel that splits k over the waves of a workgroup and reads the operands
- * at their own alignment; k = 0 writes +0. */
+ * otherwise.  Outputs with too few tiles to fill the device (at most 32 rows
+ * or columns, or about one round of 64x32 blocks), whatever the alignment,
+ * take a kernel that splits k over the waves of a workgroup and reads the
+ * operands at their own alignment.  For other k or alignments the rows that
+ * cannot be read in place are first copied into aligned rows of k rounded up
+ * to 8 (zeros past k) in stream-ordered scratch from the library's pool and
+ * the tile runs on them; when m or n is below 128 and k short, and on devices
+ * without a pool, a kernel reads them where they are and sums in the tile's
+ * order.  An operand that is only misaligned gives the aligned operand's bits
+ * on every one of these ways.  k = 0 writes +0. */
 int32_t fe2o3_gemm_bf16_nt(const uint16_t *a, uint64_t a_len,
                            const uint16_t *b, uint64_t b_len, uint16_t *c,
                            uint64_t c_len, uint32_t m, uint32_t n, uint32_t k,
@@ -485,13 +486,13 @@ int32_t fe2o3_quantize_e4m3(const float *x, uint64_t x_len, const float *scale,
  * The pipelined fp8 MFMA tile runs whenever k is a multiple of 16
  * (k*256 < 2^31; a partial last stage when k is not a multiple of 128) and
  * A and B are 16-byte aligned (edge tiles for m or n not a multiple of 256
- * or an unaligned C).  For other k or alignments, when m and n are at least
- * 128, the rows that cannot be read in place are first copied into aligned
- * rows of k rounded up to 16 (E4M3 +0 past k) in stream-ordered scratch
- * from the library's pool and the tile runs on them; outputs with too few
- * tiles to fill the device, and devices without a pool, take the kernel that
- * splits k over a workgroup's waves (as fe2o3_gemm_bf16_nt).  k = 0 writes
- * +0.  The products of two E4M3 values are exact in fp32 on every path. */
+ * or an unaligned C).  The other ways are those of fe2o3_gemm_bf16_nt, with
+ * k rounded up to 16 (E4M3 +0 past k): few output tiles split k over a
+ * workgroup's waves; rows that cannot be read in place are copied for the
+ * tile, or summed in its order where they are.  A misaligned operand gives
+ * the aligned one's bits.  k = 0 writes +0 whatever the scales, which are not
+ * read then.  The products of two E4M3 values are exact in fp32 on every
+ * path. */
 int32_t fe2o3_gemm_fp8_nt(const uint8_t *a, uint64_t a_len, const uint8_t *b,
                           uint64_t b_len, const float *scale_a,
                           const float *scale_b, uint16_t *c, uint64_t c_len,

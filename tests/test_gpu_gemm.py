@@ -396,13 +396,23 @@ def test_gemm_bf16_nt_fast_path(gpu, oracle, m, n, k):
     _nt_case(gpu, oracle, m, n, k, seed=1)
 
 
+# the first three take the direct kernel on both sides, the next four the
+# repack and the tile, those with fewer than 128 rows or columns the repack
+# where K is long and else the in-order kernel against the tile: remainders in
+# rows, columns and K
 @pytest.mark.parametrize("m,n,k,which", [(512, 384, 1000, "a"), (512, 384, 1000, "b"),
-                                         (384, 640, 4096, "ab"), (4096, 4096, 4096, "a")])
+                                         (384, 640, 4096, "ab"), (4096, 4096, 4096, "a"),
+                                         (1600, 1500, 1000, "a"), (1600, 1500, 1000, "b"),
+                                         (1600, 1500, 1032, "ab"),
+                                         (100, 8192, 4096, "a"), (100, 8192, 4096, "b"),
+                                         (100, 8200, 1032, "ab"), (100, 8200, 1016, "ab"),
+                                         (120, 9000, 1024, "ab"), (16, 40000, 256, "ab"),
+                                         (40001, 33, 72, "ab"), (127, 9000, 8, "a")])
 def test_gemm_bf16_nt_misaligned_operands_match_aligned(gpu, m, n, k, which):
-    """A and/or B two bytes past a 16-byte boundary: their rows are copied
-    into aligned scratch and the pipelined tile runs on the copies, so C is
-    bit-identical to the aligned operands' (inputs unchanged, C's guards
-    intact)."""
+    """A and/or B two bytes past a 16-byte boundary: C is bit-identical to the
+    aligned operands' (inputs unchanged, C's guards intact), whether their
+    rows are copied into aligned scratch for the pipelined tile or read where
+    they are."""
     kern = _kernels()
     da, db = gpu.alloc(m * k, np.uint16), gpu.alloc(n * k, np.uint16)
     kern.fill_normal_bf16(da, 9, 0xA, 1.0 / np.sqrt(k))

@@ -605,12 +605,22 @@ def test_gemm_fp8_k_tail_matches_zero_padded_k(gpu, m, n, k, kp):
     assert_same(c.download(), cp.download(), f"K {k} vs zero-padded K {kp}")
 
 
+# the first three take the direct kernel on both sides, the next four the
+# repack and the tile, those with fewer than 128 rows or columns the repack
+# where K is long and else the in-order kernel against the tile: remainders in
+# rows, columns and K
 @pytest.mark.parametrize("m,n,k,which", [(512, 384, 1024, "a"), (384, 640, 4096, "b"),
-                                         (256, 256, 208, "ab")])
+                                         (256, 256, 208, "ab"),
+                                         (1600, 1500, 1008, "a"), (1600, 1500, 1008, "b"),
+                                         (1600, 1500, 1040, "ab"), (1024, 1024, 2048, "b"),
+                                         (100, 8192, 4096, "a"), (100, 8192, 4096, "b"),
+                                         (100, 8200, 2064, "ab"), (100, 8200, 2032, "ab"),
+                                         (120, 9000, 2048, "ab"), (16, 40000, 512, "ab"),
+                                         (40001, 33, 144, "ab"), (127, 9000, 16, "a")])
 def test_gemm_fp8_misaligned_operands_match_aligned(gpu, m, n, k, which):
-    """A and/or B one byte past a 16-byte boundary: their rows are copied
-    into aligned scratch and the pipelined tile runs on the copies, so C is
-    bit-identical to the aligned operands' (inputs unchanged)."""
+    """A and/or B one byte past a 16-byte boundary: C is bit-identical to the
+    aligned operands' (inputs unchanged), whether their rows are copied into
+    aligned scratch for the pipelined tile or read where they are."""
     kern = _k()
     rng = np.random.default_rng(m + k)
     a = rng.integers(0, 0x7F, m * k, dtype=np.uint8) | (rng.integers(0, 2, m * k, dtype=np.uint8) << 7)
