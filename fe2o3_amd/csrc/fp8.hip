@@ -507,7 +507,7 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   // zeros anyway, so an operand that is only misaligned gives the bits of
   // the aligned one.  Smaller outputs, and devices without stream-ordered
   // scratch, take the direct kernel, in K order where the tile could run the
-  // sizes (gemm_direct::tile_sizes).
+  // sizes or K is short (gemm_direct::in_order).
   const uint32_t kp = (k + 15u) & ~15u;
   const bool repack = !fast && gemm_direct::repack(m, n, k, 1u);
   void* scratch = nullptr;
@@ -521,7 +521,7 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   }
   if (!fast && scratch == nullptr) {
     if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
-    if (gemm_direct::tile_sizes(m, n, k, 1u))
+    if (gemm_direct::in_order(m, n, k, 1u))
       return launch_in_order(a, b, scale_a, scale_b, c, m, n, k, s);
     return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
   }

@@ -300,7 +300,7 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
   // puts zeros anyway, so an operand that is only misaligned gives the bits
   // of the aligned one.  Smaller outputs, and devices without stream-ordered
   // scratch, take the direct kernel, in K order where the tile could run the
-  // sizes (gemm_direct::tile_sizes).
+  // sizes or K is short (gemm_direct::in_order).
   const uint32_t kp = (k + 7u) & ~7u;
   if (fast || gemm_direct::repack(m, n, k, 2u)) {
     const int32_t lds_rc = set_fast_lds();  // before any launch: a failure leaves C untouched
@@ -331,6 +331,6 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
     (void)hipGetLastError();  // no stream-ordered scratch: the direct kernel
   }
   if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
-  if (gemm_direct::tile_sizes(m, n, k, 2u)) return launch_in_order(a, b, c, m, n, k, s);
+  if (gemm_direct::in_order(m, n, k, 2u)) return launch_in_order(a, b, c, m, n, k, s);
   return launch_direct(a, b, c, m, n, k, topo, s);
 }

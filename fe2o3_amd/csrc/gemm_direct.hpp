@@ -279,16 +279,31 @@ FE2O3_DEVICE void block(const uint8_t* __restrict__ a, const uint8_t* __restrict
   }
   if (kbytes % kUnit != 0u && units % kStride == first_unit) {  // the partial last unit
     const Off at = (Off)units * kUnit + 16u * pc;
-    auto row_of = [](const uint8_t* base, Off off) {
-      __builtin_amdgcn_sched_barrier(0);  // one piece at a time: registers, not latency
-      return base + off;
-    };
+    if (kbytes >= 16u) {
+      // a piece that the row's end cuts (or that lies past it) is read 16
+      // bytes before it and shifted down, zeros shifted in: every load at once
+      const Off from = min(at, kbytes - 16u);
+      const uint32_t past = (uint32_t)min(at - from, (Off)16u);
+      auto load_last = [&](const uint8_t* base, Off row) {
+        return load16(base + (row - 16u * pc) + from);
+      };
+      auto cut = [&](u32x4_t v) { return past < 16u ? shift_down(v, 8u * past) : u32x4_t{}; };
 #pragma unroll
-    for (int j = 0; j < 2 * NB; ++j)
-      bf[0][j] = load_end<T::kBytes>(row_of(b0, bo[j] - 16u * pc), at, kbytes);
+      for (int j = 0; j < 2 * NB; ++j) bf[0][j] = load_last(b0, bo[j]);
 #pragma unroll
-    for (int i = 0; i < 2 * MB; ++i)
-      af[0][i] = load_end<T::kBytes>(row_of(a0, ao[i] - 16u * pc), at, kbytes);
+      for (int i = 0; i < 2 * MB; ++i) af[0][i] = load_last(a0, ao[i]);
+#pragma unroll
+      for (int j = 0; j < 2 * NB; ++j) bf[0][j] = cut(bf[0][j]);
+#pragma unroll
+      for (int i = 0; i < 2 * MB; ++i) af[0][i] = cut(af[0][i]);
+    } else {  // rows shorter than a piece
+#pragma unroll
+      for (int j = 0; j < 2 * NB; ++j)
+        bf[0][j] = load_end<T::kBytes>(b0 + (bo[j] - 16u * pc), at, kbytes);
+#pragma unroll
+      for (int i = 0; i < 2 * MB; ++i)
+        af[0][i] = load_end<T::kBytes>(a0 + (ao[i] - 16u * pc), at, kbytes);
+    }
     mma(0);
   }
 
@@ -401,6 +416,7 @@ inline bool rows_ok(uint32_t m) { return ((uint64_t)m + 63u) / 64u <= 65535u; }
 //     fp8 38 | 59; bf16 127 x 9000 x 1024 29 | 31, fp8 29 | 17; bf16 16 x 40000
 //     x 256 25 | 10).
 constexpr uint32_t kRepackMin = 128;
+constexpr uint32_t kShortK = 2048;  // bytes, 16 units
 inline bool tile_sizes(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) {
   const uint64_t kbytes = (uint64_t)k * elem_bytes, padded = (kbytes + 15u) / 16u * 16u;
   return 256ull * padded < (1ull << 31) &&
@@ -409,7 +425,14 @@ inline bool tile_sizes(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) 
 inline bool repack(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) {
   return tile_sizes(m, n, k, elem_bytes) &&
          ((m >= kRepackMin && n >= kRepackMin) ||
-          ((uint64_t)k * elem_bytes > 2048u && rows_ok(m)));
+          ((uint64_t)k * elem_bytes > kShortK && rows_ok(m)));
+}
+// The in-order form also takes the short K of sizes that no tile runs: at most
+// two units a wave do not pay for the split's merge.  Split | in order, us:
+//   bf16 100000 x 5 x 65 21 | 7   40001 x 33 x 75 23 | 10   20000 x 100 x 401 33 | 24
+//   fp8 20000 x 100 x 1601 48 | 44   past the line: bf16 20000 x 100 x 1601 55 | 73
+inline bool in_order(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) {
+  return tile_sizes(m, n, k, elem_bytes) || (uint64_t)k * elem_bytes <= kShortK;
 }
 
 // 64 rows of K within 32-bit byte offsets, as the chosen forms need

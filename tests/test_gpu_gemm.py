@@ -464,6 +464,15 @@ def test_gemm_bf16_nt_direct_forms(gpu, oracle, m, n, k):
     assert_same(got.download()[1:], want.download(), "2-byte offsets vs aligned")
 
 
+# odd K on more output than the split takes, short enough for the in-order form
+# (16 units and less) and just past it: rows of less than a piece, of a piece
+# and a bit, of a unit and a bit
+@pytest.mark.parametrize("m,n,k", [(20000, 33, 7), (20000, 33, 9), (40001, 33, 75), (5, 100000, 65),
+                                   (20000, 100, 401), (20000, 100, 1023), (20000, 100, 1025)])
+def test_gemm_bf16_nt_short_odd_k(gpu, oracle, m, n, k):
+    _nt_case(gpu, oracle, m, n, k, seed=23, rows=sorted({0, m // 3, m - 2, m - 1}))
+
+
 def test_gemm_bf16_nt_direct_limits(gpu):
     """More workgroups than a grid's x dimension takes (2^32 threads, 512 a
     workgroup, 64 columns each): C = 1 * B exactly; and the shape error for

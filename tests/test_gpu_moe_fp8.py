@@ -564,6 +564,16 @@ def test_gemm_fp8_direct_forms_and_small_grids(gpu, oracle, m, n, k):
     assert_same(off.download()[1:], got, "offset operands vs aligned")
 
 
+@pytest.mark.parametrize("m,n,k", [(20000, 33, 15), (20000, 33, 17), (40001, 33, 75),
+                                   (5, 100000, 129), (20000, 100, 2047), (20000, 100, 2049)])
+def test_gemm_fp8_short_odd_k(gpu, oracle, m, n, k):
+    """As for bf16, 4000 outputs and the last row and column."""
+    rng = np.random.default_rng(m + n + k)
+    rows, cols = rng.integers(0, m, 4000), rng.integers(0, n, 4000)
+    rows[:200], cols[200:400] = m - 1, n - 1
+    assert _fp8_case(gpu, oracle, m, n, k, (rows, cols)) <= 1e-2
+
+
 # K a multiple of 16 but not of 128: the pipelined tiles with a partial last
 # stage (its chunks past K load zeros) on the 128x128 form (three and two
 # stages), the 256x256 tile and its tail round
