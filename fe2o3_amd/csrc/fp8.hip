@@ -267,40 +267,17 @@ __global__ void __launch_bounds__(gemm_direct::kThreads, WIDE ? 2 : 4) gemm_fp8_
     const float* __restrict__ scale_a, const float* __restrict__ scale_b,
     uint16_t* __restrict__ c, uint32_t m, uint32_t n, uint32_t k, uint32_t xcds) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  gemm_direct::run_form<gemm_direct::Fp8, WIDE>(form, a, b, c, m, n, k, scale_a[0] * scale_b[0],
-                                                xcds, smem);
+  const float scale = k == 0u ? 1.0f : scale_a[0] * scale_b[0];
+  gemm_direct::run_form<gemm_direct::Fp8, WIDE>(form, a, b, c, m, n, k, scale, xcds, smem);
 }
 
-__global__ void __launch_bounds__(gemm_direct::kThreads, 2) gemm_fp8_in_order_kernel(
-    const uint8_t* __restrict__ a, const uint8_t* __restrict__ b,
-    const float* __restrict__ scale_a, const float* __restrict__ scale_b,
-    uint16_t* __restrict__ c, uint32_t m, uint32_t n, uint32_t k) {
-  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  gemm_direct::in_order_block<gemm_direct::Fp8>(a, b, c, m, n, k, scale_a[0] * scale_b[0], smem);
-}
-
-int32_t launch_in_order(const uint8_t* a, const uint8_t* b, const float* sa, const float* sb,
-                        uint16_t* c, uint32_t m, uint32_t n, uint32_t k, hipStream_t s) {
-  static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
-      {(const void*)gemm_fp8_in_order_kernel}, gemm_direct::kLightSmem);
-  if (lds_rc != FE2O3_OK) return lds_rc;
-  const uint64_t blocks = gemm_direct::in_order_blocks(m, n);
-  if (blocks > 0x7fffffffu) return FE2O3_ERR_SHAPE;
-  const dim3 grid =
-      gemm_direct::list_grid((blocks + gemm_direct::kWaves - 1u) / gemm_direct::kWaves);
-  gemm_fp8_in_order_kernel<<<grid, gemm_direct::kThreads, gemm_direct::kLightSmem, s>>>(
-      a, b, sa, sb, c, m, n, k);
-  return fe2o3_host::after_launch();
-}
-
-int32_t launch_direct(const uint8_t* a, const uint8_t* b, const float* sa, const float* sb,
-                      uint16_t* c, uint32_t m, uint32_t n, uint32_t k,
-                      const tile_plan::Topology& topo, hipStream_t s) {
+int32_t launch_direct(const gemm_direct::Launch& l, const uint8_t* a, const uint8_t* b,
+                      const float* sa, const float* sb, uint16_t* c, uint32_t m, uint32_t n,
+                      uint32_t k, const tile_plan::Topology& topo, hipStream_t s) {
   static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
       {(const void*)gemm_fp8_direct_kernel<true>,
        (const void*)gemm_fp8_direct_kernel<false>}, gemm_direct::kWideSmem);
   if (lds_rc != FE2O3_OK) return lds_rc;
-  const gemm_direct::Launch l = gemm_direct::plan(m, n, k, 1u, topo.cus);
   if (l.grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
   const dim3 grid = gemm_direct::list_grid(l.grid);
   if (l.wide)
@@ -347,9 +324,7 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_128_kernel<3, edge, tail, k tail>", (const void*)gemm_fp8_128_kernel<3, false, true, true>, 256, kFp8SmallSmem<3>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel", (const void*)gemm_fp8_direct_kernel<false>, gemm_direct::kThreads, gemm_direct::kLightSmem}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "repack_bytes_kernel", (const void*)repack_bytes_kernel, 256, 0}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel<wide>", (const void*)gemm_fp8_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_in_order_kernel", (const void*)gemm_fp8_in_order_kernel, gemm_direct::kThreads, gemm_direct::kLightSmem}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "zero_fill_kernel", (const void*)gemm_core::zero_fill_kernel<uint16_t>, 256, 0})};
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_fp8_nt", "gemm_fp8_direct_kernel<wide>", (const void*)gemm_fp8_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem})};
 
 }  // namespace
 
@@ -484,13 +459,12 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   if (c_len == 0) return FE2O3_OK;
   if ((a_len && !a) || (b_len && !b) || !c || !scale_a || !scale_b) return FE2O3_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
-  if (k == 0) {  // the empty sum: +0 whatever the scales, which are not read
-    gemm_core::zero_fill_kernel<<<gemm_core::zero_fill_grid(c_len), 256, 0, s>>>(c, c_len);
-    return fe2o3_host::after_launch();
-  }
   tile_plan::Topology topo;
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
+  if (k == 0)  // +0 whatever the scales, which are not read
+    return launch_direct(gemm_direct::plan_fill(c_len), a, b, scale_a, scale_b, c, m, n, k, topo,
+                         s);
   // fast path: 16-byte operand rows (K a multiple of 16) and a 256-row fp8
   // panel (256 * k bytes) within its buffer resource's 32-bit range; K not a
   // multiple of 128 takes the edge tiles with a partial last stage
@@ -499,7 +473,8 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   // few output tiles: the direct kernel, whatever the operands' alignment
   if ((fast || gemm_direct::rows_ok(m)) && gemm_direct::k_fits(k, 1u) &&
       gemm_direct::prefer(m, n, k, 1u, topo.cus))
-    return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
+    return launch_direct(gemm_direct::plan(m, n, k, 1u, topo.cus), a, b, scale_a, scale_b, c, m,
+                         n, k, topo, s);
   // Rows the tile cannot read in place (K not a multiple of 16, or A or B
   // off a 16-byte boundary) are first copied into aligned rows of kp = K
   // rounded up to 16, zeros from K on, in stream-ordered scratch; the tile
@@ -521,9 +496,10 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   }
   if (!fast && scratch == nullptr) {
     if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
-    if (gemm_direct::in_order(m, n, k, 1u))
-      return launch_in_order(a, b, scale_a, scale_b, c, m, n, k, s);
-    return launch_direct(a, b, scale_a, scale_b, c, m, n, k, topo, s);
+    return launch_direct(gemm_direct::in_order(m, n, k, 1u)
+                             ? gemm_direct::plan_in_order<gemm_direct::Fp8>(m, n)
+                             : gemm_direct::plan(m, n, k, 1u, topo.cus),
+                         a, b, scale_a, scale_b, c, m, n, k, topo, s);
   }
   // every kernel's LDS limit is raised before anything is launched, so a
   // failure leaves C untouched

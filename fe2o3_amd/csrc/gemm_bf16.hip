@@ -31,15 +31,6 @@ __global__ void __launch_bounds__(gemm_direct::kThreads, WIDE ? 2 : 4) gemm_bf16
       1.0f, xcds, smem);
 }
 
-__global__ void __launch_bounds__(gemm_direct::kThreads, 4) gemm_bf16_nt_in_order_kernel(
-    const uint16_t* __restrict__ a, const uint16_t* __restrict__ b, uint16_t* __restrict__ c,
-    uint32_t m, uint32_t n, uint32_t k) {
-  extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-  gemm_direct::in_order_block<gemm_direct::Bf16>(reinterpret_cast<const uint8_t*>(a),
-                                                 reinterpret_cast<const uint8_t*>(b), c, m, n, k,
-                                                 1.0f, smem);
-}
-
 // ---- fast path ----------------------------------------------------------------------------
 // 256x256 tiles, 64 k per LDS stage (128-byte rows), two stages, 16x16x32
 // MFMAs in a fixed issue order (gemm_pipe.hpp).
@@ -147,9 +138,7 @@ const fe2o3_host::KernelRegistrar kRegistered[] = {
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_128_kernel<2, edge, tail, k tail>", (const void*)gemm_bf16_nt_128_kernel<2, false, true, true>, 256, kSmallSmem<2>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_128_kernel<3, edge, tail, k tail>", (const void*)gemm_bf16_nt_128_kernel<3, false, true, true>, 256, kSmallSmem<3>}),
     fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel", (const void*)gemm_bf16_nt_direct_kernel<false>, gemm_direct::kThreads, gemm_direct::kLightSmem}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel<wide>", (const void*)gemm_bf16_nt_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_in_order_kernel", (const void*)gemm_bf16_nt_in_order_kernel, gemm_direct::kThreads, gemm_direct::kLightSmem}),
-    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "zero_fill_kernel", (const void*)gemm_core::zero_fill_kernel<uint16_t>, 256, 0})};
+    fe2o3_host::KernelRegistrar({"fe2o3_gemm_bf16_nt", "gemm_bf16_nt_direct_kernel<wide>", (const void*)gemm_bf16_nt_direct_kernel<true>, gemm_direct::kThreads, gemm_direct::kWideSmem})};
 
 // Raises every fast-path kernel's dynamic-LDS limit once per process.
 int32_t set_fast_lds() {
@@ -234,13 +223,13 @@ int32_t launch_fast(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t 
 }  // namespace
 
 namespace {
-int32_t launch_direct(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m, uint32_t n,
-                      uint32_t k, const tile_plan::Topology& topo, hipStream_t s) {
+int32_t launch_direct(const gemm_direct::Launch& l, const uint16_t* a, const uint16_t* b,
+                      uint16_t* c, uint32_t m, uint32_t n, uint32_t k,
+                      const tile_plan::Topology& topo, hipStream_t s) {
   static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
       {(const void*)gemm_bf16_nt_direct_kernel<true>,
        (const void*)gemm_bf16_nt_direct_kernel<false>}, gemm_direct::kWideSmem);
   if (lds_rc != FE2O3_OK) return lds_rc;
-  const gemm_direct::Launch l = gemm_direct::plan(m, n, k, 2u, topo.cus);
   if (l.grid > 0x7fffffffu) return FE2O3_ERR_SHAPE;
   const dim3 grid = gemm_direct::list_grid(l.grid);
   if (l.wide)
@@ -249,20 +238,6 @@ int32_t launch_direct(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_
   else
     gemm_bf16_nt_direct_kernel<false><<<grid, gemm_direct::kThreads, l.smem, s>>>(
         l.form, a, b, c, m, n, k, topo.xcds);
-  return fe2o3_host::after_launch();
-}
-
-int32_t launch_in_order(const uint16_t* a, const uint16_t* b, uint16_t* c, uint32_t m, uint32_t n,
-                        uint32_t k, hipStream_t s) {
-  static const int32_t lds_rc = fe2o3_host::set_dynamic_lds(
-      {(const void*)gemm_bf16_nt_in_order_kernel}, gemm_direct::kLightSmem);
-  if (lds_rc != FE2O3_OK) return lds_rc;
-  const uint64_t blocks = gemm_direct::in_order_blocks(m, n);
-  if (blocks > 0x7fffffffu) return FE2O3_ERR_SHAPE;
-  const dim3 grid =
-      gemm_direct::list_grid((blocks + gemm_direct::kWaves - 1u) / gemm_direct::kWaves);
-  gemm_bf16_nt_in_order_kernel<<<grid, gemm_direct::kThreads, gemm_direct::kLightSmem, s>>>(
-      a, b, c, m, n, k);
   return fe2o3_host::after_launch();
 }
 }  // namespace
@@ -276,13 +251,10 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
   if (c_len == 0) return FE2O3_OK;
   if ((a_len && !a) || (b_len && !b) || !c) return FE2O3_ERR_NULL;
   hipStream_t s = (hipStream_t)stream;
-  if (k == 0) {
-    gemm_core::zero_fill_kernel<<<gemm_core::zero_fill_grid(c_len), 256, 0, s>>>(c, c_len);
-    return fe2o3_host::after_launch();
-  }
   tile_plan::Topology topo;
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
+  if (k == 0) return launch_direct(gemm_direct::plan_fill(c_len), a, b, c, m, n, k, topo, s);
   // fast path: 16-byte operand rows (K a multiple of 8), and a 256-row panel
   // (512 * k bytes) inside the 32-bit range of its buffer resource; whole
   // tiles with a 16-byte aligned C take the plain tile, any other M and N
@@ -292,7 +264,7 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
   // few output tiles: the direct kernel, whatever the operands' alignment
   if ((fast || gemm_direct::rows_ok(m)) && gemm_direct::k_fits(k, 2u) &&
       gemm_direct::prefer(m, n, k, 2u, topo.cus))
-    return launch_direct(a, b, c, m, n, k, topo, s);
+    return launch_direct(gemm_direct::plan(m, n, k, 2u, topo.cus), a, b, c, m, n, k, topo, s);
   // Rows the tile cannot read in place (K not a multiple of 8, or A or B two
   // bytes past a 16-byte boundary) are first copied into aligned rows of kp
   // = K rounded up to 8, zeros from K on, in stream-ordered scratch; the
@@ -331,6 +303,8 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
     (void)hipGetLastError();  // no stream-ordered scratch: the direct kernel
   }
   if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
-  if (gemm_direct::in_order(m, n, k, 2u)) return launch_in_order(a, b, c, m, n, k, s);
-  return launch_direct(a, b, c, m, n, k, topo, s);
+  return launch_direct(gemm_direct::in_order(m, n, k, 2u)
+                           ? gemm_direct::plan_in_order<gemm_direct::Bf16>(m, n)
+                           : gemm_direct::plan(m, n, k, 2u, topo.cus),
+                       a, b, c, m, n, k, topo, s);
 }

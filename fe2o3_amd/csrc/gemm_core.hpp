@@ -1,6 +1,6 @@
 // gemm_core.hpp -- what the 256x256 GEMM kernels (dense bf16, fp8, general)
 // share besides the pipelined tile itself (gemm_pipe.hpp): the tile order
-// and launch plan (tile_plan.hpp), the choice of epilogue and the empty sum.
+// and launch plan (tile_plan.hpp) and the choice of epilogue.
 #pragma once
 
 #include "common.hpp"
@@ -23,21 +23,6 @@ using tile_plan::xcd_tile_order;
 constexpr uint64_t kStagedOperandBytes = 192ull << 20;
 inline bool staged_epilogue(uint64_t operand_bytes) {
   return operand_bytes >= kStagedOperandBytes;
-}
-
-// K = 0: C is all +0 (an empty sum), whatever else the call scales it by.  A
-// grid-stride fill kernel rather than a memset node, so a caller may capture
-// the launch in a HIP graph.
-namespace {
-template <class T>
-__global__ void __launch_bounds__(256) zero_fill_kernel(T* __restrict__ c, uint64_t n) {
-  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) c[i] = 0;
-}
-}  // namespace
-inline dim3 zero_fill_grid(uint64_t n) {
-  const uint64_t blocks = (n + 255u) / 256u;
-  return dim3((unsigned)(blocks < 4096u ? blocks : 4096u));
 }
 
 }  // namespace gemm_core

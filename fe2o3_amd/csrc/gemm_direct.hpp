@@ -1,6 +1,6 @@
 // gemm_direct.hpp -- GEMMs with too few output tiles for the pipelined tile
 // (gemm_pipe.hpp) to fill the device: a decoding step's few activation rows,
-// small outputs, and operands at any alignment with any K above 0.
+// small outputs, and operands at any alignment with any K.
 //
 // C[m][n] = A[m][k] B[n][k]^T, both operands k-contiguous.  A workgroup of 8
 // waves owns an output block of 16 MB x 16 NB and splits K over its waves:
@@ -16,7 +16,7 @@
 // (bf16 16 x 4096 x 14336: 34.1 us against 24.7; 128 x 4096 x 4096: 23.9
 // against 13.6).
 //
-// The in-order form (in_order_block) gives every wave an output block of its
+// The in-order form gives every wave an output block of its
 // own and all of K instead: C's bits are then those of the pipelined tile, for
 // the calls that would take the tile if their operands could be read in place
 // or copied.
@@ -54,6 +54,7 @@ struct Bf16 {
   static constexpr uint32_t kBytes = 2;  // per element
   static constexpr bool kScaled = false;
   static constexpr int kDeep = 3;  // units in flight of the widest forms
+  static constexpr bool kOrderedWide = false;  // the in-order form is in the light kernel
   static FE2O3_DEVICE uint32_t tile_piece(uint32_t g, uint32_t h) { return 4u * h + g; }
   static FE2O3_DEVICE void mma(const Frag& b, const Frag& a, f32x4_t& acc) {
 #pragma unroll
@@ -71,6 +72,7 @@ struct Fp8 {
   static constexpr uint32_t kBytes = 1;
   static constexpr bool kScaled = true;
   static constexpr int kDeep = 2;
+  static constexpr bool kOrderedWide = true;  // the light one has no registers for it
   static FE2O3_DEVICE uint32_t tile_piece(uint32_t g, uint32_t h) { return 2u * g + h; }
   static FE2O3_DEVICE void mma(const Frag& b, const Frag& a, f32x4_t& acc) {
     acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
@@ -441,6 +443,8 @@ inline bool k_fits(uint32_t k, uint32_t elem_bytes) { return 64ull * k * elem_by
 constexpr uint32_t smem_of(uint32_t mb, uint32_t nb) {
   return kWaves * 1024u * (mb * nb > 2u * (mb + nb) ? mb * nb : 2u * (mb + nb));
 }
+// Launches of the light kernel or the wide one.
+constexpr int kAnyK = kNumForms, kInOrder = kNumForms + 1, kFill = kNumForms + 2;
 struct Launch {
   int form;
   bool wide;
@@ -448,23 +452,45 @@ struct Launch {
   uint32_t smem;
 };
 inline Launch plan(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes, uint32_t cus) {
-  const int form = k_fits(k, elem_bytes) ? choose(m, n, cus) : kNumForms;
+  const int form = k_fits(k, elem_bytes) ? choose(m, n, cus) : kAnyK;
   const Form f = form < kNumForms ? kForms[form] : Form{1, 4, true};
   return {form, f.wide, grid_of(f, m, n), smem_of(f.mb, f.nb)};
 }
-
-// the in-order form's blocks, one per wave
-inline uint64_t in_order_blocks(uint32_t m, uint32_t n) {
-  return grid_of(Form{2, 2, false}, m, n);
+// 2 x 2 blocks, one per wave; their ids are 32-bit, so more of them stay a grid
+// that the launch refuses
+template <class T>
+inline Launch plan_in_order(uint32_t m, uint32_t n) {
+  const uint64_t blocks = grid_of(Form{2, 2, false}, m, n);
+  return {kInOrder, T::kOrderedWide, blocks > 0x7fffffffu ? blocks : (blocks + kWaves - 1u) / kWaves,
+          smem_of(2, 2)};
+}
+// K = 0: C is all +0 (an empty sum, whatever the scales).  A grid-stride fill
+// rather than a memset node, so a caller may capture it, and rather than the
+// blocks' walk over nothing (8192 x 8192: 235 us).
+inline Launch plan_fill(uint64_t c_len) {
+  const uint64_t groups = (c_len / 8u + kThreads - 1u) / kThreads;
+  return {kFill, true, groups < 2048u ? (groups ? groups : 1u) : 2048u, 0u};
 }
 
 constexpr int kLightSmem = (int)smem_of(2, 2), kWideSmem = (int)smem_of(4, 2);
 
-// The block on form `form` (an index of kForms; kNumForms: any K).
+FE2O3_DEVICE void fill(uint16_t* __restrict__ c, uint64_t n) {
+  const uint64_t stride = (uint64_t)gridDim.x * kThreads;
+  const uint64_t t = (uint64_t)blockIdx.x * kThreads + threadIdx.x, pieces = n / 8u;
+  for (uint64_t i = t; i < pieces; i += stride)
+    *reinterpret_cast<u32x4_any_t*>(c + 8u * i) = u32x4_t{0, 0, 0, 0};
+  if (t < n % 8u) c[8u * pieces + t] = 0;
+}
+
+// A launch's workgroup on form `form` (an index of kForms, or one of the forms
+// past it).
 template <class T, bool WIDE>
 FE2O3_DEVICE void run_form(int form, const uint8_t* a, const uint8_t* b, uint16_t* c, uint32_t m,
                            uint32_t n, uint32_t k, float scale, uint32_t xcds, uint8_t* smem) {
 #define FE2O3_DIRECT(MB, NB, D) return block<T, MB, NB, D>(a, b, c, m, n, k, scale, xcds, smem)
+  if constexpr (WIDE == T::kOrderedWide)
+    if (form == kInOrder)
+      return block<T, 2, 2, 2, uint32_t, true>(a, b, c, m, n, k, scale, xcds, smem);
   if constexpr (!WIDE) {
     switch (form) {
       case 0: FE2O3_DIRECT(1, 1, 4);
@@ -478,16 +504,11 @@ FE2O3_DEVICE void run_form(int form, const uint8_t* a, const uint8_t* b, uint16_
       case 5: FE2O3_DIRECT(4, 1, 3);
       case 6: FE2O3_DIRECT(2, 4, T::kDeep);
       case 7: FE2O3_DIRECT(4, 2, T::kDeep);
+      case kFill: return fill(c, (uint64_t)m * n);
       default: return block<T, 1, 4, 1, uint64_t>(a, b, c, m, n, k, scale, xcds, smem);
     }
   }
 #undef FE2O3_DIRECT
-}
-
-template <class T>
-FE2O3_DEVICE void in_order_block(const uint8_t* a, const uint8_t* b, uint16_t* c, uint32_t m,
-                                 uint32_t n, uint32_t k, float scale, uint8_t* smem) {
-  block<T, 2, 2, 2, uint32_t, true>(a, b, c, m, n, k, scale, 1u, smem);
 }
 
 }  // namespace gemm_direct
