@@ -390,17 +390,46 @@ inline int choose(uint32_t m, uint32_t n, uint32_t cus, uint64_t* cost = nullptr
 //   bf16 64 x 4096 x 4096   24.3 |  9.6     fp8 64 x 8192 x 8192  24.7 | 16.4
 //   bf16 128 x 4096 x 4096  22.5 | 13.6     fp8 128 x 4096 x 8192 22.8 | 13.7
 //   bf16 128 x 8192 x 4096  23.5 | 25.4     fp8 128 x 8192 x 2048  8.7 | 10.1
-// (the last line costs 12).  At most 32 rows or columns are the weights'
-// stream whatever the cost (32 x 28672 x 4096: 55.1 | 48.7; a K below eight
-// units leaves waves idle).  Where the tile needs its operands repacked
-// first, the lines cross between 18 and 24 (256 x 4096 x 4097: 58.1 | 36.2,
-// 320: 58.0 | 52.9, 512 x 4096 x 4090: 42.7 | 77.4).  The rule looks at sizes
-// only, so that a misaligned operand gives the aligned one's bits.
+// (the last line costs 12).  Where the tile needs its operands repacked first,
+// the lines cross between 18 and 24 (256 x 4096 x 4097: 58.1 | 36.2, 320: 58.0 |
+// 52.9, 512 x 4096 x 4090: 42.7 | 77.4).  At most 32 rows or columns (of K from
+// eight units on, one a wave) stream the other operand, and stream_prefer
+// decides.  The rules look at sizes only, so that a misaligned operand gives
+// the aligned one's bits.
+//
+// stream_prefer: `rows` of the streamed operand, the other's at most 32; tall:
+// it is A, and C has few columns.  Up to a round of tiles the line lies at the
+// cost again, and past it once the tiles fill most CUs and no longer stream
+// faster for being more.  Beyond a round the direct kernel's smaller blocks
+// spread better, unless K is so short that its merge shows more than the
+// tile's stores (of a tall C they cost most).  Tile against direct, us, the
+// streamed operand from HBM and (in brackets) from the last-level cache, which
+// a program that streams its weights does not see:
+//   bf16 16 x 14336 x 4096  36.5 | 24.5 (23.3 | 19.5)   cost 5, 112 tiles
+//   bf16 16 x 20000 x 512    8.3 |  7.1  (6.1 |  4.7)   cost 9, 157 tiles
+//   bf16 16 x 20000 x 4096  40.8 | 37.8 (26.6 | 34.3)
+//   bf16 32 x 20000 x 4096  42.3 | 44.8 (28.5 | 34.1)   cost 12
+//   bf16 16 x 28672 x 1024  13.5 | 15.0 (12.1 | 12.9)   cost 10, 224 tiles
+//   bf16 16 x 28672 x 4096  46.5 | 43.9 (34.5 | 36.9)
+//   bf16 32 x 28672 x 1024  13.3 | 16.4 (11.9 | 13.8)   cost 12
+//   bf16 32 x 28672 x 4096  53.3 | 48.9 (36.3 | 38.6)
+//   bf16 16 x 40000 x 512   15.9 | 13.3 (13.6 | 10.0)   cost 15, 313 tiles
+//   bf16 16 x 65536 x 1024  30.1 | 31.8 (26.9 | 26.5)   cost 20, 512 tiles
+//   bf16 65536 x 16 x 1024  38.5 | 31.5 (34.7 | 25.8)
+//   bf16 16 x 65536 x 4096 131.2 | 97.8                 fp8 69.8 | 58.9 (47.2 | 44.2)
+inline bool stream_prefer(uint32_t rows, bool tall, uint64_t kbytes, uint64_t cost,
+                          uint32_t cus) {
+  const uint64_t tiles = ((uint64_t)rows + 127u) / 128u;
+  if (tiles > cus) return tall || kbytes >= 4096u || 2u * tiles <= 3ull * cus;
+  if (kbytes < 4096u) return cost <= (tall ? 10u : 9u);
+  return cost <= 10u || 4u * tiles >= 3ull * cus;
+}
 inline bool prefer(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes, uint32_t cus) {
   const uint64_t kbytes = (uint64_t)k * elem_bytes;
-  if ((m <= 32u || n <= 32u) && kbytes >= kWaves * kUnit) return true;
   uint64_t cost = 0;
   choose(m, n, cus, &cost);
+  if ((m <= 32u || n <= 32u) && kbytes >= kWaves * kUnit)
+    return kbytes % 16u != 0u || stream_prefer(m > n ? m : n, m > n, kbytes, cost, cus);
   return cost <= (kbytes % 16u == 0u ? 10u : 18u);
 }
 // Operands that the pipelined tiles cannot read in place are taken up to 65535

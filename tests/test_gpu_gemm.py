@@ -407,6 +407,7 @@ def test_gemm_bf16_nt_fast_path(gpu, oracle, m, n, k):
                                          (100, 8192, 4096, "a"), (100, 8192, 4096, "b"),
                                          (100, 8200, 1032, "ab"), (100, 8200, 1016, "ab"),
                                          (120, 9000, 1024, "ab"), (16, 40000, 256, "ab"),
+                                         (32, 20000, 1024, "ab"), (20000, 32, 2048, "a"),
                                          (40001, 33, 72, "ab"), (127, 9000, 8, "a")])
 def test_gemm_bf16_nt_misaligned_operands_match_aligned(gpu, m, n, k, which):
     """A and/or B two bytes past a 16-byte boundary: C is bit-identical to the
@@ -501,9 +502,11 @@ def test_gemm_bf16_nt_direct_limits(gpu):
                                    (1024, 1024, 320), (1024, 1024, 8), (1024, 1024, 72),
                                    (1000, 1032, 1000), (1600, 1500, 77), (1600, 1500, 1003),
                                    # a last column that cuts an 8-column store, on both tiles
-                                   (1001, 1035, 200), (2500, 4099, 136)])
+                                   (1001, 1035, 200), (2500, 4099, 136),
+                                   # at most 32 rows or columns past stream_prefer's lines
+                                   (32, 20000, 520), (16, 65536, 512), (20001, 32, 1024)])
 def test_gemm_bf16_nt_small_grid_tiles(gpu, oracle, m, n, k):
-    _nt_case(gpu, oracle, m, n, k, seed=22, rows=[0, 63, 127, 128, 511, 895, 897, m - 2, m - 1])
+    _nt_case(gpu, oracle, m, n, k, seed=22, rows=sorted(r for r in {0, 63, 127, 128, 511, 895, 897, m - 2, m - 1} if r < m))
 
 
 # M or N not a multiple of 256 with whole 64-k stages: edge tiles of the
