@@ -222,7 +222,11 @@ FE2O3_DEVICE void flash_block(const uint16_t* __restrict__ q, const uint16_t* __
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
-  float m_ref = -INFINITY;  // exp reference, log2 domain (>= running max - slack)
+  // exp reference, log2 domain (>= running max - slack).  From the lowest finite
+  // value on: a tile of scores of -inf alone (keys that the caller shut out) has
+  // exponentials of 0 against it, where against -inf they would be NaN; the
+  // first tile with a finite score raises it.
+  float m_ref = -__FLT_MAX__;
   float l_run = 0.0f;       // this lane's partial row sum of exp2(s*c - m_ref)
 
   const uint32_t kv_tiles = (seq + BKV - 1u) / BKV;
@@ -324,8 +328,8 @@ FE2O3_DEVICE void flash_block(const uint16_t* __restrict__ q, const uint16_t* __
       };
       probabilities();
       // The reference is raised only when some lane's sum of this tile is not
-      // <= 2^slack: every p is at most that sum, and the first tile (reference
-      // -inf) gives +inf or NaN.  Then the row's tile max, the rescale, and
+      // <= 2^slack: every p is at most that sum, and against the first reference
+      // a finite score gives +inf.  Then the row's tile max, the rescale, and
       // this tile's probabilities again.
       if (__any(!(psum <= kLazyBound))) {
         float mloc = -INFINITY;
@@ -504,10 +508,7 @@ FE2O3_DEVICE void flash_split_block(const uint16_t* __restrict__ q, const uint16
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = 0.0f;
-  // As in flash_block, but from the lowest finite value on: a group's own first
-  // tile may hold only scores of -inf (keys that the caller shut out), whose
-  // exponentials against -inf would be NaN and against this are 0.
-  float m_ref = -__FLT_MAX__, l_run = 0.0f;
+  float m_ref = -__FLT_MAX__, l_run = 0.0f;  // as in flash_block
 
   const uint32_t kv_tiles = (seq + SK - 1u) / SK;
   const uint32_t n_kv = CAUSAL ? min((qt + 1u) * (uint32_t)(S_ROWS / SK), kv_tiles) : kv_tiles;

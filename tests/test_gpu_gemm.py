@@ -506,7 +506,8 @@ def test_gemm_bf16_nt_direct_limits(gpu):
                                    # at most 32 rows or columns past stream_prefer's lines
                                    (32, 20000, 520), (16, 65536, 512), (20001, 32, 1024)])
 def test_gemm_bf16_nt_small_grid_tiles(gpu, oracle, m, n, k):
-    _nt_case(gpu, oracle, m, n, k, seed=22, rows=sorted(r for r in {0, 63, 127, 128, 511, 895, 897, m - 2, m - 1} if r < m))
+    rows = sorted(r for r in {0, 63, 127, 128, 511, 895, 897, m - 2, m - 1} if r < m)
+    _nt_case(gpu, oracle, m, n, k, seed=22, rows=rows)
 
 
 # M or N not a multiple of 256 with whole 64-k stages: edge tiles of the

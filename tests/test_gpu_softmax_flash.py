@@ -442,6 +442,34 @@ def test_flash_split_keys_shut_out_tile(gpu, oracle, s, causal, first):
     assert rel_err(lse, ref_lse) <= 1e-5  # fp32 output: the 1e-5 bar
 
 
+@pytest.mark.parametrize("rep", [1, 320])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("s", [200, 256])
+def test_flash_shut_out_first_tile_any_heads(gpu, oracle, s, causal, rep):
+    """The first 64 keys' scores are all -inf, for two heads (the kernel that
+    splits the keys) and the same two repeated over 640 (whole and partial
+    tiles of the others): rows with keys of their own match the f64 oracle
+    however many heads the call has; rows that see only shut-out keys are NaN
+    with an LSE of -inf."""
+    rng = np.random.default_rng(s)
+    q, k, v = (rng.standard_normal((2, s, 128)).astype(np.float32) for _ in range(3))
+    q[:, :, 0] = 1.0
+    k[:, :64, 0] = -np.inf
+    one = [oracle.bf16_from_f32(np.ascontiguousarray(x).ravel()) for x in (q, k, v)]
+    _, out, lse, scale = _flash(gpu, 1, 2 * rep, s, causal, seed=0,
+                                qkv=[np.tile(x, rep) for x in one])
+    first = 64 if causal else 0
+    rows = np.tile(np.arange(first, s, dtype=np.uint32), 2)
+    bh = np.repeat(np.arange(2, dtype=np.uint32), s - first)
+    rc, ref, ref_lse = oracle.flash_attention_rows_bf16(*one, s, 128, causal, scale, bh, rows)
+    assert rc == 0 and np.all(np.isfinite(ref))
+    out, lse = out.reshape(rep, 2, s, 128), lse.reshape(rep, 2, s)
+    for r in range(rep):
+        assert rel_err(out[r, :, first:].reshape(-1, 128), ref) <= 1e-2
+        assert rel_err(lse[r, :, first:].ravel(), ref_lse) <= 1e-5  # fp32 output: the 1e-5 bar
+    assert np.all(np.isnan(out[:, :, :first])) and np.all(lse[:, :, :first] == -np.inf)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("pattern", ["normal", "ramp", "jump"])
 @pytest.mark.parametrize("s", [37, 64, 200, 256, 300, 512, 640])
