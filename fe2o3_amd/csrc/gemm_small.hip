@@ -258,8 +258,8 @@ constexpr int kGpSmem = kGpStages * 2 * gemm_pipe::Geo<kGpRowBytes>::kTileBytes;
 // 16-row block: every C load of the lane first (one wait), then the products
 // and stores.  A lane's 4 columns move as one access of 16 bytes at C's own
 // 4-byte alignment (gfx950 global accesses of four dwords need no more).  In
-// a tile that the last column cuts, the group it cuts (and those past it)
-// moves element by element, loads clamped to that column.
+// a tile that the last column cuts, the group it cuts moves element by
+// element, loads clamped to that column.
 typedef float f32x4_any_t __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int TN, int RPW, int CPW, class Acc>
@@ -298,7 +298,7 @@ FE2O3_DEVICE void general_epilogue(const Acc& acc, float* c_tile, uint32_t rows,
         if (col + 4u <= cols) {
           *reinterpret_cast<f32x4_any_t*>(out + col) =
               combined(i, j, *reinterpret_cast<const f32x4_any_t*>(out + col));
-        } else {
+        } else if (col < cols) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) cv[j][e] = out[min(col + e, cols - 1u)];
           const f32x4_t y = combined(i, j, cv[j]);
@@ -470,9 +470,12 @@ FE2O3_DEVICE void general_tile(const uint16_t* __restrict__ a, const uint16_t* _
     for (int j = 0; j < 2; ++j) acc.v[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   constexpr int D = MODE == Cols::narrow ? 2 : kGsDepth;
   u32x4_t ra[D][2], rb[D][2];
-  uint32_t loaded = 0;  // the next step to load; the last one is loaded again past it
+  // the next step to load; the last one is loaded again past it (unless the
+  // loads of B's short rows cost more than the branch)
+  uint32_t loaded = 0;
   auto load = [&](int s) {
     __builtin_amdgcn_sched_barrier(0);
+    if (MODE == Cols::narrow && loaded >= steps) return;
     const bool more = loaded + 1u < steps;
     ++loaded;
 #pragma unroll
@@ -540,7 +543,7 @@ FE2O3_DEVICE void general_tile(const uint16_t* __restrict__ a, const uint16_t* _
 #pragma unroll
       for (int s = 0; s < D; ++s) {
         if (t0 + s >= steps) break;
-        put_set((s + 1) & 1, (s + 1) % D);
+        if (MODE != Cols::narrow || t0 + s + 1u < steps) put_set((s + 1) & 1, (s + 1) % D);
         load(s);
         compute(s & 1);
         lds_barrier();
