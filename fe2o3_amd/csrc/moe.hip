@@ -458,17 +458,17 @@ __global__ void __launch_bounds__(256) gather_kernel(const uint16_t* __restrict_
 }
 
 // This workgroup's entry of the expert tile list (moe_tiles.hpp), computed
-// by each wave as expert_tile_lanes spells out: lane l loads expert
-// e_begin + l's row bounds (one memory round trip for all experts, where the
-// serial walk took two dependent scalar loads per expert, ~8% of a gate/up
-// tile), a wave scan sums the tile counts, a ballot finds the entry's
-// expert, and lane reads return its bounds as wave-uniform values.
-FE2O3_DEVICE bool expert_tile(const uint32_t* offsets, uint32_t e_begin, uint32_t e_end,
-                              uint32_t routes, uint32_t n_blocks, uint32_t xcds, uint32_t* e_out,
-                              uint32_t* row0, uint32_t* rows, uint32_t* nb) {
+// by each wave as expert_tile_lanes spells out for all experts: lane l loads
+// expert l's row bounds (one memory round trip, where the serial walk took two
+// dependent scalar loads per expert, ~8% of a gate/up tile), a wave scan sums
+// the tile counts, a ballot finds the entry's expert, and lane reads return its
+// bounds as wave-uniform values.
+FE2O3_DEVICE bool expert_tile(const uint32_t* offsets, uint32_t experts, uint32_t routes,
+                              uint32_t n_blocks, uint32_t xcds, uint32_t* e_out, uint32_t* row0,
+                              uint32_t* rows, uint32_t* nb) {
   const uint32_t l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   uint32_t lo = 0, n = 0;
-  if (l < e_end - e_begin) expert_rows(offsets, e_begin + l, routes, &lo, &n);
+  if (l < experts) expert_rows(offsets, l, routes, &lo, &n);
   uint32_t incl = expert_m_tiles(n) * n_blocks;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -487,7 +487,7 @@ FE2O3_DEVICE bool expert_tile(const uint32_t* offsets, uint32_t e_begin, uint32_
   const uint32_t incl_e = (uint32_t)__builtin_amdgcn_readlane((int)incl, le);
   const uint32_t m_tiles = expert_m_tiles(n_e);
   const uint32_t xi = x - (incl_e - m_tiles * n_blocks);
-  *e_out = e_begin + (uint32_t)le;
+  *e_out = (uint32_t)le;
   *nb = xi / m_tiles;
   m_tile(lo_e, n_e, m_tiles, xi % m_tiles, row0, rows);
   return true;
@@ -649,12 +649,11 @@ template <bool TOKENS>
 __global__ void __launch_bounds__(256, 1) gate_up_kernel(
     const uint16_t* __restrict__ xa, uint32_t x_bytes, const uint32_t* __restrict__ permutation,
     const uint16_t* __restrict__ wg, const uint16_t* __restrict__ wu,
-    const uint32_t* __restrict__ offsets, uint32_t e_begin, uint32_t e_end, uint32_t hidden,
-    uint32_t ffn, uint32_t routes, uint16_t* __restrict__ hc, uint32_t xcds) {
+    const uint32_t* __restrict__ offsets, uint32_t experts, uint32_t hidden, uint32_t ffn,
+    uint32_t routes, uint16_t* __restrict__ hc, uint32_t xcds) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   uint32_t e, row0, rows, nb;
-  if (!expert_tile(offsets, e_begin, e_end, routes, ffn / 128u, xcds, &e, &row0, &rows, &nb))
-    return;
+  if (!expert_tile(offsets, experts, routes, ffn / 128u, xcds, &e, &row0, &rows, &nb)) return;
   by_tile_rows(rows, [&](auto rpw) {
     constexpr int R = decltype(rpw)::value;
     if constexpr (R == 0)
@@ -699,14 +698,14 @@ FE2O3_DEVICE void down_tile(const uint16_t* __restrict__ hc, const uint16_t* __r
 __global__ void __launch_bounds__(256, 1) down_kernel(const uint16_t* __restrict__ hc,
                                                       const uint16_t* __restrict__ wd,
                                                       const uint32_t* __restrict__ offsets,
-                                                      uint32_t e_begin, uint32_t e_end,
-                                                      uint32_t hidden, uint32_t ffn,
+                                                      uint32_t experts, uint32_t hidden,
+                                                      uint32_t ffn,
                                                       uint64_t routes, uint32_t kparts,
                                                       float* __restrict__ yc, uint32_t xcds) {
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
   uint32_t e, row0, rows, nb;
-  if (!expert_tile(offsets, e_begin, e_end, (uint32_t)routes, kparts * (hidden / 256u), xcds, &e,
-                   &row0, &rows, &nb))
+  if (!expert_tile(offsets, experts, (uint32_t)routes, kparts * (hidden / 256u), xcds, &e, &row0,
+                   &rows, &nb))
     return;
   by_tile_rows(rows, [&](auto rpw) {
     constexpr int R = decltype(rpw)::value;
@@ -804,16 +803,14 @@ int32_t route(const void* logits, uint64_t logits_len, uint32_t dtype, uint32_t*
                                                             experts, capacity, status);
     return fe2o3_host::after_launch();
   }
-  {
-    const unsigned blocks = (tokens + 255u) / 256u;
-    if (dtype == 0)
-      route_select_kernel<float><<<blocks, 256, 0, s>>>((const float*)logits, tokens, experts,
-                                                        top2, weights, status);
-    else
-      route_select_kernel<uint16_t><<<blocks, 256, 0, s>>>((const uint16_t*)logits, tokens,
-                                                           experts, top2, weights, status);
-  }
-  const unsigned assign_blocks = routes ? (unsigned)((routes + RA_ROUTES - 1) / RA_ROUTES) : 1u;
+  const unsigned blocks = (tokens + 255u) / 256u;
+  if (dtype == 0)
+    route_select_kernel<float><<<blocks, 256, 0, s>>>((const float*)logits, tokens, experts, top2,
+                                                      weights, status);
+  else
+    route_select_kernel<uint16_t><<<blocks, 256, 0, s>>>((const uint16_t*)logits, tokens, experts,
+                                                         top2, weights, status);
+  const unsigned assign_blocks = (unsigned)((routes + RA_ROUTES - 1) / RA_ROUTES);
   // Many routes: the count / scan / assign kernels, on stream-ordered
   // scratch of (experts + 1) words per workgroup and the totals.  Without
   // scratch on this device, the single kernel.
@@ -1277,7 +1274,11 @@ uint32_t down_k_parts(uint64_t routes, uint32_t experts, uint32_t hidden, uint32
 // cost more in the events that join them -- the combine started 10 us after
 // the last down tile -- than the rounds gave: 8 experts, hidden 4096, ffn
 // 14336, 535 us against 511 at 32 tokens, 692 against 665 at 512, 1195 against
-// 1172 at 2048, 2168 against 2157 at 4096.)
+// 1172 at 2048, 2168 against 2157 at 4096.  Over 728 layers of 2 to 64 experts
+// and 1 to 8192 tokens one stream took 0.76 of the time.  Where it took more:
+// two experts of 4096 rows and up, 1777 against 1934 at 4096 tokens of 4096 x
+// 14336; 16 experts of 256 rows when the routing gives one of them a second
+// tile and so a second round, 193 against 212 at 2048 tokens of 2048 x 2048.)
 int32_t ffn_top2(const uint16_t* x, uint64_t x_len, const uint16_t* w_gate, uint64_t w_gate_len,
                  const uint16_t* w_up, uint64_t w_up_len, const uint16_t* w_down,
                  uint64_t w_down_len, uint64_t top2_len, const uint32_t* expert_offsets,
@@ -1337,13 +1338,13 @@ int32_t ffn_top2(const uint16_t* x, uint64_t x_len, const uint16_t* w_gate, uint
                                                   (uint32_t)routes, ws.xc);
   if (tokens_direct)
     gate_up_kernel<true><<<(unsigned)gu, 256, kSmem, s>>>(
-        x, (uint32_t)x_bytes, permutation, w_gate, w_up, expert_offsets, 0u, experts, hidden, ffn,
+        x, (uint32_t)x_bytes, permutation, w_gate, w_up, expert_offsets, experts, hidden, ffn,
         (uint32_t)routes, ws.hc, xcds);
   else
     gate_up_kernel<false><<<(unsigned)gu, 256, kSmem, s>>>(
-        ws.xc, 0u, permutation, w_gate, w_up, expert_offsets, 0u, experts, hidden, ffn,
+        ws.xc, 0u, permutation, w_gate, w_up, expert_offsets, experts, hidden, ffn,
         (uint32_t)routes, ws.hc, xcds);
-  down_kernel<<<(unsigned)dn, 256, kSmem, s>>>(ws.hc, w_down, expert_offsets, 0u, experts, hidden,
+  down_kernel<<<(unsigned)dn, 256, kSmem, s>>>(ws.hc, w_down, expert_offsets, experts, hidden,
                                               ffn, routes, kparts, ws.yc, xcds);
   const uint64_t threads = (uint64_t)tokens * (hidden / 4u);
   combine_kernel<<<(unsigned)((threads + 255u) / 256u), 256, 0, s>>>(ws.yc, inverse, route_weights,
