@@ -420,11 +420,8 @@ int32_t fe2o3_amax_f32(const float* x, uint64_t x_len, float* amax, void* stream
   const int32_t topo_rc = fe2o3_host::device_topology(&topo);
   if (topo_rc != FE2O3_OK) return topo_rc;
   zero_f32_kernel<<<1, 1, 0, s>>>(amax);
-  // one workgroup per 4096 elements, at most one per CU (two from 256 MiB on,
-  // where the stream is worth more than the atomics: a linear of 8192^3 took
-  // 490 us before and 488 with them)
-  const unsigned most = topo.cus * (x_len >= (1u << 26) ? 2u : 1u);
-  if (x_len) amax_kernel<<<grid_for(x_len, 4096, most), kAmaxThreads, 0, s>>>(x, x_len, amax);
+  // one workgroup per 4096 elements, at most one per CU
+  if (x_len) amax_kernel<<<grid_for(x_len, 4096, topo.cus), kAmaxThreads, 0, s>>>(x, x_len, amax);
   return fe2o3_host::after_launch();
 }
 
