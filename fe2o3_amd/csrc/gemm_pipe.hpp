@@ -89,7 +89,7 @@ struct Geo {
 // load past the operand's k goes through this mask.  For a [k][n] operand a
 // chunk is one k row (cbytes = 2 * its row within the stage).  Dense rows
 // have k_end a multiple of 16 bytes, so no chunk straddles it.  The zeros'
-// products are zero, the zero padding the staged kernels give a partial k
+// products are zero, the zero padding the register tiles give a partial k
 // step.
 constexpr uint32_t kOutOfRange = 0x80000000u;  // past any extent (extents are < 2^31)
 

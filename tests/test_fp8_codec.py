@@ -1,7 +1,7 @@
 """CPU check (no GPU): the product's fp8 E4M3FN encoder
 (fe2o3_amd/csrc/fp8_codec.hpp, the function the quantize kernel runs) equals
 the oracle's OCP closed form (oracle/fp8.c) on every one of the 2^32 binary32
-bit patterns, and the decoder the generic fp8 GEMM stages operands with
+bit patterns, and its exact widening to bf16
 (bf16_bits_from_e4m3) equals the oracle's decode table on all 256 codes.
 Built with g++ against oracle/liboracle.so."""
 import os

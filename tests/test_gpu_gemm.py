@@ -117,6 +117,16 @@ def test_general_hardware_matrix_bit_exact(gpu, oracle, case, schedule):
     ((65, 63, 97), (101, 64, 70), 0.75, -0.5),
     ((128, 256, 320), (320, 256, 256), 1.0, 1.0),
     ((200, 130, 77), (77, 131, 140), -2.0, 0.125),
+    # in place on the pipelined tiles, and repacked for them, whole and partial
+    # last stages
+    ((1300, 1304, 1600), (1600, 1304, 1310), 1.5, -0.25),
+    ((1400, 1200, 1816), (1816, 1208, 1203), 0.5, 1.0),
+    # B alone repacked; both repacked, K odd
+    ((1300, 1310, 1600), (1600, 1311, 1312), -1.0, 0.5),
+    ((1300, 1304, 1603), (1608, 1304, 1304), 1.0, 0.75),
+    # few rows in place: one tile row, cut
+    ((17, 30000, 128), (136, 30008, 30003), 2.0, 0.5),
+    ((65, 25000, 200), (200, 25000, 25001), 1.0, -1.0),
 ])
 def test_general_random_within_tolerance(gpu, oracle, dims, strides, alpha, beta):
     """Random bf16 inputs: MFMA summation order differs from the sequential
@@ -169,14 +179,26 @@ def test_general_random_within_tolerance(gpu, oracle, dims, strides, alpha, beta
     # both repacked, K not a multiple of 64 (B's repacked rows end inside the
     # last stage)
     ((200, 130, 77), (77, 131, 140), -2.0, 0.125),
+    # in place on the pipelined tiles, and repacked for them, whole and partial
+    # last stages
+    ((1300, 1304, 1600), (1600, 1304, 1310), 1.5, -0.25),
+    ((1400, 1200, 1816), (1816, 1208, 1203), 0.5, 1.0),
+    # B alone repacked; both repacked, K odd
+    ((1300, 1310, 1600), (1600, 1311, 1312), -1.0, 0.5),
+    ((1300, 1304, 1603), (1608, 1304, 1304), 1.0, 0.75),
+    # few rows in place: one tile row, cut
+    ((17, 30000, 128), (136, 30008, 30003), 2.0, 0.5),
+    ((65, 25000, 200), (200, 25000, 25001), 1.0, -1.0),
 ])
 def test_general_pipelined_tile_matches_staged_kernel(gpu, oracle, dims, strides, alpha, beta):
     """One GEMM three ways, the same bits: the pipelined tiles on the
     operands as given; the same with A two bytes past a 16-byte boundary
     (the tiles cannot read it in place, so it is repacked into aligned,
-    zero-padded rows first when M and N reach 128); and the 64x64 staged
-    kernel, reached through row strips of 64 (below the repack size), the
-    reference's schedule.  Also with NaN and infinity in A's and B's stride
+    zero-padded rows first, or read by the register tiles where those are
+    faster); and the 64x64 register tiles, reached through row strips of 64.
+    Small outputs take the register tiles on all three ways; past their lines
+    (register_tiles in gemm_small.hip) are the 3000 x 2900 outputs, the last
+    six here and the last two of the test below.  Also with NaN and infinity in A's and B's stride
     padding; C's padding untouched; rel-err <= 1e-5 against the tiled CPU
     schedule."""
     m, n, k = dims
@@ -203,7 +225,7 @@ def test_general_pipelined_tile_matches_staged_kernel(gpu, oracle, dims, strides
                  beta).launch()
     assert gr.guards_intact() and a_off.unchanged()
     assert_same(gr.download(), got, "A at a 2-byte offset vs in place")
-    # the staged kernel, 64 rows at a time (strips of C, A and C offset by rows)
+    # the register tiles, 64 rows at a time (strips of C, A and C offset by rows)
     ga_s = gpu.to_device(a)
     gs = gpu.to_device(c)
     for r0 in range(0, m, 64):
@@ -211,7 +233,7 @@ def test_general_pipelined_tile_matches_staged_kernel(gpu, oracle, dims, strides
         kern.prepare(ga_s.view(r0 * lda, (rows - 1) * lda + k), gb,
                      gs.view(r0 * ldc, (rows - 1) * ldc + n), rows, n, k, lda, ldb, ldc, alpha,
                      beta).launch()
-    assert_same(gs.download(), got, "pipelined tile vs staged kernel")
+    assert_same(gs.download(), got, "pipelined tile vs register tiles")
     for r in range(m - 1):
         assert got[r * ldc + n:(r + 1) * ldc].tobytes() == c[r * ldc + n:(r + 1) * ldc].tobytes()
     rows = np.concatenate([got[r * ldc:r * ldc + n] for r in range(m)])
@@ -435,10 +457,11 @@ def test_gemm_bf16_nt_misaligned_operands_match_aligned(gpu, m, n, k, which):
 
 
 @pytest.mark.parametrize("m,n,k", [(300, 260, 1003), (256, 512, 4097), (1024, 1024, 77),
-                                   (128, 128, 9)])
+                                   (128, 128, 9), (1600, 1500, 1003)])
 def test_gemm_bf16_nt_odd_k_repacked(gpu, oracle, m, n, k):
     """K not a multiple of 8 (rows not 16-byte aligned): both operands are
-    repacked into rows of K rounded up to 8 and the tile runs on them."""
+    repacked into rows of K rounded up to 8 and the tile runs on them (the
+    last shape); outputs of few tiles are read in place by the direct kernel."""
     _nt_case(gpu, oracle, m, n, k, seed=4)
 
 
@@ -511,7 +534,8 @@ def test_gemm_bf16_nt_small_grid_tiles(gpu, oracle, m, n, k):
 
 
 # M or N not a multiple of 256 with whole 64-k stages: edge tiles of the
-# pipelined kernel (clamped operand rows, element-wise masked stores)
+# pipelined kernel (clamped operand rows, masked 16-byte stores), and the
+# direct kernel for the outputs of few tiles
 @pytest.mark.parametrize("m,n,k", [(300, 520, 512), (257, 255, 128), (1, 1000, 64),
                                    (1000, 264, 1024), (4000, 4000, 256), (4000, 2000, 128)])
 def test_gemm_bf16_nt_edge_tiles(gpu, oracle, m, n, k):
@@ -598,10 +622,11 @@ def test_gemm_bf16_nt_tail_round_matches_row_blocks(gpu, m, n, k):
         assert_same(part.download(), whole[r0 * n:(r0 + rows) * n], f"rows {r0}..{r0 + rows}")
 
 
-def test_gemm_bf16_nt_whole_tiles_unaligned_c(gpu, oracle):
-    """Whole tiles but C at an odd element offset: the edge form, 2-byte
-    stores; every output against the oracle and the neighbours untouched."""
-    m, n, k = 256, 512, 192
+# the direct kernel, 128x128 tiles and 256x256 tiles
+@pytest.mark.parametrize("m,n,k", [(256, 512, 192), (1024, 1024, 192), (2048, 4352, 64)])
+def test_gemm_bf16_nt_whole_tiles_unaligned_c(gpu, oracle, m, n, k):
+    """Whole tiles but C at an odd element offset: 16-byte stores at C's own
+    alignment; every output against the oracle and the neighbours untouched."""
     kern = _kernels()
     da, db = gpu.alloc(m * k, np.uint16), gpu.alloc(n * k, np.uint16)
     kern.fill_normal_bf16(da, 8, 0xA, 1.0 / np.sqrt(k))

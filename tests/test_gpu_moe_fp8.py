@@ -230,8 +230,8 @@ def test_moe_ffn_small_all_tokens(gpu, oracle):
 
 @pytest.mark.parametrize("experts", [2, 3])
 def test_moe_ffn_few_experts(gpu, oracle, experts):
-    """Two and three experts: the expert halves that run on the caller's
-    stream and on the side stream are 1 + 1 and 1 + 2 experts."""
+    """Two and three experts: tile lists whose last XCD pieces are short or
+    empty."""
     tokens, hidden, ffn = 256, 256, 256
     worst, _ = _ffn_case(gpu, oracle, tokens, hidden, ffn, experts, 0xFFFFFFFF, range(tokens))
     assert worst <= 1e-2, worst
@@ -517,9 +517,7 @@ def test_gemm_fp8_all_outputs(gpu, oracle, m, n, k):
     assert _fp8_case(gpu, oracle, m, n, k, (rr.ravel(), cc.ravel())) <= 1e-2
 
 
-# any M, N: edge tiles on the fast path (K a multiple of 16, the last stage
-# partial when K is not a multiple of 128), the generic bounds-checked kernel
-# otherwise (E4M3 widened exactly to bf16)
+# any M, N and K on the direct kernel: cut rows, columns and units of K
 @pytest.mark.parametrize("m,n,k", [(300, 520, 256), (1, 257, 128), (257, 256, 384),
                                    (100, 70, 96), (33, 65, 200), (256, 256, 160), (5, 3, 1)])
 def test_gemm_fp8_any_shape(gpu, oracle, m, n, k):
