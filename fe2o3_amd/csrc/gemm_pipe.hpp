@@ -84,9 +84,9 @@ struct Geo {
 // chunk at or past k_end (chunk byte offset cbytes[j] along k within its
 // stage, plus the stage's kbytes) loads from a VGPR offset past the
 // buffer's extent, which the range check turns into 16 zero bytes in LDS.
-// The range check covers the VGPR offset only, not the scalar offset soff
-// carries, so a stage offset alone never makes a load return zeros: every
-// load past the operand's k goes through this mask.  For a [k][n] operand a
+// A chunk past k mostly lies inside the extent (in a row further on), so a
+// stage offset alone does not make its load return zeros: every load past the
+// operand's k goes through this mask.  For a [k][n] operand a
 // chunk is one k row (cbytes = 2 * its row within the stage).  Dense rows
 // have k_end a multiple of 16 bytes, so no chunk straddles it.  The zeros'
 // products are zero, the zero padding the register tiles give a partial k
@@ -179,6 +179,13 @@ FE2O3_DEVICE uint32_t kn_swz(uint32_t krow) {
   // 8-byte pieces fill 32 distinct 16-byte positions of the 512-byte rows
   return 2u * ((krow & 3u) | (((krow >> 3) & 3u) << 2));
 }
+// The extent ends with the last row's last valid column, in whole dwords: the
+// range check drops a dword that the extent cuts, and with it an odd
+// valid_cols' last element.  Rows are 16-byte aligned, so the two bytes past
+// it lie in the element's own dword.
+FE2O3_DEVICE uint32_t kn_extent(uint32_t ld, uint32_t valid_cols, uint32_t k16) {
+  return ((k16 - 1u) * ld + ((valid_cols + 1u) & ~1u)) * 2u;
+}
 // MASK: k16 is not a multiple of 64 and the last stage's rows from k16 on
 // load zeros (Rows::off).
 template <bool MASK = false>
@@ -187,7 +194,7 @@ FE2O3_DEVICE Rows<128, 8, true, MASK> kn_rows(const uint16_t* base, uint32_t ld,
   Rows<128, 8, true, MASK> t;
   const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
   const uint32_t last_chunk = (valid_cols - 1u) / 8u;
-  t.bytes = ((k16 - 1u) * ld + valid_cols) * 2u;
+  t.bytes = kn_extent(ld, valid_cols, k16);
   t.kmul = ld;  // a stage of 64 k (128 bytes along a k row) is 64 rows of ld elements
   if constexpr (MASK) t.k_end = k16 * 2u;
 #pragma unroll
@@ -247,7 +254,7 @@ FE2O3_DEVICE Rows<128, 4, true, MASK> kn_rows128(const uint16_t* base, uint32_t 
   Rows<128, 4, true, MASK> t;
   const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
   const uint32_t last_chunk = (valid_cols - 1u) / 8u;
-  t.bytes = ((k16 - 1u) * ld + valid_cols) * 2u;
+  t.bytes = kn_extent(ld, valid_cols, k16);
   t.kmul = ld;  // a stage of 64 k (128 bytes along a k row) is 64 rows of ld elements
   if constexpr (MASK) t.k_end = k16 * 2u;
 #pragma unroll

@@ -124,6 +124,13 @@ def test_general_hardware_matrix_bit_exact(gpu, oracle, case, schedule):
     # B alone repacked; both repacked, K odd
     ((1300, 1310, 1600), (1600, 1311, 1312), -1.0, 0.5),
     ((1300, 1304, 1603), (1608, 1304, 1304), 1.0, 0.75),
+    # N odd: the last element of B ends in the middle of a dword (in place, one
+    # column in the last tile, repacked, on the 256x256 tile; K within a stage)
+    ((1300, 1303, 1600), (1600, 1304, 1303), 1.0, 0.5),
+    ((1300, 1409, 1608), (1608, 1416, 1410), -1.5, 0.5),
+    ((1300, 1303, 1600), (1600, 1303, 1304), 1.0, 1.0),
+    ((3000, 2901, 64), (64, 2904, 2901), 2.0, -1.0),
+    ((3000, 2903, 40), (40, 2904, 2903), 1.0, 0.0),
     # few rows in place: one tile row, cut
     ((17, 30000, 128), (136, 30008, 30003), 2.0, 0.5),
     ((65, 25000, 200), (200, 25000, 25001), 1.0, -1.0),
@@ -186,6 +193,13 @@ def test_general_random_within_tolerance(gpu, oracle, dims, strides, alpha, beta
     # B alone repacked; both repacked, K odd
     ((1300, 1310, 1600), (1600, 1311, 1312), -1.0, 0.5),
     ((1300, 1304, 1603), (1608, 1304, 1304), 1.0, 0.75),
+    # N odd: the last element of B ends in the middle of a dword (in place, one
+    # column in the last tile, repacked, on the 256x256 tile; K within a stage)
+    ((1300, 1303, 1600), (1600, 1304, 1303), 1.0, 0.5),
+    ((1300, 1409, 1608), (1608, 1416, 1410), -1.5, 0.5),
+    ((1300, 1303, 1600), (1600, 1303, 1304), 1.0, 1.0),
+    ((3000, 2901, 64), (64, 2904, 2901), 2.0, -1.0),
+    ((3000, 2903, 40), (40, 2904, 2903), 1.0, 0.0),
     # few rows in place: one tile row, cut
     ((17, 30000, 128), (136, 30008, 30003), 2.0, 0.5),
     ((65, 25000, 200), (200, 25000, 25001), 1.0, -1.0),
@@ -198,7 +212,7 @@ def test_general_pipelined_tile_matches_staged_kernel(gpu, oracle, dims, strides
     faster); and the 64x64 register tiles, reached through row strips of 64.
     Small outputs take the register tiles on all three ways; past their lines
     (register_tiles in gemm_small.hip) are the 3000 x 2900 outputs, the last
-    six here and the last two of the test below.  Also with NaN and infinity in A's and B's stride
+    eleven here and the last two of the test below.  Also with NaN and infinity in A's and B's stride
     padding; C's padding untouched; rel-err <= 1e-5 against the tiled CPU
     schedule."""
     m, n, k = dims
