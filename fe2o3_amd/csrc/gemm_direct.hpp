@@ -16,10 +16,9 @@
 // (bf16 16 x 4096 x 14336: 34.1 us against 24.7; 128 x 4096 x 4096: 23.9
 // against 13.6).
 //
-// The in-order form gives every wave an output block of its
-// own and all of K instead: C's bits are then those of the pipelined tile, for
-// the calls that would take the tile if their operands could be read in place
-// or copied.
+// The in-order form gives every wave an output block of its own and all of K
+// instead: C's bits are then those of the pipelined tile, for the calls that
+// would take the tile if their operands could be read in place or copied.
 //
 // What bounds it: with one block row (m <= 16 MB) the weights' HBM stream,
 // else the 64 bytes a clock that a CU loads (16 (MB + NB) rows of K per
