@@ -481,7 +481,7 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   // scratch, take the direct kernel, in K order where the tile could run the
   // sizes or K is short (gemm_direct::in_order).
   const uint32_t kp = (k + 15u) & ~15u;
-  const bool repack = !fast && gemm_direct::repack(m, n, k, 1u);
+  const bool repack = !fast && gemm_direct::repack(m, n, k, 1u, s);
   void* scratch = nullptr;
   if (repack) {
     const bool ra = k % 16 != 0 || !aligned_a, rb = k % 16 != 0 || !aligned_b;
@@ -494,7 +494,7 @@ int32_t fe2o3_gemm_fp8_nt(const uint8_t* a, uint64_t a_len, const uint8_t* b, ui
   if (!fast && scratch == nullptr) {
     if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
     return launch_direct(gemm_direct::in_order(m, n, k, 1u)
-                             ? gemm_direct::plan_in_order<gemm_direct::Fp8>(m, n)
+                             ? gemm_direct::plan_in_order(m, n)
                              : gemm_direct::plan(m, n, k, 1u, topo.cus),
                          a, b, scale_a, scale_b, c, m, n, k, topo, s);
   }

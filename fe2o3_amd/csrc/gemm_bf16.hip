@@ -274,7 +274,7 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
   // scratch, take the direct kernel, in K order where the tile could run the
   // sizes or K is short (gemm_direct::in_order).
   const uint32_t kp = (k + 7u) & ~7u;
-  if (fast || gemm_direct::repack(m, n, k, 2u)) {
+  if (fast || gemm_direct::repack(m, n, k, 2u, s)) {
     const int32_t lds_rc = set_fast_lds();  // before any launch: a failure leaves C untouched
     if (lds_rc != FE2O3_OK) return lds_rc;
     const tile_plan::Plan plan = tile_plan::plan(m, n, topo);
@@ -304,7 +304,7 @@ extern "C" int32_t fe2o3_gemm_bf16_nt(const uint16_t* a, uint64_t a_len, const u
   }
   if (!gemm_direct::rows_ok(m)) return FE2O3_ERR_SHAPE;
   return launch_direct(gemm_direct::in_order(m, n, k, 2u)
-                           ? gemm_direct::plan_in_order<gemm_direct::Bf16>(m, n)
+                           ? gemm_direct::plan_in_order(m, n)
                            : gemm_direct::plan(m, n, k, 2u, topo.cus),
                        a, b, c, m, n, k, topo, s);
 }

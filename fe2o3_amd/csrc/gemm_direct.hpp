@@ -30,6 +30,7 @@
 
 #include "common.hpp"
 #include "gemm_pipe.hpp"
+#include "internal.hpp"
 
 namespace gemm_direct {
 
@@ -53,7 +54,6 @@ struct Bf16 {
   static constexpr uint32_t kBytes = 2;  // per element
   static constexpr bool kScaled = false;
   static constexpr int kDeep = 3;  // units in flight of the widest forms
-  static constexpr bool kOrderedWide = false;  // the in-order form is in the light kernel
   static FE2O3_DEVICE uint32_t tile_piece(uint32_t g, uint32_t h) { return 4u * h + g; }
   static FE2O3_DEVICE void mma(const Frag& b, const Frag& a, f32x4_t& acc) {
 #pragma unroll
@@ -71,7 +71,6 @@ struct Fp8 {
   static constexpr uint32_t kBytes = 1;
   static constexpr bool kScaled = true;
   static constexpr int kDeep = 2;
-  static constexpr bool kOrderedWide = true;  // the light one has no registers for it
   static FE2O3_DEVICE uint32_t tile_piece(uint32_t g, uint32_t h) { return 2u * g + h; }
   static FE2O3_DEVICE void mma(const Frag& b, const Frag& a, f32x4_t& acc) {
     acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
@@ -441,10 +440,10 @@ inline bool rows_ok(uint32_t m) { return ((uint64_t)m + 63u) / 64u <= 65535u; }
 //   tile_sizes: outputs from 128 x 128 on (any K, copied into rows of whole
 //     pieces), and smaller ones whose rows are whole pieces.
 //   repack: they are copied into scratch for the tile; small ones only when
-//     K is long, else the in-order form, which also serves without scratch
-//     (us, copies and tile against in order: bf16 100 x 8192 x 4096 53 | 114,
-//     fp8 38 | 59; bf16 127 x 9000 x 1024 29 | 31, fp8 29 | 17; bf16 16 x 40000
-//     x 256 25 | 10).
+//     K is long and the call is not captured into a graph, else the in-order
+//     form, which also serves without scratch (us, copies and tile against
+//     in order: bf16 100 x 8192 x 4096 53 | 114, fp8 38 | 59; bf16 127 x 9000 x
+//     1024 29 | 31, fp8 29 | 17; bf16 16 x 40000 x 256 25 | 10).
 constexpr uint32_t kRepackMin = 128;
 constexpr uint32_t kShortK = 2048;  // bytes, 16 units
 inline bool tile_sizes(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) {
@@ -452,14 +451,14 @@ inline bool tile_sizes(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) 
   return 256ull * padded < (1ull << 31) &&
          (padded == kbytes || (m >= kRepackMin && n >= kRepackMin));
 }
-inline bool repack(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) {
+inline bool repack(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes, hipStream_t s) {
   return tile_sizes(m, n, k, elem_bytes) &&
          ((m >= kRepackMin && n >= kRepackMin) ||
-          ((uint64_t)k * elem_bytes > kShortK && rows_ok(m)));
+          ((uint64_t)k * elem_bytes > kShortK && rows_ok(m) && !fe2o3_host::capturing(s)));
 }
 // The in-order form also takes the short K of sizes that no tile runs: at most
 // two units a wave do not pay for the split's merge.  Split | in order, us:
-//   bf16 100000 x 5 x 65 21 | 7   40001 x 33 x 75 23 | 10   20000 x 100 x 401 33 | 24
+//   bf16 100000 x 5 x 65 21 | 8   40001 x 33 x 75 23 | 9   20000 x 100 x 401 33 | 25
 //   fp8 20000 x 100 x 1601 48 | 44   past the line: bf16 20000 x 100 x 1601 55 | 73
 inline bool in_order(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes) {
   return tile_sizes(m, n, k, elem_bytes) || (uint64_t)k * elem_bytes <= kShortK;
@@ -471,7 +470,8 @@ inline bool k_fits(uint32_t k, uint32_t elem_bytes) { return 64ull * k * elem_by
 constexpr uint32_t smem_of(uint32_t mb, uint32_t nb) {
   return kWaves * 1024u * (mb * nb > 2u * (mb + nb) ? mb * nb : 2u * (mb + nb));
 }
-// Launches of the light kernel or the wide one.
+// Launches of the light kernel or the wide one, which also holds the last three
+// (in the light one they would cost its forms registers).
 constexpr int kAnyK = kNumForms, kInOrder = kNumForms + 1, kFill = kNumForms + 2;
 struct Launch {
   int form;
@@ -486,10 +486,9 @@ inline Launch plan(uint32_t m, uint32_t n, uint32_t k, uint32_t elem_bytes, uint
 }
 // 2 x 2 blocks, one per wave; their ids are 32-bit, so more of them stay a grid
 // that the launch refuses
-template <class T>
 inline Launch plan_in_order(uint32_t m, uint32_t n) {
   const uint64_t blocks = grid_of(Form{2, 2, false}, m, n);
-  return {kInOrder, T::kOrderedWide, blocks > 0x7fffffffu ? blocks : (blocks + kWaves - 1u) / kWaves,
+  return {kInOrder, true, blocks > 0x7fffffffu ? blocks : (blocks + kWaves - 1u) / kWaves,
           smem_of(2, 2)};
 }
 // K = 0: C is all +0 (an empty sum, whatever the scales).  A grid-stride fill
@@ -516,9 +515,6 @@ template <class T, bool WIDE>
 FE2O3_DEVICE void run_form(int form, const uint8_t* a, const uint8_t* b, uint16_t* c, uint32_t m,
                            uint32_t n, uint32_t k, float scale, uint32_t xcds, uint8_t* smem) {
 #define FE2O3_DIRECT(MB, NB, D) return block<T, MB, NB, D>(a, b, c, m, n, k, scale, xcds, smem)
-  if constexpr (WIDE == T::kOrderedWide)
-    if (form == kInOrder)
-      return block<T, 2, 2, 2, uint32_t, true>(a, b, c, m, n, k, scale, xcds, smem);
   if constexpr (!WIDE) {
     switch (form) {
       case 0: FE2O3_DIRECT(1, 1, 4);
@@ -532,6 +528,8 @@ FE2O3_DEVICE void run_form(int form, const uint8_t* a, const uint8_t* b, uint16_
       case 5: FE2O3_DIRECT(4, 1, 3);
       case 6: FE2O3_DIRECT(2, 4, T::kDeep);
       case 7: FE2O3_DIRECT(4, 2, T::kDeep);
+      case kInOrder:
+        return block<T, 2, 2, 2, uint32_t, true>(a, b, c, m, n, k, scale, xcds, smem);
       case kFill: return fill(c, (uint64_t)m * n);
       default: return block<T, 1, 4, 1, uint64_t>(a, b, c, m, n, k, scale, xcds, smem);
     }

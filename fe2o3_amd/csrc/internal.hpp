@@ -49,6 +49,9 @@ int32_t device_topology(tile_plan::Topology* out);
 // before it.  0, or a hipError_t.
 int32_t scratch_alloc(void** p, size_t bytes, hipStream_t s);
 int32_t scratch_free(void* p, hipStream_t s);
+// Whether s is being captured into a graph, where a call that has a way
+// without scratch takes it rather than leave allocation nodes in the graph.
+bool capturing(hipStream_t s);
 
 // `rows` rows of `cols` bf16 elements, `ld` apart from src (any 2-byte
 // alignment), copied on stream s into rows of dst_cols elements (a multiple

@@ -174,6 +174,15 @@ int32_t scratch_free(void* p, hipStream_t s) {
   return p == nullptr ? 0 : (int32_t)hipFreeAsync(p, s);
 }
 
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 }  // namespace fe2o3_host
 
 static_assert(sizeof(Fe2o3KernelResources) == 120, "resource record is 120 bytes");

@@ -265,9 +265,11 @@ int32_t fe2o3_scalar_gemm_v1(const float *a, uint64_t a_len, const float *b,
  * cannot be read in place are first copied into aligned rows of k rounded up
  * to 8 (zeros past k) in stream-ordered scratch from the library's pool and
  * the tile runs on them; when m or n is below 128 (k a multiple of 8 and
- * short, or any other k), and on devices without a pool, a kernel reads them
- * where they are and, where the tile could run the sizes, sums in its order.  An operand that is only misaligned gives the aligned operand's bits
- * on every one of these ways.  k = 0 writes +0. */
+ * short, or any other k), in a captured call of such a size, and on devices
+ * without a pool, a kernel reads them where they are and, where the tile
+ * could run the sizes, sums in its order.  An operand that is only misaligned
+ * gives the aligned operand's bits on every one of these ways.  k = 0 writes
+ * +0. */
 int32_t fe2o3_gemm_bf16_nt(const uint16_t *a, uint64_t a_len,
                            const uint16_t *b, uint64_t b_len, uint16_t *c,
                            uint64_t c_len, uint32_t m, uint32_t n, uint32_t k,

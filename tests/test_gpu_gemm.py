@@ -8,6 +8,8 @@ otherwise the reference's bounded policies, and max|y - yhat| / max|yhat|
 """
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -468,6 +470,61 @@ def test_gemm_bf16_nt_misaligned_operands_match_aligned(gpu, m, n, k, which):
     prep.prepare(ga, gb, got.body, m, n, k).launch()
     assert got.guards_intact() and all(o.unchanged() for o in offs.values())
     assert_same(got.download(), want.download(), f"{which} at a 2-byte offset vs aligned")
+
+
+def _hip():
+    """The HIP runtime that the library is linked to, as it is mapped here."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    return ctypes.CDLL(path)
+
+
+# the direct kernel, the K = 0 fill, the in-order form, and the in-order form of
+# a call that is repacked when it is not captured
+@pytest.mark.parametrize("m,n,k,off", [(64, 1000, 520, 1), (300, 260, 0, 0), (120, 9000, 1024, 1),
+                                       (100, 8200, 1032, 1)])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_gemm_nt_captured(gpu, m, n, k, off, fp8):
+    """Captured into a graph without allocations: every one of three replays,
+    with eager calls and a fresh C between them, gives the eager call's bits."""
+    from fe2o3_amd.runtime import Stream
+    if fp8:
+        k *= 2
+    rng = np.random.default_rng(m + k)
+    dt = np.uint8 if fp8 else np.uint16
+    a, b = ((rng.integers(0, 0x50, s + off).astype(np.uint8) if fp8 else
+             (rng.standard_normal(s + off).astype(np.float32).view(np.uint32) >> 16).astype(dt))
+            for s in (m * k, n * k))
+    da, db = gpu.to_device(a).view(off, m * k), gpu.to_device(b).view(off, n * k)
+    c, blank = gpu.alloc(m * n, np.uint16), np.full(m * n, 0x7FDE, np.uint16)
+    one = gpu.to_device(np.ones(1, np.float32))
+    kern = _kernels()
+
+    def call(stream=None):
+        if fp8:
+            kern.gemm_fp8_nt(da, db, one, one, c, m, n, k, stream=stream, sync=False)
+        else:
+            kern.gemm_bf16_nt_gpu.Kernel.load(gpu).prepare(da, db, c, m, n, k).launch_async(stream)
+
+    call()
+    gpu.synchronize()
+    want = c.download()
+    hip, side = _hip(), Stream(gpu)
+    graph, ready = ctypes.c_void_p(), ctypes.c_void_p()
+    handle = ctypes.c_void_p(side.handle)
+    assert hip.hipStreamBeginCapture(handle, 2) == 0  # relaxed
+    call(side)
+    assert hip.hipStreamEndCapture(handle, ctypes.byref(graph)) == 0
+    nodes = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(nodes)) == 0 and nodes.value == 1
+    assert hip.hipGraphInstantiate(ctypes.byref(ready), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        c.upload(blank)
+        assert hip.hipGraphLaunch(ready, handle) == 0
+        side.synchronize()
+        assert_same(c.download(), want, "replay vs eager")
+        call()
+        gpu.synchronize()
+    assert hip.hipGraphExecDestroy(ready) == 0 and hip.hipGraphDestroy(graph) == 0
 
 
 @pytest.mark.parametrize("m,n,k", [(300, 260, 1003), (256, 512, 4097), (1024, 1024, 77),
